@@ -460,9 +460,11 @@ Grid Engine::grid() const {
     g.nb_scell = nb_scell_;
     g.nfoams = (int)foams.size();
     g.stream = stream;
-    g.walls = false;
-    for (const FoamRec &r : foams)
+    g.walls = g.big = false;
+    for (const FoamRec &r : foams) {
         for (int a = 0; a < r.h.c.dim; ++a) g.walls = g.walls || r.h.c.wall[a] != 0;
+        g.big = g.big || r.h.nblk > kFuseBlocks;
+    }
     return g;
 }
 
@@ -475,18 +477,21 @@ void Engine::enqueue_attempt(uint32_t flags) {
     launch_correct(g, flags, CUBBLE_PREC_MIXED == precision);
 }
 
-void Engine::enqueue_group(uint32_t flags) {
+void Engine::enqueue_groups(uint32_t flags, int groups) {
     const Grid g = grid();
-    enqueue_attempt(flags);
-    launch_remove(g);
-    launch_search(g);
+    for (int k = 1; k <= groups; ++k) {
+        enqueue_attempt(flags);
+        launch_apply(g);
+        if (0 == k % kSearchEvery || groups == k) launch_search(g);
+    }
 }
 
 int Engine::capture(uint32_t flags, int groups) {
-    // the graph holds the kernel variants chosen for the foams it was
-    // captured with (walls or not)
-    const bool walls = grid().walls;
-    if (graph_ && graph_flags_ == flags && graph_groups_ == groups && graph_walls_ == walls)
+    // the graph holds the kernels chosen for the foams it was captured with
+    // (walls or not, a sums launch or not)
+    const Grid g = grid();
+    if (graph_ && graph_flags_ == flags && graph_groups_ == groups && graph_walls_ == g.walls &&
+        graph_big_ == g.big)
         return CUBBLE_OK;
     if (graph_) {
         (void)hipGraphExecDestroy(graph_);
@@ -494,7 +499,7 @@ int Engine::capture(uint32_t flags, int groups) {
     }
     hipGraph_t gr = nullptr;
     E_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < groups; ++k) enqueue_group(flags);
+    enqueue_groups(flags, groups);
     E_TRY(hipStreamEndCapture(stream, &gr));
     const hipError_t e = hipGraphInstantiate(&graph_, gr, nullptr, nullptr, 0);
     (void)hipGraphDestroy(gr);
@@ -504,7 +509,8 @@ int Engine::capture(uint32_t flags, int groups) {
     }
     graph_flags_ = flags;
     graph_groups_ = groups;
-    graph_walls_ = walls;
+    graph_walls_ = g.walls;
+    graph_big_ = g.big;
     return CUBBLE_OK;
 }
 
@@ -602,8 +608,12 @@ int Engine::fail_foam(int k, int code) {
 }
 
 int Engine::settle(std::vector<Dyn> &d) {
-    int rc = read_dyn_all(d);
-    if (rc) return rc;
+    const int rc = read_dyn_all(d);
+    return rc ? rc : settle_read(d);
+}
+
+int Engine::settle_read(std::vector<Dyn> &d) {
+    int rc = CUBBLE_OK;
     bool grew = false;
     for (int k = 0; k < (int)d.size(); ++k) {
         if (!d[k].overflow || foams[k].failed) continue;
@@ -665,17 +675,30 @@ int Engine::set_limits(int64_t steps, const std::vector<int64_t> *per_foam) {
     return CUBBLE_OK;
 }
 
+int Engine::lift_limits(std::vector<Dyn> &d) {
+    const int rc = set_limits(0, nullptr);
+    for (Dyn &x : d) x.halt = x.overflow = x.step_limit = 0;
+    return rc;
+}
+
 int Engine::integrate(uint32_t flags, std::vector<Dyn> &d) {
     int rc = set_limits(1, nullptr);
     if (rc) return rc;
     for (int tries = 0; tries < 100000; ++tries) {
-        enqueue_group(flags);
+        enqueue_attempt(flags);
+        launch_apply(grid());
         E_TRY(hipGetLastError());
-        if ((rc = settle(d))) return rc;
-        if (steps_left(d) == 0) {
-            if ((rc = set_limits(0, nullptr))) return rc;
-            return read_dyn_all(d);
+        if ((rc = read_dyn_all(d))) return rc;
+        // the search's launches only when some foam needs them
+        bool search = false;
+        for (const Dyn &x : d) search = search || x.need_search;
+        if (search) {
+            launch_search(grid());
+            E_TRY(hipGetLastError());
+            if ((rc = read_dyn_all(d))) return rc;
         }
+        if ((rc = settle_read(d))) return rc;
+        if (steps_left(d) == 0) return lift_limits(d);
     }
     return fail(CUBBLE_E_STATE, "integrate: no accepted step after 100000 attempts");
 }
@@ -691,19 +714,22 @@ int Engine::run_steps(uint32_t flags, int64_t steps, std::vector<Dyn> &d,
     int rc = capture(flags, groups);
     if (rc) return rc;
     if ((rc = set_limits(steps, per_foam))) return rc;
-    for (int64_t guard = 0; guard < (int64_t)1 << 40; ++guard) {
-        if ((rc = read_dyn_all(d))) return rc;
-        const int64_t left = steps_left(d);
-        if (left <= 0) break;
+    // set_limits left every foam `steps`, or its own number of them, to go
+    int64_t left = steps;
+    if (per_foam) {
+        left = 1;
+        for (int64_t s : *per_foam) left = std::max(left, s);
+    }
+    while (left > 0) {
         // rounds of at most kRoundGroups attempt groups, so a halted foam
         // (capacity growth) waits at most that long for the host
         const int64_t launches = std::min<int64_t>(std::max(1, kRoundGroups / groups),
                                                    std::max<int64_t>(1, (left + groups - 1) / groups));
         for (int64_t k = 0; k < launches; ++k) E_TRY(hipGraphLaunch(graph_, stream));
         if ((rc = settle(d))) return rc;
+        left = steps_left(d);
     }
-    if ((rc = set_limits(0, nullptr))) return rc;
-    return read_dyn_all(d);
+    return lift_limits(d);
 }
 
 int Engine::search_pending() {

@@ -53,6 +53,13 @@ struct Tuning {
 // Smallest neighbour-search tile, in bubbles.
 constexpr int kMinSearchTile = 32;
 
+// Attempts between two search phases of a captured run.  A search is needed
+// every 20 to 80 steps (14 in the first steps after seeding), and its seven
+// launches cost 1.5 to 4.5 us each when no foam needs them; a foam that does
+// stands still until the next phase, which costs it the few idle launches of
+// the attempts between.
+constexpr int kSearchEvery = 8;
+
 // Most attempt groups between two host checks of the foams' flags in
 // run_steps (halts, list-capacity growth).
 constexpr int kRoundGroups = 128;
@@ -105,7 +112,9 @@ class Engine {
 
     Grid grid() const;
     void enqueue_attempt(uint32_t flags);
-    void enqueue_group(uint32_t flags);
+    // `groups` attempts with their removals; a search phase after every
+    // kSearchEvery of them and at the end
+    void enqueue_groups(uint32_t flags, int groups);
     int capture(uint32_t flags, int groups);
 
     int read_dyn_all(std::vector<Dyn> &out);
@@ -115,6 +124,10 @@ class Engine {
     // Read every foam's scalars; grow and rebuild the neighbour lists of
     // foams whose search overflowed the list capacity.
     int settle(std::vector<Dyn> &d);
+    // The same with the scalars just read.
+    int settle_read(std::vector<Dyn> &d);
+    // Lift the step limits: clears halt and overflow, on the device and in d.
+    int lift_limits(std::vector<Dyn> &d);
 
     // Host-driven: one attempt group at a time until each foam accepted one
     // step (integrate()).
@@ -170,7 +183,7 @@ class Engine {
     hipGraphExec_t graph_ = nullptr;
     uint32_t graph_flags_ = 0;
     int graph_groups_ = 0;
-    bool graph_walls_ = false;
+    bool graph_walls_ = false, graph_big_ = false;
     int committed_nf_ = 0;  // foams in the device array at the last commit
 
   public:

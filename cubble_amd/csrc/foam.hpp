@@ -21,6 +21,7 @@ namespace cubble_amd {
 constexpr int kBlock = 256;         // threads per block, bubble- and cell-space
 constexpr int kMaxBlocks = 2048;    // bubble-space blocks per foam (partials)
 constexpr int kNumXcd = 8;          // MI355X: 8 XCDs, workgroups round-robin
+constexpr int kFuseBlocks = 256;    // foams of at most this many blocks sum their partials in k_correct
 constexpr int kPartD = 8;           // doubles per block partial record
 constexpr int kPartI = 4;           // ints per block partial record
 
@@ -142,6 +143,10 @@ __host__ __device__ inline bool stop_reached(const Dyn &d) {
     return d.time_stop &&
            (d.time_int > d.stop_int || (d.time_int == d.stop_int && d.time_frac >= d.stop_frac));
 }
+
+// A foam that stands still in an attempt: halted, or waiting for its search
+// (a graph holds one search for several attempts).
+__host__ __device__ inline bool standing(const Dyn &d) { return (d.halt | d.need_search) != 0; }
 
 struct Foam {
     Consts c;

@@ -20,6 +20,7 @@ struct Grid {
     int nfoams;
     hipStream_t stream;
     bool walls;  // some foam of the launch has a wall
+    bool big;    // some foam of the launch has more than kFuseBlocks blocks
 };
 
 void launch_predict(const Grid &g, uint32_t flags);
@@ -27,15 +28,21 @@ void launch_pair(const Grid &g, uint32_t flags);
 // The mixed pair kernel, then (fix) the second pass over the bubbles that met
 // a pair needing FP64 values.
 void launch_pair_mixed(const Grid &g, uint32_t flags, bool fix = true);
-// S_A, S_Ar, S_OA, S_OAr from the predictor and pair partials (one block per foam)
+// S_A, S_Ar, S_OA, S_OAr of foams of more than kFuseBlocks blocks, from the
+// predictor and pair partials (one block per foam; the others sum their own
+// in the corrector)
 void launch_sums(const Grid &g);
 // corrector (mixed: the mixed-precision variant, for engines of that
-// precision), then (control) the dt controller / commit (one block per foam)
+// precision), then (control) the dt controller / commit and the plan of a
+// removal (one block per foam)
 void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control = true);
 
-// removeBubbles: emit the sorted deletion list and plan the moves, then move
-// the tail survivors into the holes, filter / remap the neighbour lists and
-// apply the volume fix.  Runs only for foams whose need_remove flag is set.
+// The planned removals: move the tail survivors into the holes, filter /
+// remap the neighbour lists and apply the volume fix.  Runs only for foams
+// whose need_remove flag is set; the next controller clears it.
+void launch_apply(const Grid &g);
+// removeBubbles by itself: the plan (sorted deletion list, moves), then the
+// above.  The caller clears the flag.
 void launch_remove(const Grid &g);
 
 // searchNeighbors: wrap + cell ids + counts, two-pass scan, binning,

@@ -379,7 +379,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FLOW ? 1
 k_pair_mixed(Foam *foams, const int2 *bt, uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
-    if (F->d.halt) return;
+    if (standing(F->d)) return;
     double soa = 0.0, soar = 0.0;
     bool near = false;
     mixed_block_dispatch<FLOW, false>(F, cx.lb, flags, soa, soar, near);
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(kBlock) void k_fix_mixed(Foam *foams, const int2 *b
                                                       uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
-    if (F->d.halt) return;
+    if (standing(F->d)) return;
     const int mark = F->s.part_i[cx.lb * kPartI + 2];
     if (!mark) return;
     double soa = 0.0, soar = 0.0;

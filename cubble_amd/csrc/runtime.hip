@@ -213,13 +213,15 @@ int time_search(Engine &e, int reps, cubble_search_times *out) {
     }
     if (!rc) rc = timed([&] { launch_search_part(g, kPartListKernel); }, kernel_ms);
     if (!rc) rc = timed([&] { launch_search_part(g, kPartReorder); }, reorder_ms);
-    // an attempt group's removal and search kernels when no foam needs them
+    // an attempt's removal launch and its share of a search phase when no foam
+    // needs them
     if (!rc) {
         launch_set_flags(g, 0, 0, 1);
         rc = timed([&] {
-            launch_remove(g);
+            for (int k = 0; k < kSearchEvery; ++k) launch_apply(g);
             launch_search(g);
         }, idle_ms);
+        idle_ms /= kSearchEvery;
     }
     for (auto &v : ev) (void)hipEventDestroy(v);
     const int rr = e.restore(snap);
@@ -393,6 +395,7 @@ int cubble_remove_bubbles(cubble_sim *s) {
     const Grid g = e.grid();
     launch_set_flags(g, -1, 1, 0);
     launch_remove(g);
+    launch_set_flags(g, -1, 0, 0);
     R_TRY(e, hipGetLastError());
     return e.sync();
 }

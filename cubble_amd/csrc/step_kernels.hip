@@ -23,6 +23,7 @@
 
 #include "dev_util.hpp"
 #include "launch.hpp"
+#include "remove_plan.hpp"
 
 namespace cubble_amd {
 
@@ -70,7 +71,7 @@ __device__ __forceinline__ void predict_dispatch(const Consts &c, const Roles &R
 __global__ __launch_bounds__(kBlock) void k_predict(Foam *foams, const int2 *bt, uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
-    if (F->d.halt) return;
+    if (standing(F->d)) return;
     const int n = F->d.count, ipt = F->ipt;
     const double h = 0.5 * F->d.dt;
     const Roles R = F->r;
@@ -200,7 +201,7 @@ template <bool FLOW>
 __global__ __launch_bounds__(kBlock) void k_pair(Foam *foams, const int2 *bt, uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
-    if (F->d.halt) return;
+    if (standing(F->d)) return;
     const int n = F->d.count, ipt = F->ipt;
     const Consts c = F->c;
     const Roles R = F->r;
@@ -228,10 +229,11 @@ __global__ __launch_bounds__(kBlock) void k_pair(Foam *foams, const int2 *bt, ui
 // One block per foam: S_A, S_Ar, S_OA, S_OAr from the predictor and pair
 // partials, in a fixed order.  (A separate launch: on MI355X the eight XCD
 // L2 caches are not coherent, so an in-kernel last-block reduction would
-// need an agent-scope release -- an L2 write-back -- in every block.)
+// need an agent-scope release -- an L2 write-back -- in every block.)  Foams
+// of at most kFuseBlocks blocks form the same sums in k_correct.
 __global__ __launch_bounds__(kBlock) void k_sums(Foam *foams) {
     Foam *F = foams + blockIdx.x;
-    if (F->d.halt) return;
+    if (standing(F->d) || F->nblk <= kFuseBlocks) return;
     double r[4];
     int none;
     reduce_parts4(F->s.part, F->s.part_i, F->nblk, 0, 0u, -1, r, none);
@@ -240,6 +242,29 @@ __global__ __launch_bounds__(kBlock) void k_sums(Foam *foams) {
         F->d.s_ar = r[1];
         F->d.s_oa = r[2];
         F->d.s_oar = r[3];
+    }
+}
+
+// S_A, S_Ar, S_OA, S_OAr of a foam of at most kFuseBlocks = kBlock blocks, by
+// every wave for itself and without a barrier: 64 block partials per round,
+// the rounds in order -- the waves of k_sums, so the same bits.  Reading them
+// again in every block of the corrector costs under a microsecond; the launch
+// of k_sums it replaces cost 2.5 us of a small foam's 46 us attempt.  Beyond
+// 256 blocks the reads grow with the square of the foam, and the launch is
+// the cheaper one.
+__device__ __forceinline__ void wave_foam_sums(const double *__restrict__ part, int nb,
+                                               double (&r)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[k] = 0.0;
+    for (int b0 = 0; b0 < nb; b0 += 64) {
+        const int b = b0 + (int)(threadIdx.x & 63);
+        double v[4] = {0.0, 0.0, 0.0, 0.0};
+        if (b < nb) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = part[b * kPartD + k];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) r[k] += wave_sum(v[k]);
     }
 }
 
@@ -382,7 +407,8 @@ __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, c
 }
 
 // dt controller and commit: reference src/simulator.cu:239-246, :258-321.
-__device__ void control(Foam *F, uint32_t flags, const CorrAcc &a) {
+// Returns whether the step removes bubbles.
+__device__ bool control(Foam *F, uint32_t flags, const CorrAcc &a) {
     Dyn &d = F->d;
     const Consts &c = F->c;
     d.s_v = a.s_v;
@@ -402,7 +428,8 @@ __device__ void control(Foam *F, uint32_t flags, const CorrAcc &a) {
     }
     d.dt = ndt;
     d.accepted = too_large ? 0 : 1;
-    if (too_large || !(flags & kCommit)) return;
+    d.need_remove = 0;  // the last one is done
+    if (too_large || !(flags & kCommit)) return false;
     const bool gas = (flags & kGas) != 0;
     Roles &R = F->r;
     for (int k = 0; k < 4; ++k) {
@@ -436,6 +463,7 @@ __device__ void control(Foam *F, uint32_t flags, const CorrAcc &a) {
     d.ts_max = fmax(d.ts_max, ndt);
     d.ts_sum += ndt;
     if (stop_reached(d)) d.halt = 1;
+    return d.need_remove != 0;
 }
 
 template <int D, bool M, bool W>
@@ -459,13 +487,28 @@ template <bool MIXED, bool WALLS>
 __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt, uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
-    if (F->d.halt) return;
+    if (standing(F->d)) return;
     const int n = F->d.count, ipt = F->ipt;
     const Consts c = F->c;
     const Roles R = F->r;
     const Scratch S = F->s;
-    const Dyn dyn = F->d;
+    Dyn dyn = F->d;
     const int base = cx.lb * kBlock * ipt;
+    if (F->nblk <= kFuseBlocks) {
+        double r[4];
+        wave_foam_sums(S.part, F->nblk, r);
+        dyn.s_a = r[0];
+        dyn.s_ar = r[1];
+        dyn.s_oa = r[2];
+        dyn.s_oar = r[3];
+        // for the host; the other blocks use their own
+        if (0 == cx.lb && 0 == threadIdx.x) {
+            F->d.s_a = r[0];
+            F->d.s_ar = r[1];
+            F->d.s_oa = r[2];
+            F->d.s_oar = r[3];
+        }
+    }
     CorrAcc a{0.0, 0.0, 0.0, 0.0, 0};
     if (3 == c.dim) correct_dispatch<3, MIXED, WALLS>(c, R, S, dyn, base, ipt, n, flags, a);
     else correct_dispatch<2, MIXED, WALLS>(c, R, S, dyn, base, ipt, n, flags, a);
@@ -483,10 +526,17 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
 }
 
 // One block per foam: reduce the corrector partials, then the dt controller
-// and (when committing) the role rotation.
+// and (when committing) the role rotation and the plan of a removal, which
+// the next launch applies.
 __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags) {
     Foam *F = foams + blockIdx.x;
-    if (F->d.halt) return;
+    if (standing(F->d)) {
+        // the removal of its last step is done
+        if (0 == threadIdx.x) F->d.need_remove = 0;
+        return;
+    }
+    __shared__ int s_del;
+    const int n = F->d.count;
     // the volume sum, the maxima of error, radius and expansion, the
     // deletion count
     double r[4];
@@ -499,8 +549,10 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
         t.max_r = r[2];
         t.max_exp = r[3];
         t.n_del = nd;
-        control(F, flags, t);
+        s_del = control(F, flags, t) ? nd : 0;
     }
+    __syncthreads();
+    if (s_del > 0) plan_removal(F, n, s_del);
 }
 
 // ---------------------------------------------------------------- launches
@@ -519,7 +571,7 @@ void launch_pair(const Grid &g, uint32_t flags) {
 }
 
 void launch_sums(const Grid &g) {
-    hipLaunchKernelGGL(k_sums, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams);
+    if (g.big) hipLaunchKernelGGL(k_sums, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams);
 }
 
 // AB2 bootstrap of init (reference src/simulator.cu:739-787): the Euler step
