@@ -105,9 +105,9 @@ void shape_foam(Foam &F, const Tuning &t) {
     const int cap = F.cap;
     F.ipt = t.ipt > 0 ? t.ipt : std::max(1, (cap + kBlock * kMaxBlocks - 1) / (kBlock * kMaxBlocks));
     F.nblk = std::max(1, (cap + kBlock * F.ipt - 1) / (kBlock * F.ipt));
-    F.stile = std::max(kMinSearchTile, t.stile > 0 ? t.stile : 256);
-    // tile t holds the cells whose first bubble is in [t B, t B + B); bubbles
-    // are below the capacity, so t runs to cap / B
+    F.stile = std::max(kMinSearchTile, t.stile);
+    // tile t searches for the bubbles [t B, t B + B); bubbles are below the
+    // capacity, so t runs to cap / B
     F.sblk = F.cap / F.stile + 1;
 }
 
@@ -461,9 +461,12 @@ Grid Engine::grid() const {
     g.nfoams = (int)foams.size();
     g.stream = stream;
     g.walls = g.big = false;
+    g.search_threads = 64;
     for (const FoamRec &r : foams) {
         for (int a = 0; a < r.h.c.dim; ++a) g.walls = g.walls || r.h.c.wall[a] != 0;
         g.big = g.big || r.h.nblk > kFuseBlocks;
+        g.search_threads =
+            std::max(g.search_threads, std::min(kBlock, (r.h.stile + 63) / 64 * 64));
     }
     return g;
 }
@@ -491,7 +494,7 @@ int Engine::capture(uint32_t flags, int groups) {
     // (walls or not, a sums launch or not)
     const Grid g = grid();
     if (graph_ && graph_flags_ == flags && graph_groups_ == groups && graph_walls_ == g.walls &&
-        graph_big_ == g.big)
+        graph_big_ == g.big && graph_threads_ == g.search_threads)
         return CUBBLE_OK;
     if (graph_) {
         (void)hipGraphExecDestroy(graph_);
@@ -511,6 +514,7 @@ int Engine::capture(uint32_t flags, int groups) {
     graph_groups_ = groups;
     graph_walls_ = g.walls;
     graph_big_ = g.big;
+    graph_threads_ = g.search_threads;
     return CUBBLE_OK;
 }
 

@@ -44,14 +44,17 @@ class DeviceArena {
     bool add_chunk(size_t bytes);
 };
 
+// Smallest search workgroup, in bubbles: one matrix tile.  It is the default:
+// twice as many, shorter waves cover the list kernel's latencies best (batch
+// of 256 foams 1.21 ms against 1.36 at 64, 3D foam of 1e5 0.104 / 0.142 ms;
+// only at 1e6 64 is the faster, 0.240 / 0.226 ms of a search every 25 steps).
+constexpr int kMinSearchTile = 32;
+
 struct Tuning {
     int ipt = 0;       // bubbles per thread (0 = from the size)
-    int stile = 256;   // bubbles per neighbour-search tile
+    int stile = kMinSearchTile;  // bubbles per neighbour-search workgroup
     int groups = 16;   // attempt groups per captured graph replay
 };
-
-// Smallest neighbour-search tile, in bubbles.
-constexpr int kMinSearchTile = 32;
 
 // Attempts between two search phases of a captured run.  A search is needed
 // every 20 to 80 steps (14 in the first steps after seeding), and its seven
@@ -184,6 +187,7 @@ class Engine {
     uint32_t graph_flags_ = 0;
     int graph_groups_ = 0;
     bool graph_walls_ = false, graph_big_ = false;
+    int graph_threads_ = 0;
     int committed_nf_ = 0;  // foams in the device array at the last commit
 
   public:

@@ -17,6 +17,7 @@ struct Grid {
     int nb_cell;
     const int2 *bt_scell;  // neighbour-search grid (Foam::stile bubbles per tile)
     int nb_scell;
+    int search_threads;    // threads of a search workgroup: 64 per 64 bubbles of a tile
     int nfoams;
     hipStream_t stream;
     bool walls;  // some foam of the launch has a wall
