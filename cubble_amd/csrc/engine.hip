@@ -88,15 +88,13 @@ size_t carve_foam(Foam &F, char *base) {
     S.cell_count = L.take<int32_t>((size_t)F.cell_cap);
     S.cell_cursor = L.take<int32_t>((size_t)F.cell_cap);
     S.cell_start = L.take<int32_t>((size_t)F.cell_cap + 1);
-    // block partials sized for the smallest launch shapes (one bubble per
-    // thread, kMinSearchTile bubbles per search tile), so retuning never
-    // reallocates
+    // block partials sized for the smallest launch shape (one bubble per
+    // thread), so retuning never reallocates
     const size_t nblk_max = ((size_t)F.cap + kBlock - 1) / kBlock;
-    const size_t sblk_max = (size_t)F.cap / kMinSearchTile + 1;
     S.part = L.take<double>(nblk_max * kPartD);
     S.part_i = L.take<int32_t>(nblk_max * kPartI);
     S.cpart = L.take<int32_t>((size_t)F.cblk);
-    S.cpart_i = L.take<int32_t>(sblk_max * kPartI);
+    S.cpart_i = L.take<int32_t>((size_t)kSearchParts * kPartI);
     return L.off;
 }
 

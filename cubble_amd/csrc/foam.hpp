@@ -22,6 +22,7 @@ constexpr int kBlock = 256;         // threads per block, bubble- and cell-space
 constexpr int kMaxBlocks = 2048;    // bubble-space blocks per foam (partials)
 constexpr int kNumXcd = 8;          // MI355X: 8 XCDs, workgroups round-robin
 constexpr int kFuseBlocks = 256;    // foams of at most this many blocks sum their partials in k_correct
+constexpr int kSearchParts = 64;    // records the search workgroups add their totals to
 constexpr int kPartD = 8;           // doubles per block partial record
 constexpr int kPartI = 4;           // ints per block partial record
 
@@ -90,7 +91,7 @@ struct Scratch {
     double *part;        // bubble-space block partials [nblk][kPartD]
     int32_t *part_i;     // bubble-space block partials [nblk][kPartI]
     int32_t *cpart;      // cell-space block partials (cell-count sums)
-    int32_t *cpart_i;    // neighbour-search tile partials [sblk][kPartI]
+    int32_t *cpart_i;    // neighbour-search totals [kSearchParts][kPartI]
     int32_t *del_list;   // sorted deleted indices
     int32_t *plan_src;   // source (tail survivor) of hole k
     int32_t *moved_to;   // new slot of tail survivor (old index - new count)

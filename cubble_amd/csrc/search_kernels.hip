@@ -27,6 +27,7 @@
 
 #include "dev_util.hpp"
 #include "launch.hpp"
+#include "tiles.hpp"
 
 namespace cubble_amd {
 
@@ -282,38 +283,6 @@ __device__ void swap_reordered_roles(Roles &W) {
     W.idx_alt = u;
 }
 
-// Sorted, de-duplicated neighbour coordinates of cell coordinate `x` along
-// one axis: periodic axes wrap, wall axes drop out-of-range cells.  With
-// fewer than 3 cells the wrapped offsets coincide and appear once.  Held in
-// three named values, not an array, so no kernel indexes private memory.
-struct AxisCells {
-    int v0, v1, v2, n;
-    __device__ __forceinline__ int at(int k) const { return 0 == k ? v0 : 1 == k ? v1 : v2; }
-};
-
-__device__ __forceinline__ AxisCells axis_cells(int x, int n, bool wall) {
-    AxisCells r;
-    if (wall) {
-        const bool lo = x - 1 >= 0, hi = x + 1 < n;
-        r.v0 = lo ? x - 1 : x;
-        r.v1 = lo ? x : x + 1;
-        r.v2 = x + 1;
-        r.n = 1 + (lo ? 1 : 0) + (hi ? 1 : 0);
-        return r;
-    }
-    int v0 = (x - 1 + n) % n, v1 = x, v2 = (x + 1) % n, t;
-    if (v0 > v1) { t = v0; v0 = v1; v1 = t; }
-    if (v1 > v2) { t = v1; v1 = v2; v2 = t; }
-    if (v0 > v1) { t = v0; v0 = v1; v1 = t; }
-    // drop duplicates, keeping order
-    const bool d1 = v1 == v0, d2 = v2 == v1;
-    r.v0 = v0;
-    r.v1 = d1 ? v2 : v1;
-    r.v2 = v2;
-    r.n = 3 - (d1 ? 1 : 0) - (d2 ? 1 : 0);
-    return r;
-}
-
 // The x-cells of one row as at most two runs of consecutive cells,
 // [a0, b0] and (if two) [a1, b1], in ascending order.
 struct XRuns {
@@ -331,32 +300,6 @@ __device__ __forceinline__ XRuns x_runs(const AxisCells &X) {
     r.two = f0 + 1 < X.n;
     r.a1 = r.two ? X.at(f0 + 1) : 0;
     r.b1 = r.two ? X.at(X.n - 1) : -1;
-    return r;
-}
-
-// The x-cells [x0 - 1, x0 + k] around k consecutive own cells x0 .. x0 + k - 1
-// of one row, as at most two runs in ascending order, each with its image
-// code as `side` gives it for a neighbour cell (0; 1: the run lies past the
-// high end, its candidates take d - L; 2: past the low end, d + L).  On a
-// periodic axis k + 4 <= n, so the window wraps at one end at most and a
-// cell appears once.  A pair of cells more than one apart in the window is
-// at least a cell width apart under either image, so it never holds a pair
-// within reach.
-struct XWindow {
-    int a0, b0, f0, a1, b1, f1;
-    bool two;
-};
-
-__device__ __forceinline__ XWindow x_window(int x0, int k, int n, bool wall) {
-    XWindow r{x0 - 1, x0 + k, 0, 0, -1, 0, false};
-    if (wall) {
-        r.a0 = max(r.a0, 0);
-        r.b0 = min(r.b0, n - 1);
-    } else if (x0 - 1 < 0) {  // [0, x0 + k], then cell n - 1 past the low end
-        r = XWindow{0, x0 + k, 0, n - 1, n - 1, 2, true};
-    } else if (x0 + k >= n) {  // cells past the high end first, then [x0 - 1, n - 1]
-        r = XWindow{0, x0 + k - n, 1, x0 - 1, n - 1, 0, true};
-    }
     return r;
 }
 
@@ -410,15 +353,14 @@ __device__ __forceinline__ void finish_group(int cb, int nb, int cnt, int nbr_ca
 // wave-uniform scalar loads; hits are found with a wave ballot and appended
 // to that bubble's list in lane order, which keeps every list ascending.
 // Lists longer than the capacity are counted, never written out of bounds.
-// `cell` must be wave-uniform.  A function of its own: its loops would raise
-// the register use of the common path.
+// `cell` must be wave-uniform.
 struct ListTotals {
     int sum_nn, max_nn, ovf;
 };
 
 template <int D>
-__device__ __forceinline__ ListTotals search_cell_general(const Foam *F, int cell,
-                                                                    int i0, int i1) {
+__device__ __forceinline__ ListTotals search_cell_general(const Foam *F, int cell, int i0,
+                                                          int i1) {
     const Consts &c = F->c;
     const auto x4 = gmem(F->s.x4);
     const auto x4s = cmem(F->s.x4);
@@ -483,47 +425,7 @@ __device__ __forceinline__ ListTotals search_cell_general(const Foam *F, int cel
     return sum;
 }
 
-constexpr int kMaxRuns = 18;    // 3 z-rows x 3 y-rows x 2 x-runs
 constexpr int kOwnUnit = 32;    // own bubbles per work unit of the general path
-constexpr int kSub = 32;        // own bubbles per matrix tile
-constexpr int kWindow = 10;     // most own cells of one row in a tile
-constexpr int kSegment = 512;   // candidate places per pass of a tile
-// Error bound of the matrix product's |d|^2 - (r_i + r_j + skin)^2 for a pair
-// within reach, or nearly so, relative to Q, which bounds |u|^2 + r^2 of own
-// bubbles and candidates (u relative to the window's centre).  In units of
-// 2^-22 Q: rounding the coordinates and radii to FP32 1, their split into two
-// FP16 values (2^-22 each, both sides) 4, the products of the two low parts
-// left out 2, the FP32 norms and their split 4, sixteen products added with
-// partial sums of at most 2 Q 8.  Pairs farther apart have a larger value by
-// more than their error grows.
-constexpr float kBand = 0x1.6p-18f;  // 22 2^-22
-constexpr float kFar = 3e4f;         // norm of an empty place: never a hit
-
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-
-union Operand {  // eight FP16 values of a lane: half the K range of its row
-    uint32_t u[4];
-    v8h h;
-};
-
-// a, b rounded to FP16, and what that leaves of them.
-__device__ __forceinline__ uint32_t pack_hi(float a, float b) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2h));
-}
-__device__ __forceinline__ uint32_t pack_lo(float a, float b, uint32_t hi) {
-    const v2h h = __builtin_bit_cast(v2h, hi);
-    return pack_hi(a - (float)h.x, b - (float)h.y);
-}
-
-// Sixteen candidate places of one run: bubbles j0 .. j0 + n - 1, and the
-// run's image code.
-struct Piece {
-    int j0;
-    int n_code;  // n | code << 8
-};
 
 // LDS of one wave: the hit masks of its two tiles over a segment of
 // candidates (word w of own bubble o: places 32 w .. 32 w + 31), and the
@@ -533,43 +435,10 @@ struct SearchLds {
     Piece piece[2][kSegment / 16];
 };
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// A wave-uniform value of vector arithmetic, into scalar registers.
-__device__ __forceinline__ double uniform_d(double v) { return readlane_d(v, 0); }
-__device__ __forceinline__ float uniform_f(float v) {
-    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-
-// One tile: own bubbles [i0, i0 + n), n <= kSub, in at most kWindow
-// consecutive cells of one row, and its candidates: the bubbles of the rows
-// around, from one cell before the own cells to one after.
-struct Tile {
-    int i0, n;
-    int total;                          // candidate places, 16 per piece
-    int run_piece, run_j, run_len, run_code;  // lane s: run s (first piece, ...)
-    double o[3];                        // window centre
-    float q_max, scale;                 // norm bound; power of two: cells of about 1
-    Operand own;
-    bool force;                         // an own bubble outside the bound
-};
-
-// Lane l's own bubble, position i0 + l of the span, and its cell.  (Its record
-// is loaded again for each tile: eight registers over the loops otherwise.)
-struct Own {
-    int i, cx, cy, cz;
-};
-
 template <int D>
 __device__ __forceinline__ Own load_own(const Consts &c, const D4 *__restrict__ x4, const int cd[3],
                                         int i) {
 #pragma clang fp contract(off)
-    Own w;
-    w.i = i;
     const D4 r = load_rec(gmem(x4) + i);
     const double p[3] = {r.x, r.y, r.z};
     // the cell as k_s_cells forms it
@@ -579,117 +448,33 @@ __device__ __forceinline__ Own load_own(const Consts &c, const D4 *__restrict__ 
         const double f = floor(cd[q] * (p[q] - c.lbb[q]) / c.interval[q]);
         id[q] = f < 0.0 ? 0 : (f >= (double)cd[q] ? cd[q] - 1 : (int)f);
     }
-    w.cx = id[0];
-    w.cy = id[1];
-    w.cz = id[2];
-    return w;
-}
-
-// The three cells around x of an axis of n >= 5 cells (or any number between
-// walls) in ascending order; wrapped cells first or last.
-__device__ __forceinline__ AxisCells near_cells(int x, int n, bool wall) {
-    const bool lo = x > 0, hi = x + 1 < n;
-    AxisCells r;
-    if (wall) {
-        r.n = 1 + (lo ? 1 : 0) + (hi ? 1 : 0);
-        r.v0 = lo ? x - 1 : x;
-        r.v1 = r.v0 + 1;
-        r.v2 = r.v0 + 2;
-        return r;
-    }
-    r.n = 3;
-    r.v0 = !lo || !hi ? 0 : x - 1;
-    r.v1 = !lo ? 1 : !hi ? n - 2 : x;
-    r.v2 = !lo || !hi ? n - 1 : x + 1;
-    return r;
-}
-
-// Inclusive prefix sum over lanes 0-31 (DPP row shifts; the second row of 16
-// adds the first one's total).
-__device__ __forceinline__ int prefix_32(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-    const int row = __builtin_amdgcn_readlane(v, 15);
-    return (int)(threadIdx.x & 63) >= 16 ? v + row : v;
+    return Own{i, id[0], id[1], id[2]};
 }
 
 // The tile of the own bubbles from lane q0 of the span on, `left` of them at
-// most.  e: the cell edges.
+// most, and the centre o of its window.  e: the cell edges.
 template <int D>
-__device__ __forceinline__ void tile_setup(Tile &t, const Consts &c, const Own &w,
-                                           const D4 *__restrict__ x4, const int *__restrict__ start_, const int cd[3],
+__device__ __forceinline__ void tile_setup(Tile &t, double o[3], const Consts &c, const Own &w,
+                                           const D4 *__restrict__ x4,
+                                           const int *__restrict__ start, const int cd[3],
                                            const double e[3], double rmax, int span0, int q0,
                                            int left) {
-    const auto start = gmem(start_);
-    const int lane = (int)(threadIdx.x & 63);
     t.i0 = span0 + q0;
     t.n = 0;
     t.total = 0;
     if (left <= 0) return;
-    const int ccx = __builtin_amdgcn_readlane(w.cx, q0);
-    const int ccy = __builtin_amdgcn_readlane(w.cy, q0);
-    const int ccz = 3 == D ? __builtin_amdgcn_readlane(w.cz, q0) : 0;
-    const int kmax = min(kWindow, c.wall[0] ? cd[0] : cd[0] - 4);
-    // positions are in cell order: those of the row's next kmax cells come first
-    const bool in = lane >= q0 && lane < q0 + min(left, kSub) && w.cy == ccy &&
-                    (2 == D || w.cz == ccz) && w.cx < ccx + kmax;
-    t.n = __popcll(__builtin_amdgcn_ballot_w64(in));
-    const int kx = __builtin_amdgcn_readlane(w.cx, q0 + t.n - 1) - ccx + 1;
-    const AxisCells Y = near_cells(ccy, cd[1], c.wall[1] != 0);
-    const AxisCells Z = 3 == D ? near_cells(ccz, cd[2], c.wall[2] != 0) : AxisCells{0, 0, 0, 1};
-    const XWindow xw = x_window(ccx, kx, cd[0], c.wall[0] != 0);
-    // 0: neighbour cell a of own cell b does not cross the boundary; 1: its
-    // bubbles' image lies at x + L; 2: at x - L
-    auto side = [](int a, int b) { return b - a > 1 ? 1 : (a - b > 1 ? 2 : 0); };
-    {
-        const int r = lane >> 1, part = lane & 1;
-        const int a = r / 3, b = r % 3;
-        const bool ok = lane < kMaxRuns && a < Z.n && b < Y.n && (0 == part || xw.two);
-        const int zc = Z.at(a), yc = Y.at(b);
-        const int row = (zc * cd[1] + yc) * cd[0];
-        const int js = ok ? start[row + (0 == part ? xw.a0 : xw.a1)] : 0;
-        const int je = ok ? start[row + (0 == part ? xw.b0 : xw.b1) + 1] : 0;
-        t.run_j = js;
-        t.run_len = je - js;
-        t.run_code = (side(yc, ccy) << 2) | (side(zc, ccz) << 4) | (0 == part ? xw.f0 : xw.f1);
-        // a run starts a piece of its own
-        const int np = (t.run_len + 15) >> 4;
-        const int incl = prefix_32(np);
-        t.run_piece = incl - np;
-        t.total = 16 * __builtin_amdgcn_readlane(incl, kMaxRuns - 1);
-    }
-    const D4 wp = load_rec(gmem(x4) + w.i);
-    t.o[0] = uniform_d(c.lbb[0] + (ccx + 0.5 * kx) * e[0]);
-    t.o[1] = uniform_d(c.lbb[1] + (ccy + 0.5) * e[1]);
-    t.o[2] = 3 == D ? uniform_d(c.lbb[2] + (ccz + 0.5) * e[2]) : 0.0;
-    const double hx = (0.5 * kx + 1.0) * e[0], hy = 1.5 * e[1], hz = 1.5 * e[2],
+    const bool wall[3] = {c.wall[0] != 0, c.wall[1] != 0, c.wall[2] != 0};
+    const bool in = tile_runs<D>(t, w, start, cd, wall, span0, q0, left);
+    o[0] = uniform_d(c.lbb[0] + (t.cx + 0.5 * t.kx) * e[0]);
+    o[1] = uniform_d(c.lbb[1] + (t.cy + 0.5) * e[1]);
+    o[2] = 3 == D ? uniform_d(c.lbb[2] + (t.cz + 0.5) * e[2]) : 0.0;
+    const double hx = (0.5 * t.kx + 1.0) * e[0], hy = 1.5 * e[1], hz = 1.5 * e[2],
                  hr = rmax + c.skin;
     t.q_max = uniform_f((float)(1.001 * (hx * hx + hy * hy + hz * hz + hr * hr)));
-    const float ux = (float)(wp.x - t.o[0]), uy = (float)(wp.y - t.o[1]);
-    const float uz = 3 == D ? (float)(wp.z - t.o[2]) : 0.f;
-    const float ur = (float)(wp.r + c.skin);
-    const float d2 = fmaf(ux, ux, fmaf(uy, uy, uz * uz));
-    t.force = __builtin_amdgcn_ballot_w64(in && !(fmaf(ur, ur, d2) <= t.q_max)) != 0ull;
-    // the own operand of the own bubble that lane q0 + (lane mod 32) holds:
-    // lanes 0-31 (x y z r) high twice, lanes 32-63 (x y z r) low, 1, 1 and
-    // the norm's two parts
-    const float sc = t.scale, nr = fmaf(-ur, ur, d2) * (sc * sc);
-    const uint32_t h0 = pack_hi(ux * sc, uy * sc), h1 = pack_hi(uz * sc, ur * sc);
-    const uint32_t l0 = pack_lo(ux * sc, uy * sc, h0), l1 = pack_lo(uz * sc, ur * sc, h1);
-    const float nh = (float)(_Float16)nr;
-    const uint32_t n2 = pack_hi(nh, nr - nh);
-    const int ow = lane & (kSub - 1), from = (q0 + ow) & 63;
-    const bool have = ow < t.n, half = lane >= kSub;
-    const uint32_t s0 = __shfl((int)(h0), from), s1 = __shfl((int)(h1), from);
-    const uint32_t s2 = __shfl((int)(l0), from), s3 = __shfl((int)(l1), from);
-    const uint32_t s4 = __shfl((int)(n2), from);
-    const uint32_t one = pack_hi(1.f, 1.f), far = pack_hi(kFar, 0.f);
-    t.own.u[0] = have ? (half ? s2 : s0) : 0u;
-    t.own.u[1] = have ? (half ? s3 : s1) : 0u;
-    t.own.u[2] = half ? one : (have ? s0 : 0u);
-    t.own.u[3] = half ? (have ? s4 : far) : (have ? s1 : 0u);
+    // (the record is loaded again: eight registers over the loops otherwise)
+    const D4 p = load_rec(gmem(x4) + w.i);
+    own_operand(t, in, q0, (float)(p.x - o[0]), (float)(p.y - o[1]),
+                3 == D ? (float)(p.z - o[2]) : 0.f, (float)(p.r + c.skin));
 }
 
 // Tiles the FP32 values do not settle (bit 2 k + q of `marks`: candidates
@@ -738,43 +523,17 @@ struct Chunk {
     D4 p;
 };
 
-// The hit masks of candidates [seg, seg + kSegment) of a tile, decided as the
-// FP64 test decides them.
-//
-// |d|^2 - (r_i + r_j + skin)^2 with both points relative to the window's
-// centre is N_i + N_j - 2 (u_i . u_j + r_i' r_j), N = |u|^2 - r^2: a product
-// of the own operand (u, r', 1, N_i) with the candidate's (-2u, -2r, N_j, 1).
-// With every factor split into two FP16 values, a = a_h + a_l, and a_l b_l
-// left out, that is a product over K = 16 -- a_h b_h and a_l b_h in lanes
-// 0-31's half, a_h b_l and the norms in lanes 32-63's --, so 32 candidates
-// against 32 own bubbles are one 32x32x16 matrix instruction (32 cycles of
-// the matrix cores for 1024 pairs; three FP32 ones take 192, and as FP64
-// vector instructions the same tests took 13 each).  A lane ends with one own
-// bubble and 16 candidates; their sign bits are its part of the mask.  Where
-// a value lies within the rounding bound of zero, or a bubble outside the
-// bound's window, the tile's pairs are decided again in FP64.
+// The hit masks of candidates [seg, seg + kSegment) of a tile with window
+// centre o, decided as the FP64 test decides them.
 template <int D>
-__device__ __forceinline__ void tile_masks(const Tile &t, const Consts &c,
+__device__ __forceinline__ void tile_masks(const Tile &t, const double o[3], const Consts &c,
                                            const Foam *F, int seg, int h, SearchLds &lds) {
     const auto x4 = gmem(F->s.x4);
-    const int lane = (int)(threadIdx.x & 63), ow = lane & (kSub - 1);
-    // the row of a candidate is placed so that a lane's 16 rows are 16
-    // consecutive candidates
-    const int m = lane & 31;
-    const int slot = (lane & 32) | (((m >> 2) & 1) << 4) | ((m >> 3) << 2) | (m & 3);
+    const int lane = (int)(threadIdx.x & 63), ow = lane & (kSub - 1), slot = candidate_slot();
     const int p_end = min(seg + kSegment, t.total);
     const float eps = kBand * t.q_max * (t.scale * t.scale);
     Piece *const piece = lds.piece[h];
-    // the segment's pieces, each run's by its lane; the places after the last
-    // run hold none
-    if (lane < 4) piece[min((p_end - seg) / 16 + lane, kSegment / 16 - 1)] = Piece{0, 0};
-    wave_sync();
-    for (int k = 0; __builtin_amdgcn_ballot_w64(16 * k < t.run_len) != 0ull; ++k) {
-        const int g = t.run_piece + k - (seg >> 4);
-        if (16 * k < t.run_len && g >= 0 && g < kSegment / 16)
-            piece[g] = Piece{t.run_j + 16 * k, min(16, t.run_len - 16 * k) | t.run_code << 8};
-    }
-    wave_sync();
+    tile_pieces(t, seg, piece);
     auto fetch = [&](int p0) {
         const int g = min(p0 - seg + slot, kSegment - 1);
         const Piece pc = piece[g >> 4];
@@ -789,8 +548,7 @@ __device__ __forceinline__ void tile_masks(const Tile &t, const Consts &c,
     Chunk k = fetch(seg);
 #pragma unroll 1
     for (int p0 = seg; p0 < p_end; p0 += 64) {
-        const bool valid = k.j >= 0;
-        double ox = t.o[0], oy = t.o[1], oz = t.o[2];
+        double ox = o[0], oy = o[1], oz = o[2];
         if (__builtin_amdgcn_ballot_w64(k.f != 0) != 0ull) {
             // the candidate's image at x + L or x - L
             auto shift = [&](int a) {
@@ -802,58 +560,15 @@ __device__ __forceinline__ void tile_masks(const Tile &t, const Consts &c,
             oy -= shift(1);
             if (3 == D) oz -= shift(2);
         }
-        const float ux = (float)(k.p.x - ox), uy = (float)(k.p.y - oy);
-        const float uz = 3 == D ? (float)(k.p.z - oz) : 0.f;
-        const float ur = (float)k.p.r;
-        const float d2 = fmaf(ux, ux, fmaf(uy, uy, uz * uz));
-        const bool exact =
-            t.force || __builtin_amdgcn_ballot_w64(valid && !(fmaf(ur, ur, d2) <= t.q_max)) != 0ull;
-        const float m2 = -2.f * t.scale;
-        const uint32_t h0 = pack_hi(ux * m2, uy * m2), h1 = pack_hi(uz * m2, ur * m2);
-        const uint32_t l0 = pack_lo(ux * m2, uy * m2, h0), l1 = pack_lo(uz * m2, ur * m2, h1);
-        // a place without a candidate: any operand with the norm of one far away
-        const float nr = valid ? fmaf(-ur, ur, d2) * (t.scale * t.scale) : kFar;
-        const float nh = (float)(_Float16)nr;
-        const uint32_t n2 = pack_hi(nh, nr - nh), one = pack_hi(1.f, 1.f);
-        // the K halves of candidates 0-31 and of 32-63
-        Operand op[2];
-        auto halves = [&](int d, uint32_t a, uint32_t b) {
-            const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-            op[0].u[d] = r[0];
-            op[1].u[d] = r[1];
-        };
-        halves(0, h0, h0);
-        halves(1, h1, h1);
-        halves(2, l0, n2);
-        halves(3, l1, one);
+        const ChunkOperand op =
+            chunk_operand(t, k.j >= 0, (float)(k.p.x - ox), (float)(k.p.y - oy),
+                          3 == D ? (float)(k.p.z - oz) : 0.f, (float)k.p.r);
         // the next chunk's records are in flight while this one is tested
         // (past the end too: a branch around the loads would wait for them)
         k = fetch(p0 + 64);
-        uint32_t w16[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const v16f acc =
-                __builtin_amdgcn_mfma_f32_32x32x16_f16(op[q].h, t.own.h, v16f{}, 0, 0, 0);
-            uint32_t w = 0;
-            float near = kFar;
-#pragma unroll
-            for (int r = 15; r >= 0; --r) {
-                w = __builtin_amdgcn_alignbit(w, __float_as_uint(acc[r]), 31);
-                near = fminf(near, fabsf(acc[r]));
-            }
-            // (no branch: it would hold the products of both halves in registers)
-            const unsigned mark =
-                (exact | (__builtin_amdgcn_ballot_w64(near <= eps) != 0ull)) ? 1u : 0u;
-            marks |= mark << (((p0 - seg) >> 5) + q);
-            w16[q] = w;
-        }
-        // words of candidates p0 .. p0 + 31 (lanes 0-31) and p0 + 32 .. (lanes
-        // 32-63) of own bubble ow, from the halves of both
-        const uint32_t w = w16[0] | (w16[1] << 16);
-        const auto x = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-        const uint32_t word = lane < 32 ? (x[0] & 0xffffu) | (x[1] << 16)
-                                        : (x[0] >> 16) | (x[1] & 0xffff0000u);
-        lds.mask[h][((p0 - seg) >> 5) + (lane >> 5)][ow] = word;
+        unsigned mk;
+        lds.mask[h][((p0 - seg) >> 5) + (lane >> 5)][ow] = chunk_words(t, op, eps, mk);
+        marks |= mk << ((p0 - seg) >> 5);
     }
     if (marks) {
         wave_sync();
@@ -912,11 +627,13 @@ __device__ __forceinline__ void search_span(const Foam *F, const Consts &c, cons
 #pragma unroll 1
             for (int g = 0; g < 2; ++g) {
                 Tile t;
+                double o[3];
                 t.scale = scale;
-                tile_setup<D>(t, c, own, S.x4, S.cell_start, cd, e, rmax, span0, next, all - next);
+                tile_setup<D>(t, o, c, own, S.x4, S.cell_start, cd, e, rmax, span0, next,
+                              all - next);
                 next += t.n;
                 most = max(most, t.total);
-                if (seg < t.total) tile_masks<D>(t, c, F, seg, g, lds);
+                if (seg < t.total) tile_masks<D>(t, o, c, F, seg, g, lds);
                 if (h == g) {
                     have = ow < t.n;
                     i = t.i0 + ow;
@@ -992,7 +709,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
     for (int k = 0; k < 3; ++k)
         if (k < c.dim) {
             if (!c.wall[k] && cd[k] < 5) fast = false;
-            if (!((2.0 * rmax + c.skin) * 1.000001 <= c.interval[k] / cd[k])) fast = false;
+            const double e = c.interval[k] / cd[k];
+            if (!((2.0 * rmax + c.skin) * 1.000001 <= e)) fast = false;
+            if (!(e > 1e-12 && e < 1e12)) fast = false;  // within FP32's squares
         }
     const int w = (int)(threadIdx.x >> 6), nw = (int)(blockDim.x >> 6);
     if (fast) {
@@ -1041,28 +760,34 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) 
             max_nn = max(max_nn, s_red[1][k]);
             ovf = max(ovf, s_red[2][k]);
         }
-        S.cpart_i[cx.lb * kPartI + 1] = sum_nn;
-        S.cpart_i[cx.lb * kPartI + 2] = max_nn;
-        S.cpart_i[cx.lb * kPartI + 3] = ovf;
+        int32_t *const p = S.cpart_i + (cx.lb & (kSearchParts - 1)) * kPartI;
+        atomicAdd(p + 1, sum_nn);
+        atomicMax(p + 2, max_nn);
+        if (ovf) atomicMax(p + 3, ovf);
     }
 }
 
+// (The workgroups' totals are integers, added with atomics to kSearchParts
+// records of the foam; one record per workgroup took a workgroup per foam 157
+// us to reduce at 4e6 bubbles.)
+//
 // One block per foam: make the reordered buffers current (swap = 1), pair
 // count, list-capacity check, counters.
-__global__ __launch_bounds__(kBlock) void k_s_fin(Foam *foams, int swap) {
+__global__ __launch_bounds__(kSearchParts) void k_s_fin(Foam *foams, int swap) {
     Foam *F = foams + blockIdx.x;
     if (!F->d.need_search) return;
     const Scratch S = F->s;
-    const int nb = F->sblk;
     int s = 0, mx = 0, of = 0;
-    for (int b = threadIdx.x; b < nb; b += kBlock) {
-        s += S.cpart_i[b * kPartI + 1];
-        mx = max(mx, S.cpart_i[b * kPartI + 2]);
-        of = max(of, S.cpart_i[b * kPartI + 3]);
+    if ((int)threadIdx.x < min(F->sblk, kSearchParts)) {
+        int32_t *const p = S.cpart_i + (int)threadIdx.x * kPartI;
+        s = p[1];
+        mx = p[2];
+        of = p[3];
+        p[1] = p[2] = p[3] = 0;  // for the next search
     }
-    const int tot = block_sum_i(s);
-    mx = block_max_i(mx);
-    of = block_max_i(of);
+    const int tot = wave_sum_i(s);
+    mx = wave_max_i(mx);
+    of = wave_max_i(of);
     if (threadIdx.x == 0) {
         if (swap) swap_reordered_roles(F->r);
         F->d.num_pairs = tot / 2;
@@ -1117,12 +842,12 @@ void launch_search(const Grid &g) {
     hipLaunchKernelGGL(k_s_bin, dim3(g.nb_bub), dim3(kBlock), 0, g.stream, g.foams, g.bt_bub);
     hipLaunchKernelGGL(k_s_reorder, dim3(g.nb_bub), dim3(kBlock), 0, g.stream, g.foams, g.bt_bub);
     launch_lists(g);
-    hipLaunchKernelGGL(k_s_fin, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams, 1);
+    hipLaunchKernelGGL(k_s_fin, dim3(g.nfoams), dim3(kSearchParts), 0, g.stream, g.foams, 1);
 }
 
 void launch_search_lists(const Grid &g) {
     launch_lists(g);
-    hipLaunchKernelGGL(k_s_fin, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams, 0);
+    hipLaunchKernelGGL(k_s_fin, dim3(g.nfoams), dim3(kSearchParts), 0, g.stream, g.foams, 0);
 }
 
 void launch_search_part(const Grid &g, int part) {
