@@ -188,6 +188,35 @@ __device__ __forceinline__ int block_excl_scan(int v, int &total) {
     return wo + x - v;
 }
 
+// Runs of equal keys among the wave's valid lanes (bubbles are in the cell
+// order of the previous search, so neighbouring lanes mostly share a cell):
+// `heads` has a bit for the first lane of each run; a head's run ends at the
+// next head or at the last valid lane.  One atomic per run instead of one per
+// bubble.
+struct WaveRuns {
+    unsigned long long heads;
+    int len;   // run length (valid on head lanes)
+    int head;  // lane of this lane's run head
+};
+
+__device__ __forceinline__ WaveRuns wave_runs(int key, bool valid) {
+    const int lane = (int)(threadIdx.x & 63);
+    const int prev = __shfl_up(key, 1);
+    const bool is_head = valid && (0 == lane || prev != key);
+    const unsigned long long heads = __builtin_amdgcn_ballot_w64(is_head);
+    const unsigned long long vmask = __builtin_amdgcn_ballot_w64(valid);
+    // valid lanes are a prefix of the wave (consecutive bubbles below n)
+    const int nvalid = __popcll(vmask);
+    const unsigned long long above = lane < 63 ? heads & (~0ull << (lane + 1)) : 0ull;
+    const int end = above ? __builtin_ctzll(above) : nvalid;
+    const unsigned long long upto = heads & (lane < 63 ? (2ull << lane) - 1ull : ~0ull);
+    WaveRuns r;
+    r.heads = heads;
+    r.len = end - lane;
+    r.head = upto ? 63 - __builtin_clzll(upto) : 0;
+    return r;
+}
+
 // ---- geometry (bit-identical to the FP64 restatement) --------------------
 
 // Minimum-image difference a - b: reference src/kernels.cu:1094-1114.

@@ -31,35 +31,6 @@
 
 namespace cubble_amd {
 
-// Runs of equal keys among the wave's valid lanes (bubbles are in the cell
-// order of the previous search, so neighbouring lanes mostly share a cell):
-// `heads` has a bit for the first lane of each run; a head's run ends at the
-// next head or at the last valid lane.  One atomic per run instead of one per
-// bubble.
-struct WaveRuns {
-    unsigned long long heads;
-    int len;   // run length (valid on head lanes)
-    int head;  // lane of this lane's run head
-};
-
-__device__ __forceinline__ WaveRuns wave_runs(int key, bool valid) {
-    const int lane = (int)(threadIdx.x & 63);
-    const int prev = __shfl_up(key, 1);
-    const bool is_head = valid && (0 == lane || prev != key);
-    const unsigned long long heads = __builtin_amdgcn_ballot_w64(is_head);
-    const unsigned long long vmask = __builtin_amdgcn_ballot_w64(valid);
-    // valid lanes are a prefix of the wave (consecutive bubbles below n)
-    const int nvalid = __popcll(vmask);
-    const unsigned long long above = lane < 63 ? heads & (~0ull << (lane + 1)) : 0ull;
-    const int end = above ? __builtin_ctzll(above) : nvalid;
-    const unsigned long long upto = heads & (lane < 63 ? (2ull << lane) - 1ull : ~0ull);
-    WaveRuns r;
-    r.heads = heads;
-    r.len = end - lane;
-    r.head = upto ? 63 - __builtin_clzll(upto) : 0;
-    return r;
-}
-
 template <int D>
 __device__ __forceinline__ double cells_range(const Consts &c, const Roles &R, const Scratch &S,
                                               const int cd[3], int base, int ipt, int n) {
@@ -477,43 +448,24 @@ __device__ __forceinline__ void tile_setup(Tile &t, double o[3], const Consts &c
                 3 == D ? (float)(p.z - o[2]) : 0.f, (float)(p.r + c.skin));
 }
 
-// Tiles the FP32 values do not settle (bit 2 k + q of `marks`: candidates
-// 64 k + 32 q .. of the segment), decided in FP64: each lane its own bubble i
-// against its 16 candidates of the tile, into its half of the mask word.
-// Rare, and apart from the loop over the candidates, whose registers it would
-// share.
+// Pair (i, j) as the FP64 test decides it.
 template <int D>
-__device__ __forceinline__ void exact_tiles(const Foam *F, const Piece *piece, uint32_t *mask,
-                                            unsigned marks, int i, int n) {
+__device__ __forceinline__ bool pair_hit(const Foam *F, const D4 &pi, const D4 &pj) {
 #pragma clang fp contract(off)
-    const auto x4 = gmem(F->s.x4);
     const auto c = cmem(&F->c);  // scalar loads where they are used
-    const int lane = (int)(threadIdx.x & 63), ow = lane & (kSub - 1), half = lane >> 5;
-    const D4 pi = load_rec(x4 + (ow < n ? i : i - ow));
-    for (; marks; marks &= marks - 1u) {
-        const int tile = __builtin_ctz(marks);
-        const Piece pc = piece[2 * tile + half];
-        const int cnt = pc.n_code & 0xff;
-        uint32_t w = 0;
-#pragma unroll 1
-        for (int r = 0; r < 16; ++r) {
-            const D4 pj = load_rec(x4 + (r < cnt ? pc.j0 + r : i - ow));
-            // wrapped_diff, sq_len
-            const double d1[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
-            double m = 0;
+    // wrapped_diff, sq_len
+    const double d1[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+    double m = 0;
 #pragma unroll
-            for (int k = 0; k < D; ++k) {
-                const double a = d1[k] < 0 ? -d1[k] : d1[k];
-                const double t = c->interval[k] - a;
-                const double image = d1[k] < 0 ? t : -t;
-                const double d = !c->wall[k] && t * t < d1[k] * d1[k] ? image : d1[k];
-                m += d * d;
-            }
-            const double maxd = pi.r + pj.r + c->skin;
-            if (r < cnt && ow < n && m < maxd * maxd) w |= 1u << r;
-        }
-        reinterpret_cast<uint16_t *>(mask)[2 * (tile * kSub + ow) + half] = (uint16_t)w;
+    for (int k = 0; k < D; ++k) {
+        const double a = d1[k] < 0 ? -d1[k] : d1[k];
+        const double t = c->interval[k] - a;
+        const double image = d1[k] < 0 ? t : -t;
+        const double d = !c->wall[k] && t * t < d1[k] * d1[k] ? image : d1[k];
+        m += d * d;
     }
+    const double maxd = pi.r + pj.r + c->skin;
+    return m < maxd * maxd;
 }
 
 // A chunk of 64 candidates, one per lane: bubble (-1: none), image code and
@@ -544,10 +496,7 @@ __device__ __forceinline__ void tile_masks(const Tile &t, const double o[3], con
         k.p = load_rec(x4 + (unsigned)(valid ? k.j : t.i0));
         return k;
     };
-    unsigned marks = 0;  // tiles to decide in FP64
-    Chunk k = fetch(seg);
-#pragma unroll 1
-    for (int p0 = seg; p0 < p_end; p0 += 64) {
+    auto operand = [&](const Chunk &k) {
         double ox = o[0], oy = o[1], oz = o[2];
         if (__builtin_amdgcn_ballot_w64(k.f != 0) != 0ull) {
             // the candidate's image at x + L or x - L
@@ -560,9 +509,14 @@ __device__ __forceinline__ void tile_masks(const Tile &t, const double o[3], con
             oy -= shift(1);
             if (3 == D) oz -= shift(2);
         }
-        const ChunkOperand op =
-            chunk_operand(t, k.j >= 0, (float)(k.p.x - ox), (float)(k.p.y - oy),
-                          3 == D ? (float)(k.p.z - oz) : 0.f, (float)k.p.r);
+        return chunk_operand(t, k.j >= 0, (float)(k.p.x - ox), (float)(k.p.y - oy),
+                             3 == D ? (float)(k.p.z - oz) : 0.f, (float)k.p.r);
+    };
+    unsigned marks = 0;  // halves of chunks to settle in FP64
+    Chunk k = fetch(seg);
+#pragma unroll 1
+    for (int p0 = seg; p0 < p_end; p0 += 64) {
+        const ChunkOperand op = operand(k);
         // the next chunk's records are in flight while this one is tested
         // (past the end too: a branch around the loads would wait for them)
         k = fetch(p0 + 64);
@@ -570,9 +524,28 @@ __device__ __forceinline__ void tile_masks(const Tile &t, const double o[3], con
         lds.mask[h][((p0 - seg) >> 5) + (lane >> 5)][ow] = chunk_words(t, op, eps, mk);
         marks |= mk << ((p0 - seg) >> 5);
     }
-    if (marks) {
-        wave_sync();
-        exact_tiles<D>(F, piece, &lds.mask[h][0][0], marks, t.i0 + ow, t.n);
+    if (!marks) return;
+    wave_sync();
+    const D4 pi = load_rec(x4 + t.i0 + (ow < t.n ? ow : 0));
+    uint16_t *const half = reinterpret_cast<uint16_t *>(&lds.mask[h][0][ow]) + (lane >> 5);
+#pragma unroll 1
+    for (; marks; marks &= marks - 1u) {
+        const int tile = __builtin_ctz(marks);
+        const ChunkOperand op = operand(fetch(seg + 32 * (tile & ~1)));
+        const Piece pc = piece[2 * tile + (lane >> 5)];
+        const int cnt = ow < t.n ? pc.n_code & 0xff : 0;
+        // (places without a candidate too: an own bubble far outside has no
+        // sign to go by)
+        const uint32_t places = (1u << cnt) - 1u;
+        uint32_t open = chunk_open(t, op, tile & 1, eps) & places;
+        uint32_t w = half[2 * kSub * tile] & places;
+        while (open) {
+            const int r = __builtin_ctz(open);
+            open &= open - 1u;
+            const bool hit = pair_hit<D>(F, pi, load_rec(x4 + pc.j0 + r));
+            w = hit ? w | 1u << r : w & ~(1u << r);
+        }
+        half[2 * kSub * tile] = (uint16_t)w;
     }
 }
 
@@ -596,9 +569,9 @@ __device__ __forceinline__ void tile_masks(const Tile &t, const double o[3], con
 // 13 FP64 operations each and appended the hits of each ballot: bound by
 // instruction issue (VALU 69%, SALU 62% of the cycles).  List kernel, same
 // foams: 3D 1e6 0.49 -> 0.24 ms, 3D 1e5 (mixed, 45 bubbles a cell) 0.20 ->
-// 0.10 ms, batch of 256 foams 2.09 -> 1.21 ms, 2D 1e4 0.017 ms both.  Its
-// bound now is latency at five waves per SIMD (a wave waits in two thirds of
-// its cycles); four, with ten registers more and no spills, are 4% slower.
+// 0.094 ms, batch of 256 foams 2.09 -> 1.23 ms, 2D 1e4 17 -> 11 us.  Its
+// bound now is latency at four waves per SIMD (a wave waits in two thirds of
+// its cycles); five, with 25 registers spilled, are 15% slower.
 template <int D>
 __device__ __forceinline__ void search_span(const Foam *F, const Consts &c, const Scratch &S,
                                             const int cd[3], size_t cap, int nbr_cap, double rmax,
@@ -686,7 +659,7 @@ __device__ __forceinline__ void search_span(const Foam *F, const Consts &c, cons
 // cells hold a few bubbles, crowded 3D ones a hundred and more).  A wave
 // takes 64 of them; the workgroup has as many waves as a tile has spans of
 // 64, at most kWaves.
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_s_search(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_s_search(
     Foam *foams, const int2 *bt) {
     const Ctx cx = cell_ctx(foams, bt);
     Foam *F = cx.F;

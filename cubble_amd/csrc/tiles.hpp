@@ -333,4 +333,20 @@ __device__ __forceinline__ uint32_t chunk_words(const Tile &t, const ChunkOperan
                                    : (x[0] >> 16) | (x[1] & 0xffff0000u);
 }
 
+// The places of half q (0, 1) of a chunk that the product does not settle, as
+// this lane's 16 bits of them: for the halves chunk_words marked, formed again
+// apart from the loop over the chunks, whose registers they would share.
+__device__ __forceinline__ uint32_t chunk_open(const Tile &t, const ChunkOperand &k, int q,
+                                               float eps) {
+    if (k.exact) return 0xffffu;
+    Operand op;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) op.u[d] = q ? k.op[1].u[d] : k.op[0].u[d];
+    const v16f acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(op.h, t.own.h, v16f{}, 0, 0, 0);
+    uint32_t w = 0;
+#pragma unroll
+    for (int r = 15; r >= 0; --r) w |= fabsf(acc[r]) <= eps ? 1u << r : 0u;
+    return w;
+}
+
 }  // namespace cubble_amd

@@ -85,16 +85,18 @@ def test_crowded_cells(ora, dim, n, big, tile):
 
 
 @pytest.mark.parametrize("dim,wall", [(2, (1, 1, 0)), (3, (1, 1, 1)), (3, (1, 0, 0))])
-def test_bubbles_outside_a_walled_box(ora, dim, wall):
+@pytest.mark.parametrize("reach", [9.0, 1e7])
+def test_bubbles_outside_a_walled_box(ora, dim, wall, reach):
     """Bubbles pushed past a wall stay in the edge cell, outside the window
-    the matrix product's bound covers."""
+    the matrix product's bound covers (and, far away, the range of its
+    factors)."""
     print(f"search outside dim={dim} wall={wall}", flush=True)
     n = 3000
     sim = ca.Simulator(config(dim, n, seed=31 + dim, wall=wall))
     st, sc = sim.get_state()
     rng = np.random.default_rng(dim)
     out = rng.permutation(n)[:60]
-    st["x"][0][out[:30]] = -rng.uniform(0.0, 9.0, 30)
-    st["x"][0][out[30:]] = sc["tfr"][0] + rng.uniform(0.0, 9.0, 30)
+    st["x"][0][out[:30]] = -rng.uniform(0.0, reach, 30)
+    st["x"][0][out[30:]] = sc["tfr"][0] + rng.uniform(0.0, reach, 30)
     _search_equals_oracle(ora, sim, st, sc)
     sim.close()
