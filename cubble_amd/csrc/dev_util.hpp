@@ -56,28 +56,81 @@ __device__ __forceinline__ Ctx cell_ctx(Foam *foams, const int2 *bt) {
 }
 
 // ---- deterministic reductions (fixed butterfly, every lane identical) ----
+// v and lane l ^ step's v, for the steps 32, 16, 8, 4, 2, 1 of a butterfly in
+// that order, by lane swaps and DPP: no LDS, whose round trip (a hundred
+// cycles a step and value) was a large part of a small kernel's end.  From
+// step 8 on all lanes of equal l mod (2 step) hold the same value, so a
+// rotation in the row of 16 by `step` reaches l ^ step's.
+template <int STEP>
+__device__ __forceinline__ void butterfly(uint32_t v, uint32_t &a, uint32_t &b) {
+    if (32 == STEP) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        a = r[0];
+        b = r[1];
+    } else if (16 == STEP) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        a = r[0];
+        b = r[1];
+    } else {
+        // row_ror:8, row_ror:4, quad_perm 2 3 0 1, quad_perm 1 0 3 2
+        constexpr int ctrl = 8 == STEP ? 0x128 : 4 == STEP ? 0x124 : 2 == STEP ? 0x4e : 0xb1;
+        a = v;
+        b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xf, 0xf, true);
+    }
+}
+
+template <int STEP, typename Op>
+__device__ __forceinline__ double wave_step(double v, Op op) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    uint32_t al, bl, ah, bh;
+    butterfly<STEP>((uint32_t)u, al, bl);
+    butterfly<STEP>((uint32_t)(u >> 32), ah, bh);
+    return op(__longlong_as_double((long long)((uint64_t)ah << 32 | al)),
+              __longlong_as_double((long long)((uint64_t)bh << 32 | bl)));
+}
+
+template <int STEP, typename Op>
+__device__ __forceinline__ int wave_step(int v, Op op) {
+    uint32_t a, b;
+    butterfly<STEP>((uint32_t)v, a, b);
+    return op((int)a, (int)b);
+}
+
+template <int STEP, typename Op>
+__device__ __forceinline__ float wave_step(float v, Op op) {
+    uint32_t a, b;
+    butterfly<STEP>(__float_as_uint(v), a, b);
+    return op(__uint_as_float(a), __uint_as_float(b));
+}
+
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_all(T v, Op op) {
+    v = wave_step<32>(v, op);
+    v = wave_step<16>(v, op);
+    v = wave_step<8>(v, op);
+    v = wave_step<4>(v, op);
+    v = wave_step<2>(v, op);
+    return wave_step<1>(v, op);
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    return wave_all(v, [](double a, double b) { return a + b; });
 }
 
 __device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
-    return v;
+    return wave_all(v, [](double a, double b) { return fmax(a, b); });
 }
 
 __device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    return wave_all(v, [](int a, int b) { return a + b; });
 }
 
 __device__ __forceinline__ int wave_max_i(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-    return v;
+    return wave_all(v, [](int a, int b) { return max(a, b); });
+}
+
+__device__ __forceinline__ float wave_sum_f(float v) {
+    return wave_all(v, [](float a, float b) { return a + b; });
 }
 
 constexpr int kWaves = kBlock / 64;
@@ -250,10 +303,11 @@ __device__ __forceinline__ int uniform_i(int v) { return __builtin_amdgcn_readfi
 
 // Neighbour gather of bubble i over its list (column-major, nbr[q * cap + i])
 // in chunks of kGather: the chunk's list entries are loaded, then all their
-// records, then `body(j, record)` runs for each in ascending list order.  A
-// lane's loads of one chunk are independent, so their latencies overlap
-// instead of adding up entry by entry.  Past the end of the list a lane
-// re-reads its own record and skips the body.
+// records, then `body(j[], record[])` runs on them, ascending.  A lane's loads
+// of one chunk are independent, so their latencies overlap instead of adding
+// up entry by entry; a body without branches lets the chunk's arithmetic
+// overlap too.  Past the end of the list a lane re-reads its own record, with
+// j = -1.
 constexpr int kGather = 4;
 
 // The buffers live in device global memory; pointers read from the foam
@@ -316,9 +370,7 @@ __device__ __forceinline__ void for_neighbours(const int *__restrict__ nbr_,
 #pragma unroll
         for (int u = 0; u < kGather; ++u) cur[u] = js[u];
         if (q0 + kGather < m_nn) load_ids(q0 + kGather, js);
-#pragma unroll
-        for (int u = 0; u < kGather; ++u)
-            if (cur[u] >= 0) body(cur[u], pj[u]);
+        body(cur, pj);
     }
 }
 

@@ -21,7 +21,8 @@ namespace cubble_amd {
 constexpr int kBlock = 256;         // threads per block, bubble- and cell-space
 constexpr int kMaxBlocks = 2048;    // bubble-space blocks per foam (partials)
 constexpr int kNumXcd = 8;          // MI355X: 8 XCDs, workgroups round-robin
-constexpr int kFuseBlocks = 256;    // foams of at most this many blocks sum their partials in k_correct
+constexpr int kFuseBlocks = 128;    // launches of foams of at most this many blocks sum their
+                                    // partials in k_correct
 constexpr int kSearchParts = 64;    // records the search workgroups add their totals to
 constexpr int kPartD = 8;           // doubles per block partial record
 constexpr int kPartI = 4;           // ints per block partial record
@@ -173,6 +174,7 @@ enum Flags : uint32_t {
     kPath = 2u,
     kCommit = 4u,
     kFlow = 8u,
+    kOwnSums = 16u,  // the corrector forms the foam's sums itself
 };
 
 }  // namespace cubble_amd

@@ -29,9 +29,9 @@ void launch_pair(const Grid &g, uint32_t flags);
 // The mixed pair kernel, then (fix) the second pass over the bubbles that met
 // a pair needing FP64 values.
 void launch_pair_mixed(const Grid &g, uint32_t flags, bool fix = true);
-// S_A, S_Ar, S_OA, S_OAr of foams of more than kFuseBlocks blocks, from the
-// predictor and pair partials (one block per foam; the others sum their own
-// in the corrector)
+// S_A, S_Ar, S_OA, S_OAr from the predictor and pair partials (one block per
+// foam), when some foam of the launch has more than kFuseBlocks blocks;
+// otherwise the corrector forms them
 void launch_sums(const Grid &g);
 // corrector (mixed: the mixed-precision variant, for engines of that
 // precision), then (control) the dt controller / commit and the plan of a

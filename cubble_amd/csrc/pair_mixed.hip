@@ -248,18 +248,16 @@ __device__ __forceinline__ void mixed_block(const Consts &c, const Roles &R, con
         zero_out(o);
         bool near = false;
         for_neighbours(S.nbr, S.q4, cap, i, S.nn[i],
-                       [&](int j, const Q4 &qj) { near = pair(j, qj, o) || near; });
+                       [&](const int(&js)[kGather], const Q4(&qs)[kGather]) {
+#pragma unroll
+                           for (int u = 0; u < kGather; ++u)
+                               if (js[u] >= 0) near = pair(js[u], qs[u], o) || near;
+                       });
         store_mixed<D, GAS, FLOW>(c, R, S, h, i, o, near);
         near_any = near_any || near;
         soa += (double)o.ovl;
         soar += (double)o.ovl * (1.0 / (double)qi.r);
     }
-}
-
-__device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
 }
 
 // Flagged bubble i (wave-uniform) summed again by the whole wave, the values

@@ -111,53 +111,74 @@ __device__ __forceinline__ void pair_range(const Consts &c, const Roles &R, cons
     const int *__restrict__ nnA = S.nn;
     const int *__restrict__ nbr = S.nbr;
     const double f0 = c.f0;
+    // below it, a difference is its own minimum image
+    double near[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) near[a] = c.wall[a] ? __builtin_inf() : 0.49 * c.interval[a];
     for (int k = 0; k < ipt; ++k) {
         const int i = base + k * kBlock + (int)threadIdx.x;
         if (i >= n) break;
         const D4 pi = p4[i];
         const double xi = pi.x, yi = pi.y, zi = pi.z, ri = pi.r;
-        const double inv_ri = 1.0 / ri;
+        const double inv_ri = 1.0 / ri, risq = ri * ri;
         double acc[3] = {0.0, 0.0, 0.0};
         double fv[3] = {0.0, 0.0, 0.0};
         double ovl = 0.0, dr = 0.0;
         const int m_nn = nnA[i];
-        for_neighbours(nbr, p4, cap, i, m_nn, [&](int j, const D4 &pj) {
-            const double rj = pj.r;
-            const double r1 = i < j ? ri : rj;
-            const double r2 = i < j ? rj : ri;
-            const double radii = r1 + r2;
-            double d[3];
-            wrapped_diff<D>(c, xi, yi, zi, pj.x, pj.y, pj.z, d);
-            const double m = sq_len(d);
-            if (FLOW && (j < i || radii * radii >= m)) {
+        for_neighbours(nbr, p4, cap, i, m_nn, [&](const int(&js)[kGather],
+                                                  const D4(&ps)[kGather]) {
+            double d[kGather][3];
+            bool far = false;
 #pragma unroll
-                for (int a = 0; a < D; ++a) fv[a] += field<double>(R.v[a])[j];
+            for (int u = 0; u < kGather; ++u) {
+                d[u][0] = xi - ps[u].x;
+                d[u][1] = yi - ps[u].y;
+                d[u][2] = 3 == D ? zi - ps[u].z : 0.0;
+#pragma unroll
+                for (int a = 0; a < D; ++a) far = far || fabs(d[u][a]) > near[a];
             }
-            if (radii * radii >= m) {
+            // the minimum image, for waves with a pair across the boundary
+            // (one in five at 35 cells an axis)
+            if (__builtin_amdgcn_ballot_w64(far) != 0ull) {
+#pragma unroll
+                for (int u = 0; u < kGather; ++u)
+                    wrapped_diff<D>(c, xi, yi, zi, ps[u].x, ps[u].y, ps[u].z, d[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < kGather; ++u) {
+                const int j = js[u];
+                const double rj = ps[u].r;
+                const double radii = ri + rj;
+                const double m = sq_len(d[u]);
+                const bool on = j >= 0 && radii * radii >= m;
+                if (FLOW && j >= 0 && (j < i || on)) {
+#pragma unroll
+                    for (int a = 0; a < D; ++a) fv[a] += field<double>(R.v[a])[j];
+                }
                 const double rs = rsq_nr(m);
                 const double s = rs - rcp_nr(radii);
 #pragma unroll
-                for (int a = 0; a < D; ++a) acc[a] += d[a] * f0 * s;
+                for (int a = 0; a < D; ++a) {
+                    const double t = d[u][a] * f0 * s;
+                    acc[a] += on ? t : 0.0;
+                }
                 if (GAS) {
-                    const double r1sq = r1 * r1;
-                    const double r2sq = r2 * r2;
-                    double oa = 0;
-                    if (m < r1sq || m < r2sq) {
-                        oa = r1sq < r2sq ? r1sq : r2sq;
-                    } else {
-                        oa = 0.5 * (r2sq - r1sq + m);
-                        oa *= oa;
-                        oa *= rs * rs;  // / m
-                        oa = r2sq - oa;
-                        oa = oa < 0 ? -oa : oa;
-                    }
+                    const double rjsq = rj * rj;
+                    const double r1sq = i < j ? risq : rjsq;  // of the smaller index
+                    const double r2sq = i < j ? rjsq : risq;
+                    double oa = 0.5 * (r2sq - r1sq + m);
+                    oa *= oa;
+                    oa *= rs * rs;  // / m
+                    oa = fabs(r2sq - oa);
+                    if (m < r1sq || m < r2sq) oa = r1sq < r2sq ? r1sq : r2sq;
                     if (3 == D) {
                         oa *= kPi;
                     } else {
                         oa = 2.0 * sqrt(oa);
                     }
-                    ovl += oa;
-                    dr += oa * (rcp_nr(rj) - inv_ri);
+                    const double t = oa * (rcp_nr(rj) - inv_ri);
+                    ovl += on ? oa : 0.0;
+                    dr += on ? t : 0.0;
                 }
             }
         });
@@ -196,9 +217,18 @@ __device__ __forceinline__ void reduce_parts4(const double *part, const int32_t 
 }
 
 // One kernel per FLOW value: the flow variant needs more registers, which
-// would otherwise lower the occupancy of the plain one.
+// would otherwise lower the occupancy of the plain one (96: five waves a SIMD).
+//
+// The body has no branch per neighbour: the four chains of a chunk overlap,
+// where one after another each waited for its own square root and
+// reciprocals (2D 1e4: 9.0 -> 7.5 us a launch), and terms that do not count
+// are selected away (adding 0).  At 1e6 bubbles it is bound by the gathers'
+// cache accesses, 64 lines a load: 78 us either way, and neither six waves
+// (114 us, spilled) nor halves of records gathered by neighbouring lanes (110
+// us) help.
 template <bool FLOW>
-__global__ __launch_bounds__(kBlock) void k_pair(Foam *foams, const int2 *bt, uint32_t flags) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FLOW ? 4 : 5, 8))) void
+k_pair(Foam *foams, const int2 *bt, uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
     if (standing(F->d)) return;
@@ -229,11 +259,10 @@ __global__ __launch_bounds__(kBlock) void k_pair(Foam *foams, const int2 *bt, ui
 // One block per foam: S_A, S_Ar, S_OA, S_OAr from the predictor and pair
 // partials, in a fixed order.  (A separate launch: on MI355X the eight XCD
 // L2 caches are not coherent, so an in-kernel last-block reduction would
-// need an agent-scope release -- an L2 write-back -- in every block.)  Foams
-// of at most kFuseBlocks blocks form the same sums in k_correct.
+// need an agent-scope release -- an L2 write-back -- in every block.)
 __global__ __launch_bounds__(kBlock) void k_sums(Foam *foams) {
     Foam *F = foams + blockIdx.x;
-    if (standing(F->d) || F->nblk <= kFuseBlocks) return;
+    if (standing(F->d)) return;
     double r[4];
     int none;
     reduce_parts4(F->s.part, F->s.part_i, F->nblk, 0, 0u, -1, r, none);
@@ -245,13 +274,12 @@ __global__ __launch_bounds__(kBlock) void k_sums(Foam *foams) {
     }
 }
 
-// S_A, S_Ar, S_OA, S_OAr of a foam of at most kFuseBlocks = kBlock blocks, by
+// S_A, S_Ar, S_OA, S_OAr of a foam of at most kFuseBlocks <= kBlock blocks, by
 // every wave for itself and without a barrier: 64 block partials per round,
 // the rounds in order -- the waves of k_sums, so the same bits.  Reading them
-// again in every block of the corrector costs under a microsecond; the launch
-// of k_sums it replaces cost 2.5 us of a small foam's 46 us attempt.  Beyond
-// 256 blocks the reads grow with the square of the foam, and the launch is
-// the cheaper one.
+// again in every block of the corrector costs it under a microsecond up to
+// two rounds; the launch of k_sums it replaces costs 2.5.  In a batch the
+// launch is the cheaper one: 256 foams' correctors took 36 us longer.
 __device__ __forceinline__ void wave_foam_sums(const double *__restrict__ part, int nb,
                                                double (&r)[4]) {
 #pragma unroll
@@ -494,7 +522,7 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
     const Scratch S = F->s;
     Dyn dyn = F->d;
     const int base = cx.lb * kBlock * ipt;
-    if (F->nblk <= kFuseBlocks) {
+    if (flags & kOwnSums) {
         double r[4];
         wave_foam_sums(S.part, F->nblk, r);
         dyn.s_a = r[0];
@@ -641,6 +669,7 @@ void launch_bootstrap(const Grid &g, bool mixed) {
 
 void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control) {
     const dim3 grid(g.nb_bub), block(kBlock);
+    if (!g.big) flags |= kOwnSums;
     if (mixed) {
         if (g.walls)
             hipLaunchKernelGGL((k_correct<true, true>), grid, block, 0, g.stream, g.foams,
