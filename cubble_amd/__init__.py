@@ -29,7 +29,7 @@ PREC_FP64, PREC_MIXED = 0, 1
 
 _dp = ctypes.POINTER(ctypes.c_double)
 _ip = ctypes.POINTER(ctypes.c_int32)
-_u8p = ctypes.POINTER(ctypes.c_uint8)
+_vp = ctypes.c_void_p  # arrays by address
 
 
 class CubbleError(RuntimeError):
@@ -72,15 +72,15 @@ class _Config(ctypes.Structure):
 
 
 class _StateView(ctypes.Structure):
-    _fields_ = [("x", _dp * 4), ("v", _dp * 4), ("vo", _dp * 4), ("saved", _dp * 4),
-                ("path", _dp), ("error", _dp), ("wrap", _ip * 3), ("index", _ip),
-                ("nbr_off", _ip), ("nbr", _ip), ("nbr_cap", ctypes.c_int64),
-                ("degree", _ip)]
+    _fields_ = [("x", _vp * 4), ("v", _vp * 4), ("vo", _vp * 4), ("saved", _vp * 4),
+                ("path", _vp), ("error", _vp), ("wrap", _vp * 3), ("index", _vp),
+                ("nbr_off", _vp), ("nbr", _vp), ("nbr_cap", ctypes.c_int64),
+                ("degree", _vp)]
 
 
 class _AttemptView(ctypes.Structure):
-    _fields_ = [("xc", _dp * 4), ("vp", _dp * 4), ("overlap", _dp), ("path_new", _dp),
-                ("deleted", _u8p)]
+    _fields_ = [("xc", _vp * 4), ("vp", _vp * 4), ("overlap", _vp), ("path_new", _vp),
+                ("deleted", _vp)]
 
 
 class _Scalars(ctypes.Structure):
@@ -446,6 +446,15 @@ def serving_requests(num_requests, rate_per_s=50.0, seed=77, precision=PREC_MIXE
     return out
 
 
+def _rows(field, a):
+    """The rows of the contiguous 2D array `a` as the pointers of `field`."""
+    if a.ndim != 2 or len(a) < len(field):
+        raise IndexError("needs %d rows, has shape %s" % (len(field), a.shape))
+    base, step = a.ctypes.data, a.strides[0]
+    for k in range(len(field)):
+        field[k] = base + k * step
+
+
 def _dptr(a):
     return a.ctypes.data_as(_dp)
 
@@ -548,7 +557,7 @@ class Simulator:
         the velocities, reduced on the device; with energy=True also each
         bubble's energy (state order)."""
         o = _Observables()
-        e = np.zeros(self.scalars()["count"]) if energy else None
+        e = np.empty(self._count()) if energy else None
         self._call(lib().cubble_observe(self._h, ctypes.byref(o),
                                         _dptr(e) if e is not None and len(e) else None))
         out = {name: (list(getattr(o, name)) if name == "mean_v" else getattr(o, name))
@@ -596,15 +605,20 @@ class Simulator:
         sc = self.scalars()
         return _read_state(sc, lambda v: self._call(lib().cubble_get_state(self._h, v))), sc
 
+    def _count(self):
+        s = _Scalars()
+        self._call(lib().cubble_get_scalars(self._h, ctypes.byref(s)))
+        return s.count
+
     def get_attempt(self):
-        n = self.scalars()["count"]
-        o = {"xc": np.zeros((4, n)), "vp": np.zeros((4, n)), "ov": np.zeros(n),
-             "path_new": np.zeros(n), "del": np.zeros(n, np.uint8)}
+        n = self._count()
+        o = {"xc": np.empty((4, n)), "vp": np.empty((4, n)), "ov": np.empty(n),
+             "path_new": np.empty(n), "del": np.empty(n, np.uint8)}
         a = _AttemptView()
-        for k in range(4):
-            a.xc[k], a.vp[k] = _dptr(o["xc"][k]), _dptr(o["vp"][k])
-        a.overlap, a.path_new = _dptr(o["ov"]), _dptr(o["path_new"])
-        a.deleted = o["del"].ctypes.data_as(_u8p)
+        _rows(a.xc, o["xc"])
+        _rows(a.vp, o["vp"])
+        a.overlap, a.path_new = o["ov"].ctypes.data, o["path_new"].ctypes.data
+        a.deleted = o["del"].ctypes.data
         self._call(lib().cubble_get_attempt(self._h, ctypes.byref(a)))
         return o
 
@@ -624,18 +638,16 @@ class Simulator:
 
         v = _StateView()
         x, vv, vo, sv = d(st["x"]), d(st["v"]), d(st["vo"]), d(st["saved"])
-        for k in range(4):
-            v.x[k], v.v[k], v.vo[k], v.saved[k] = _dptr(x[k]), _dptr(vv[k]), _dptr(vo[k]), _dptr(sv[k])
-        wc = i32(st["wc"])
-        for k in range(3):
-            v.wrap[k] = _iptr(wc[k])
+        for field, a in ((v.x, x), (v.v, vv), (v.vo, vo), (v.saved, sv)):
+            _rows(field, a)
+        _rows(v.wrap, i32(st["wc"]))
         path, err, idx = d(st["path"]), d(st["err"]), i32(st["idx"])
-        v.path, v.error, v.index = _dptr(path), _dptr(err), _iptr(idx)
+        v.path, v.error, v.index = path.ctypes.data, err.ctypes.data, idx.ctypes.data
         off = i32(st["nbr_off"])
         nbr = i32(st["nbr"] if len(st["nbr"]) else [0])
-        v.nbr_off, v.nbr, v.nbr_cap = _iptr(off), _iptr(nbr), len(st["nbr"])
+        v.nbr_off, v.nbr, v.nbr_cap = off.ctypes.data, nbr.ctypes.data, len(st["nbr"])
         if st.get("deg") is not None:
-            v.degree = _iptr(i32(st["deg"]))
+            v.degree = i32(st["deg"]).ctypes.data
         s = _Scalars()
         for name, _ in _Scalars._fields_:
             if name in scalars:
@@ -657,20 +669,18 @@ class Simulator:
 
 def _read_state(sc, fill):
     n = sc["count"]
-    st = {"x": np.zeros((4, n)), "v": np.zeros((4, n)), "vo": np.zeros((4, n)),
-          "saved": np.zeros((4, n)), "path": np.zeros(n), "err": np.zeros(n),
-          "wc": np.zeros((3, n), np.int32), "idx": np.zeros(n, np.int32),
-          "nbr_off": np.zeros(n + 1, np.int32), "deg": np.zeros(n, np.int32)}
-    nbr = np.zeros(max(1, sc["nbr_cap"] * n), np.int32)
+    # the call writes every element (and nbr up to the lists' total)
+    st = {"x": np.empty((4, n)), "v": np.empty((4, n)), "vo": np.empty((4, n)),
+          "saved": np.empty((4, n)), "path": np.empty(n), "err": np.empty(n),
+          "wc": np.empty((3, n), np.int32), "idx": np.empty(n, np.int32),
+          "nbr_off": np.empty(n + 1, np.int32), "deg": np.empty(n, np.int32)}
+    nbr = np.empty(max(1, sc["nbr_cap"] * n), np.int32)
     v = _StateView()
-    for k in range(4):
-        v.x[k], v.v[k] = _dptr(st["x"][k]), _dptr(st["v"][k])
-        v.vo[k], v.saved[k] = _dptr(st["vo"][k]), _dptr(st["saved"][k])
-    for k in range(3):
-        v.wrap[k] = _iptr(st["wc"][k])
-    v.path, v.error, v.index = _dptr(st["path"]), _dptr(st["err"]), _iptr(st["idx"])
-    v.nbr_off, v.nbr, v.nbr_cap = _iptr(st["nbr_off"]), _iptr(nbr), nbr.size
-    v.degree = _iptr(st["deg"])
+    for field, key in ((v.x, "x"), (v.v, "v"), (v.vo, "vo"), (v.saved, "saved"), (v.wrap, "wc")):
+        _rows(field, st[key])
+    v.path, v.error = st["path"].ctypes.data, st["err"].ctypes.data
+    v.index, v.degree = st["idx"].ctypes.data, st["deg"].ctypes.data
+    v.nbr_off, v.nbr, v.nbr_cap = st["nbr_off"].ctypes.data, nbr.ctypes.data, nbr.size
     fill(ctypes.byref(v))
     st["nbr"] = nbr[: st["nbr_off"][n]].copy()
     return st

@@ -23,7 +23,7 @@ CLI = os.path.join(HERE, "cubble-cli")
 ARCH = os.environ.get("CUBBLE_AMD_ARCH", "gfx950")
 
 HIP_SOURCES = ["step_kernels.hip", "pair_mixed.hip", "search_kernels.hip", "remove_kernels.hip",
-               "engine.hip", "state_io.hip", "runtime.hip", "server.hip", "autotune.hip",
+               "engine.hip", "state_io.hip", "readback.hip", "runtime.hip", "server.hip", "autotune.hip",
                "observe_kernels.hip", "pairs.hip", "pairs_noalloc.hip"]
 HOST_SOURCES = ["host_init.cpp", "cli.cpp"]
 

@@ -188,6 +188,7 @@ class Engine {
     int graph_groups_ = 0;
     bool graph_walls_ = false, graph_big_ = false;
     int graph_threads_ = 0;
+    bool opened_ = false;  // counted among the users of the pinned blocks
     int committed_nf_ = 0;  // foams in the device array at the last commit
 
   public:

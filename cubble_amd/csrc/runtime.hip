@@ -16,6 +16,7 @@
 #include "autotune.hpp"
 #include "cubble_amd.h"
 #include "engine.hpp"
+#include "readback.hpp"
 #include "foam.hpp"
 #include "host_init.hpp"
 #include "launch.hpp"
@@ -429,13 +430,14 @@ int cubble_observe(cubble_sim *s, cubble_observables *out, double *energy) {
     if (!buf) return e.fail(CUBBLE_E_NOMEM, "observe: no device memory");
     launch_observe(h, e.dfoams(), buf, energy ? buf + kPartD : nullptr, e.stream);
     double sums[kPartD];
-    hipError_t err = hipGetLastError();
-    if (hipSuccess == err) err = hipMemcpyAsync(sums, buf, sizeof(sums), hipMemcpyDeviceToHost, e.stream);
-    if (hipSuccess == err && energy && n > 0)
-        err = hipMemcpyAsync(energy, buf + kPartD, sizeof(double) * n, hipMemcpyDeviceToHost, e.stream);
-    if (hipSuccess == err) err = hipStreamSynchronize(e.stream);
+    Readback rb;
+    rb.f64(sums, buf, kPartD);
+    rb.f64(energy, buf + kPartD, (size_t)n);
+    const hipError_t err = hipGetLastError();
+    if (hipSuccess == err) rc = rb.run(e);
     e.arena.release(buf);
     R_TRY(e, err);
+    if (rc) return rc;
     out->total_energy = sums[0];
     out->total_volume = sums[1];
     out->box_volume = h.c.interval[0] * h.c.interval[1] * (3 == h.c.dim ? h.c.interval[2] : 1.0);

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "engine.hpp"
+#include "readback.hpp"
 
 namespace cubble_amd {
 
@@ -82,12 +83,6 @@ int get_scalars(Engine &e, int k, cubble_scalars *o) {
 }
 
 namespace {
-int d2h(Engine &e, void *dst, const void *src, size_t bytes) {
-    if (!dst || !bytes) return CUBBLE_OK;
-    R_TRY(e, hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
-    return CUBBLE_OK;
-}
-
 int h2d(Engine &e, void *dst, const void *src, size_t bytes) {
     if (!src || !bytes) return CUBBLE_OK;
     R_TRY(e, hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
@@ -96,14 +91,9 @@ int h2d(Engine &e, void *dst, const void *src, size_t bytes) {
 
 // Velocities, saved positions, error and overlap are FP32 in mixed precision,
 // FP64 otherwise; host views are FP64 in both.
-int d2h_field(Engine &e, const Foam &f, double *dst, const void *src, size_t n) {
-    if (!dst || !n) return CUBBLE_OK;
-    if (CUBBLE_PREC_MIXED != f.precision) return d2h(e, dst, src, n * sizeof(double));
-    std::vector<float> t(n);
-    int rc = d2h(e, t.data(), src, n * sizeof(float));
-    if (rc) return rc;
-    for (size_t i = 0; i < n; ++i) dst[i] = (double)t[i];
-    return CUBBLE_OK;
+void read_field(Readback &rb, const Foam &f, double *dst, const void *src, size_t n) {
+    if (CUBBLE_PREC_MIXED == f.precision) rb.f32_as_f64(dst, src, n);
+    else rb.f64(dst, src, n);
 }
 
 int h2d_field(Engine &e, const Foam &f, void *dst, const double *src, size_t n) {
@@ -122,49 +112,42 @@ int get_state(Engine &e, int k, cubble_state_view *v) {
     int rc = e.read_header(k, f);
     if (rc) return rc;
     const size_t n = (size_t)f.d.count;
-    const size_t db = n * sizeof(double), ib = n * sizeof(int32_t);
+    Readback rb;
     for (int q = 0; q < 4; ++q) {
         if (2 == q && 2 == f.c.dim) {
             for (double *p : {v->x[q], v->v[q], v->vo[q], v->saved[q]})
-                if (p) std::memset(p, 0, db);
+                if (p) std::memset(p, 0, n * sizeof(double));
             continue;
         }
-        if ((rc = d2h(e, v->x[q], f.r.x[q], db)) || (rc = d2h_field(e, f, v->v[q], f.r.v[q], n)) ||
-            (rc = d2h_field(e, f, v->vo[q], f.r.vo[q], n)) ||
-            (rc = d2h_field(e, f, v->saved[q], f.r.saved[q], n)))
-            return rc;
+        rb.f64(v->x[q], f.r.x[q], n);
+        read_field(rb, f, v->v[q], f.r.v[q], n);
+        read_field(rb, f, v->vo[q], f.r.vo[q], n);
+        read_field(rb, f, v->saved[q], f.r.saved[q], n);
     }
-    if ((rc = d2h(e, v->path, f.r.path, db)) || (rc = d2h_field(e, f, v->error, f.r.err, n)))
-        return rc;
+    rb.f64(v->path, f.r.path, n);
+    read_field(rb, f, v->error, f.r.err, n);
     for (int q = 0; q < 3; ++q) {
-        if (q >= f.c.dim) {
-            if (v->wrap[q]) std::memset(v->wrap[q], 0, ib);
-            continue;
-        }
-        if ((rc = d2h(e, v->wrap[q], f.r.wc[q], ib))) return rc;
+        if (q < f.c.dim) rb.i32(v->wrap[q], f.r.wc[q], n);
+        else if (v->wrap[q]) std::memset(v->wrap[q], 0, n * sizeof(int32_t));
     }
-    if ((rc = d2h(e, v->index, f.r.idx, ib)) || (rc = d2h(e, v->degree, f.s.deg, ib))) return rc;
-    if (v->nbr_off || v->nbr) {
-        std::vector<int32_t> nn(n);
-        if ((rc = d2h(e, nn.data(), f.s.nn, ib))) return rc;
-        int maxn = 0;
-        for (size_t i = 0; i < n; ++i) maxn = std::max(maxn, nn[i]);
-        std::vector<int32_t> ell((size_t)maxn * n);
-        if (maxn > 0)
-            R_TRY(e, hipMemcpy2D(ell.data(), n * sizeof(int32_t), f.s.nbr,
-                                 (size_t)f.cap * sizeof(int32_t), n * sizeof(int32_t), maxn,
-                                 hipMemcpyDeviceToHost));
-        int64_t tot = 0;
-        if (v->nbr_off) v->nbr_off[0] = 0;
-        for (size_t i = 0; i < n; ++i) {
-            if (v->nbr) {
-                if (tot + nn[i] > v->nbr_cap)
-                    return e.fail(CUBBLE_E_CAPACITY, "get_state: nbr buffer too small");
-                for (int q = 0; q < nn[i]; ++q) v->nbr[tot + q] = ell[(size_t)q * n + i];
-            }
-            tot += nn[i];
-            if (v->nbr_off) v->nbr_off[i + 1] = (int32_t)tot;
-        }
+    rb.i32(v->index, f.r.idx, n);
+    rb.i32(v->degree, f.s.deg, n);
+    int32_t total = 0;
+    if ((v->nbr_off || v->nbr) && n > 0) {
+        // (scratch of a removal, which runs as a whole within a step)
+        launch_list_ends(f.s.nn, (int)n, f.s.plan_src, f.s.moved_to, e.stream);
+        R_TRY(e, hipGetLastError());
+        rb.i32(&total, f.s.plan_src + (n - 1), 1);
+        if (v->nbr_off) rb.i32(v->nbr_off + 1, f.s.plan_src, n);
+    }
+    if (v->nbr_off) v->nbr_off[0] = 0;
+    if ((rc = rb.run(e))) return rc;
+    if (v->nbr && total > 0) {
+        if (total > v->nbr_cap)
+            return e.fail(CUBBLE_E_CAPACITY, "get_state: nbr buffer too small");
+        Readback lists;
+        lists.lists(v->nbr, f.s.plan_src, f.s.nbr, (size_t)f.cap, (int)n, (size_t)total);
+        return lists.run(e);
     }
     return CUBBLE_OK;
 }
@@ -175,21 +158,20 @@ int get_attempt(Engine &e, int k, cubble_attempt_view *v) {
     int rc = e.read_header(k, f);
     if (rc) return rc;
     const size_t n = (size_t)f.d.count;
-    const size_t db = n * sizeof(double);
+    Readback rb;
     for (int q = 0; q < 4; ++q) {
         if (2 == q && 2 == f.c.dim) {
-            if (v->xc[q]) std::memset(v->xc[q], 0, db);
-            if (v->vp[q]) std::memset(v->vp[q], 0, db);
+            for (double *p : {v->xc[q], v->vp[q]})
+                if (p) std::memset(p, 0, n * sizeof(double));
             continue;
         }
-        if ((rc = d2h(e, v->xc[q], f.r.xp[q], db)) || (rc = d2h_field(e, f, v->vp[q], f.r.vp[q], n)))
-            return rc;
+        rb.f64(v->xc[q], f.r.xp[q], n);
+        read_field(rb, f, v->vp[q], f.r.vp[q], n);
     }
-    if ((rc = d2h_field(e, f, v->overlap, f.s.ov, n)) ||
-        (rc = d2h(e, v->path_new, f.r.path_new, db)) ||
-        (rc = d2h(e, v->deleted, f.s.del, n)))
-        return rc;
-    return CUBBLE_OK;
+    read_field(rb, f, v->overlap, f.s.ov, n);
+    rb.f64(v->path_new, f.r.path_new, n);
+    rb.u8(v->deleted, f.s.del, n);
+    return rb.run(e);
 }
 
 namespace {
