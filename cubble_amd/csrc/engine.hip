@@ -485,10 +485,14 @@ void Engine::enqueue_attempt(uint32_t flags) {
 
 void Engine::enqueue_groups(uint32_t flags, int groups) {
     const Grid g = grid();
+    // an attempt's removal is carried out by the next one's predictor, or by
+    // the launch before the search phase
+    const bool in_predict = g.nb_bub <= kApplyBlocks;
     for (int k = 1; k <= groups; ++k) {
-        enqueue_attempt(flags);
-        launch_apply(g);
-        if (0 == k % kSearchEvery || groups == k) launch_search(g);
+        enqueue_attempt(in_predict ? flags | kApply : flags);
+        const bool phase = 0 == k % kSearchEvery || groups == k;
+        if (phase || !in_predict) launch_apply(g);
+        if (phase) launch_search(g);
     }
 }
 

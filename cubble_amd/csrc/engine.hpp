@@ -63,6 +63,12 @@ struct Tuning {
 // the attempts between.
 constexpr int kSearchEvery = 8;
 
+// Launches of at most this many blocks carry out removals in the predictor: a
+// launch for them costs 2.5 us an attempt (2D 1e4: 10.9 ms with it, 10.4
+// without, 3D 1e6: 21.4 / 21.1).  In larger ones, batches of many foams, the
+// predictor's registers cost more (256 foams, 1e4 blocks: 32.0 / 32.6 ms).
+constexpr int kApplyBlocks = 2048;
+
 // Most attempt groups between two host checks of the foams' flags in
 // run_steps (halts, list-capacity growth).
 constexpr int kRoundGroups = 128;

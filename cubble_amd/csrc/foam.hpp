@@ -175,6 +175,7 @@ enum Flags : uint32_t {
     kCommit = 4u,
     kFlow = 8u,
     kOwnSums = 16u,  // the corrector forms the foam's sums itself
+    kApply = 32u,    // the predictor carries out the removal of the attempt before
 };
 
 }  // namespace cubble_amd

@@ -40,7 +40,9 @@ void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control = tr
 
 // The planned removals: move the tail survivors into the holes, filter /
 // remap the neighbour lists and apply the volume fix.  Runs only for foams
-// whose need_remove flag is set; the next controller clears it.
+// whose need_remove flag is set; the next controller or the end of the next
+// search phase clears it.  With kApply an attempt's predictor carries out the
+// removal of the attempt before, unless the foam stands still.
 void launch_apply(const Grid &g);
 // removeBubbles by itself: the plan (sorted deletion list, moves), then the
 // above.  The caller clears the flag.

@@ -1,0 +1,146 @@
+// remove_apply.hpp -- a planned removal, carried out on one block of slots.
+#pragma once
+
+#include "dev_util.hpp"
+
+namespace cubble_amd {
+
+// The state of the tail survivor `src` into the hole i, by one wave: lane f
+// moves field f (x, v, v_old, saved by component, path, error, wrap counters,
+// index, list length at the last search), so all fields' loads are in flight
+// together; one after another, each waiting for the store before it, they
+// took most of a removal's time.  The radius takes the volume fix on the way.
+__device__ __forceinline__ void move_state(const Foam *F, int i, int src, double vm) {
+    const int lane = (int)(threadIdx.x & 63), q = lane & 3, D = F->c.dim;
+    const bool fvel = CUBBLE_PREC_MIXED == F->precision;
+    const Roles *R = &F->r;
+    void *p = nullptr;
+    bool wide = !fvel;  // an FP64 field
+    if (lane < 16) {
+        if (q != 2 || 3 == D)
+            p = lane < 4 ? R->x[q] : lane < 8 ? R->v[q] : lane < 12 ? R->vo[q] : R->saved[q];
+        wide = wide || lane < 4;
+    } else if (16 == lane) {
+        p = R->path;
+        wide = true;
+    } else if (17 == lane) {
+        p = R->err;
+    } else {
+        wide = false;
+        if (lane < 18 + D) p = R->wc[lane - 18];
+        if (21 == lane) p = R->idx;
+        if (22 == lane) p = F->s.deg;  // the reference moves numNeighbors unchanged
+    }
+    if (!p) return;
+    if (wide) {
+        double v = static_cast<const double *>(p)[src];
+        if (3 == lane) v = v * vm;
+        static_cast<double *>(p)[i] = v;
+    } else {
+        static_cast<uint32_t *>(p)[i] = static_cast<const uint32_t *>(p)[src];
+    }
+}
+
+// Bubble i's list from src's, by one wave: deleted neighbours dropped, moved
+// ones mapped to their new slots, ascending.  Up to 64 entries one lane each
+// (their marks and new slots are then one load each, and an entry's place is
+// the number of smaller ones); longer lists entry by entry.
+__device__ __forceinline__ void filter_list(const Scratch &S, size_t cap, int nnew, int i,
+                                            int src) {
+    const int lane = (int)(threadIdx.x & 63);
+    const int m = uniform_i(S.nn[src]);
+    if (m <= 64) {
+        const int j = lane < m ? S.nbr[(size_t)lane * cap + src] : -1;
+        const bool keep = j >= 0 && !S.del[j];
+        const bool moved = keep && j >= nnew;
+        const int jj = moved ? S.moved_to[j - nnew] : j;
+        const unsigned long long kept = __builtin_amdgcn_ballot_w64(keep);
+        int pos = __popcll(kept & ((1ull << lane) - 1ull));
+        if (__builtin_amdgcn_ballot_w64(moved)) {
+            pos = 0;
+            for (unsigned long long t = kept; t; t &= t - 1ull)
+                pos += __builtin_amdgcn_readlane(jj, __builtin_ctzll(t)) < jj ? 1 : 0;
+        }
+        if (keep) S.nbr[(size_t)pos * cap + i] = jj;
+        if (0 == lane) S.nn[i] = __popcll(kept);
+        return;
+    }
+    if (lane) return;
+    // writes stay at positions <= the entries consumed, so this also runs in
+    // place (src == i)
+    int out = 0, last = -1;  // largest entry written so far
+    for (int q = 0; q < m; ++q) {
+        const int j = S.nbr[(size_t)q * cap + src];
+        if (S.del[j]) continue;
+        const int jj = j >= nnew ? S.moved_to[j - nnew] : j;
+        int pos = out;
+        if (jj < last) {  // a moved bubble's new index: insertion keeps the order
+            while (pos > 0) {
+                const int prev = S.nbr[(size_t)(pos - 1) * cap + i];
+                if (prev <= jj) break;
+                S.nbr[(size_t)pos * cap + i] = prev;
+                --pos;
+            }
+        } else {
+            last = jj;
+        }
+        S.nbr[(size_t)pos * cap + i] = jj;
+        ++out;
+    }
+    S.nn[i] = out;
+}
+
+// The planned removal on the slots of bubble-space block lb, by its whole
+// workgroup: each thread applies the volume fix to its bubbles; the few holes
+// and marked bubbles are listed in LDS and rebuilt by one wave each.  No block
+// reads a slot that another one writes: the survivors lie past the new count.
+// What bounds it is the rebuild's chain of dependent loads (list, marks, new
+// slots) behind one pass over marks and radii.
+__device__ __forceinline__ void apply_removal(const Foam *F, int lb) {
+    __shared__ int s_cnt, s_list[kBlock];
+    const Scratch S = F->s;
+    double *const r = F->r.x[3];
+    const int nnew = F->d.count, h = F->d.n_holes, ipt = F->ipt;
+    const double vm = F->d.vol_fix;
+    const size_t cap = (size_t)F->cap;
+    const int lane = (int)(threadIdx.x & 63);
+    for (int k = 0; k < ipt; ++k) {
+        const int base = (lb * ipt + k) * kBlock;
+        if (base >= nnew) break;  // uniform per block
+        const int i = base + (int)threadIdx.x;
+        if (0 == threadIdx.x) s_cnt = 0;
+        __syncthreads();
+        if (i < nnew) {
+            const bool hole = S.del[i] != 0;
+            const bool marked = S.dirty[i] != 0;
+            if (!hole) r[i] = r[i] * vm;
+            if (marked) S.dirty[i] = 0;
+            if (hole || marked) s_list[atomicAdd(&s_cnt, 1)] = hole ? ~i : i;
+        }
+        __syncthreads();
+        const int cnt = s_cnt;
+        for (int e = threadIdx.x >> 6; e < cnt; e += kWaves) {
+            const int v = uniform_i(s_list[e]);
+            const bool hole = v < 0;
+            const int b = hole ? ~v : v;
+            int src = b;
+            if (hole) {  // the k-th entry of the deletion list is the k-th hole
+                for (int k0 = 0; k0 < h; k0 += 64) {
+                    const bool in = k0 + lane < h;
+                    const int d = in ? S.del_list[k0 + lane] : -1;
+                    const int s = in ? S.plan_src[k0 + lane] : -1;
+                    const unsigned long long at = __builtin_amdgcn_ballot_w64(d == b);
+                    if (at) {
+                        src = __builtin_amdgcn_readlane(s, __builtin_ctzll(at));
+                        break;
+                    }
+                }
+                move_state(F, b, src, vm);
+            }
+            filter_list(S, cap, nnew, b, src);
+        }
+        __syncthreads();
+    }
+}
+
+}  // namespace cubble_amd

@@ -748,6 +748,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 // count, list-capacity check, counters.
 __global__ __launch_bounds__(kSearchParts) void k_s_fin(Foam *foams, int swap) {
     Foam *F = foams + blockIdx.x;
+    // a removal was carried out before the search
+    if (0 == threadIdx.x) F->d.need_remove = 0;
     if (!F->d.need_search) return;
     const Scratch S = F->s;
     int s = 0, mx = 0, of = 0;
@@ -794,6 +796,7 @@ __global__ void k_set_limits(Foam *foams, int nf, long long add) {
     if (f >= nf) return;
     Dyn &d = foams[f].d;
     d.step_limit = add > 0 ? d.steps + add : 0;
+    d.need_remove = 0;  // carried out
     d.halt = 0;
     d.overflow = 0;
 }

@@ -23,6 +23,7 @@
 
 #include "dev_util.hpp"
 #include "launch.hpp"
+#include "remove_apply.hpp"
 #include "remove_plan.hpp"
 
 namespace cubble_amd {
@@ -68,10 +69,18 @@ __device__ __forceinline__ void predict_dispatch(const Consts &c, const Roles &R
     else predict_range<D, GAS, false>(c, R, p4, q4, base, ipt, n, h, sa, sar);
 }
 
+// APPLY: first the removal of the attempt before, if there was one, on the
+// block's own slots (a variant of its own: it takes 84 registers, the plain
+// predictor 41).
+template <bool APPLY>
 __global__ __launch_bounds__(kBlock) void k_predict(Foam *foams, const int2 *bt, uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
     if (standing(F->d)) return;
+    if (APPLY && F->d.need_remove) {
+        apply_removal(F, cx.lb);
+        __syncthreads();  // its waves wrote this block's slots
+    }
     const int n = F->d.count, ipt = F->ipt;
     const double h = 0.5 * F->d.dt;
     const Roles R = F->r;
@@ -559,8 +568,9 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
 __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags) {
     Foam *F = foams + blockIdx.x;
     if (standing(F->d)) {
-        // the removal of its last step is done
-        if (0 == threadIdx.x) F->d.need_remove = 0;
+        // the removal of its last step is done, or (kApply) waits for the
+        // search phase
+        if (0 == threadIdx.x && !(flags & kApply)) F->d.need_remove = 0;
         return;
     }
     __shared__ int s_del;
@@ -585,8 +595,12 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
 
 // ---------------------------------------------------------------- launches
 void launch_predict(const Grid &g, uint32_t flags) {
-    hipLaunchKernelGGL(k_predict, dim3(g.nb_bub), dim3(kBlock), 0, g.stream, g.foams, g.bt_bub,
-                       flags);
+    if (flags & kApply)
+        hipLaunchKernelGGL(k_predict<true>, dim3(g.nb_bub), dim3(kBlock), 0, g.stream, g.foams,
+                           g.bt_bub, flags);
+    else
+        hipLaunchKernelGGL(k_predict<false>, dim3(g.nb_bub), dim3(kBlock), 0, g.stream, g.foams,
+                           g.bt_bub, flags);
 }
 
 void launch_pair(const Grid &g, uint32_t flags) {

@@ -72,9 +72,9 @@ def test_removal_filters_long_lists(ora, dim, ipt):
     sim.close()
 
 
-# 255, 256 and 257 blocks of 256 bubbles: the corrector forms the foam's sums
-# itself up to 256
-@pytest.mark.parametrize("n", [65, 65279, 65536, 65537])
+# 255 to 257 blocks of 256 bubbles, and around 128 of them: the corrector forms
+# the foam's sums itself up to there
+@pytest.mark.parametrize("n", [65, 32767, 32768, 32769, 65279, 65536, 65537])
 def test_attempt_around_the_fused_sums(ora, n):
     print(f"fused sums n={n}", flush=True)
     sim = ca.Simulator(config(2, n, seed=70))
@@ -113,3 +113,32 @@ def test_search_phase_places_do_not_change_a_run(dim, n, precision):
         for key in st:
             assert np.array_equal(st[key], ends[0][0][key]), key
     assert ends[0][1]["searches"] >= 3
+
+
+@pytest.mark.parametrize("precision", [ca.PREC_FP64, ca.PREC_MIXED])
+def test_removals_by_the_predictor_or_a_launch(precision):
+    """A removal is carried out by the next attempt's predictor (captured runs
+    of up to 2048 blocks), by a launch before the search phase, or by a launch
+    after every attempt (larger runs, and one step per call): the same foams
+    come out bit for bit."""
+    print(f"removal routes precision={precision}", flush=True)
+    small = [config(2, 3001, seed=91, precision=precision, kappa=1.0, r_std=0.3),
+             config(3, 9000, seed=92, precision=precision, kappa=1.0, r_std=0.3)]
+    large = config(2, 2048 * 256 + 1, seed=93, precision=precision)
+    ends = []
+    for cfgs, groups, calls in ((small, 16, False), (small, 3, False), (small, 0, True),
+                                (small + [large], 16, False)):
+        batch = ca.Batch(cfgs, tuning={"graph_steps": groups} if groups else None)
+        if calls:
+            for _ in range(400):
+                res = batch.integrate(GAS)
+        else:
+            res = batch.run_steps(400, GAS)
+        ends.append([(batch.get_state(k)[0], res[k]) for k in range(2)])
+        batch.close()
+    for end in ends[1:]:
+        for (st, res), (st0, res0) in zip(end, ends[0]):
+            assert res == res0
+            for key in st:
+                assert np.array_equal(st[key], st0[key]), key
+    assert all(res["removals"] >= 20 for _, res in ends[0])
