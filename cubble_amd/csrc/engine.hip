@@ -455,11 +455,12 @@ int Engine::restore(const Snapshot &s) {
 Grid Engine::grid() const {
     Grid g;
     g.foams = dfoams_;
-    g.bt_bub = bt_bub_;
+    const bool one = 1 == foams.size();  // its blocks are the launch's
+    g.bt_bub = one ? nullptr : bt_bub_;
     g.nb_bub = nb_bub_;
-    g.bt_cell = bt_cell_;
+    g.bt_cell = one ? nullptr : bt_cell_;
     g.nb_cell = nb_cell_;
-    g.bt_scell = bt_scell_;
+    g.bt_scell = one ? nullptr : bt_scell_;
     g.nb_scell = nb_scell_;
     g.nfoams = (int)foams.size();
     g.stream = stream;

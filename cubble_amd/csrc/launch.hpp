@@ -8,7 +8,8 @@
 namespace cubble_amd {
 
 // A launch covers one or more foams.  bt_bub[b] = (foam, local block) for
-// the bubble-space grid, bt_cell[b] likewise for the cell-space grid.
+// the bubble-space grid, bt_cell[b] likewise for the cell-space grid; null
+// for a launch of one foam (a load less before the foam's header).
 struct Grid {
     Foam *foams;
     const int2 *bt_bub;

@@ -747,7 +747,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 // One block per foam: make the reordered buffers current (swap = 1), pair
 // count, list-capacity check, counters.
 __global__ __launch_bounds__(kSearchParts) void k_s_fin(Foam *foams, int swap) {
-    Foam *F = foams + blockIdx.x;
+    Foam *F = touch_header(foams + blockIdx.x);
     // a removal was carried out before the search
     if (0 == threadIdx.x) F->d.need_remove = 0;
     if (!F->d.need_search) return;

@@ -270,7 +270,7 @@ k_pair(Foam *foams, const int2 *bt, uint32_t flags) {
 // L2 caches are not coherent, so an in-kernel last-block reduction would
 // need an agent-scope release -- an L2 write-back -- in every block.)
 __global__ __launch_bounds__(kBlock) void k_sums(Foam *foams) {
-    Foam *F = foams + blockIdx.x;
+    Foam *F = touch_header(foams + blockIdx.x);
     if (standing(F->d)) return;
     double r[4];
     int none;
@@ -566,7 +566,7 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
 // and (when committing) the role rotation and the plan of a removal, which
 // the next launch applies.
 __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags) {
-    Foam *F = foams + blockIdx.x;
+    Foam *F = touch_header(foams + blockIdx.x);
     if (standing(F->d)) {
         // the removal of its last step is done, or (kApply) waits for the
         // search phase
