@@ -465,9 +465,11 @@ Grid Engine::grid() const {
     g.nfoams = (int)foams.size();
     g.stream = stream;
     g.walls = g.big = false;
+    g.quad = CUBBLE_PREC_FP64 == precision && nb_bub_ <= kQuadBlocks;
     g.search_threads = 64;
     for (const FoamRec &r : foams) {
         for (int a = 0; a < r.h.c.dim; ++a) g.walls = g.walls || r.h.c.wall[a] != 0;
+        g.quad = g.quad && 1 == r.h.ipt;
         g.big = g.big || r.h.nblk > kFuseBlocks;
         g.search_threads =
             std::max(g.search_threads, std::min(kBlock, (r.h.stile + 63) / 64 * 64));
@@ -502,7 +504,7 @@ int Engine::capture(uint32_t flags, int groups) {
     // (walls or not, a sums launch or not)
     const Grid g = grid();
     if (graph_ && graph_flags_ == flags && graph_groups_ == groups && graph_walls_ == g.walls &&
-        graph_big_ == g.big && graph_threads_ == g.search_threads)
+        graph_big_ == g.big && graph_quad_ == g.quad && graph_threads_ == g.search_threads)
         return CUBBLE_OK;
     if (graph_) {
         (void)hipGraphExecDestroy(graph_);
@@ -522,6 +524,7 @@ int Engine::capture(uint32_t flags, int groups) {
     graph_groups_ = groups;
     graph_walls_ = g.walls;
     graph_big_ = g.big;
+    graph_quad_ = g.quad;
     graph_threads_ = g.search_threads;
     return CUBBLE_OK;
 }

@@ -192,7 +192,7 @@ class Engine {
     hipGraphExec_t graph_ = nullptr;
     uint32_t graph_flags_ = 0;
     int graph_groups_ = 0;
-    bool graph_walls_ = false, graph_big_ = false;
+    bool graph_walls_ = false, graph_big_ = false, graph_quad_ = false;
     int graph_threads_ = 0;
     bool opened_ = false;  // counted among the users of the pinned blocks
     int committed_nf_ = 0;  // foams in the device array at the last commit

@@ -23,6 +23,7 @@ constexpr int kMaxBlocks = 2048;    // bubble-space blocks per foam (partials)
 constexpr int kNumXcd = 8;          // MI355X: 8 XCDs, workgroups round-robin
 constexpr int kFuseBlocks = 128;    // launches of foams of at most this many blocks sum their
                                     // partials in k_correct
+constexpr int kQuadBlocks = 1024;   // FP64 launches of at most this many blocks use k_pair_quad
 constexpr int kSearchParts = 64;    // records the search workgroups add their totals to
 constexpr int kPartD = 8;           // doubles per block partial record
 constexpr int kPartI = 4;           // ints per block partial record
@@ -97,6 +98,13 @@ struct Scratch {
     int32_t *plan_src;   // source (tail survivor) of hole k
     int32_t *moved_to;   // new slot of tail survivor (old index - new count)
 };
+
+// Where k_pair_quad leaves its sums, [nblk][4][2]: scratch of a removal, which
+// is free from the predictor that carries the removal out to the controller
+// that plans the next.
+__host__ __device__ inline double *quad_parts(const Scratch &s) {
+    return reinterpret_cast<double *>(s.del_list);
+}
 
 struct Dyn {
     int32_t count;
@@ -175,6 +183,7 @@ enum Flags : uint32_t {
     kCommit = 4u,
     kFlow = 8u,
     kOwnSums = 16u,  // the corrector forms the foam's sums itself
+    kQuad = 64u,     // the pair kernel was k_pair_quad
     kApply = 32u,    // the predictor carries out the removal of the attempt before
 };
 

@@ -22,6 +22,7 @@ struct Grid {
     int nfoams;
     hipStream_t stream;
     bool walls;  // some foam of the launch has a wall
+    bool quad;   // the FP64 pair kernel is k_pair_quad: one bubble a thread, few blocks
     bool big;    // some foam of the launch has more than kFuseBlocks blocks
 };
 

@@ -112,6 +112,45 @@ __global__ __launch_bounds__(kBlock) void k_predict(Foam *foams, const int2 *bt,
 // larger index: the reference adds dxdt[idx1] into idx2 for every listed pair
 // (idx1 < idx2) but dxdt[idx2] into idx1 only past its overlap test
 // (src/kernels.cu:191-208 vs :281-307).
+//
+// Adds what pair (i, j) adds to bubble i: zeros unless it overlaps (or j < 0),
+// which it returns.  d = x_i - x_j (minimum image); inv_ri = 1 / ri, risq =
+// ri^2.  Without a branch, so that the chains of several pairs overlap.
+template <int D, bool GAS>
+__device__ __forceinline__ bool add_pair(double f0, int i, double ri, double risq, double inv_ri,
+                                         int j, double rj, const double (&d)[3], double (&acc)[3],
+                                         double &ovl, double &dr) {
+    const double radii = ri + rj;
+    const double m = sq_len(d);
+    const bool on = j >= 0 && radii * radii >= m;
+    const double rs = rsq_nr(m);
+    const double s = rs - rcp_nr(radii);
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        const double t = d[a] * f0 * s;
+        acc[a] += on ? t : 0.0;
+    }
+    if (GAS) {
+        const double rjsq = rj * rj;
+        const double r1sq = i < j ? risq : rjsq;  // of the smaller index
+        const double r2sq = i < j ? rjsq : risq;
+        double oa = 0.5 * (r2sq - r1sq + m);
+        oa *= oa;
+        oa *= rs * rs;  // / m
+        oa = fabs(r2sq - oa);
+        if (m < r1sq || m < r2sq) oa = r1sq < r2sq ? r1sq : r2sq;
+        if (3 == D) {
+            oa *= kPi;
+        } else {
+            oa = 2.0 * sqrt(oa);
+        }
+        const double t = oa * (rcp_nr(rj) - inv_ri);
+        ovl += on ? oa : 0.0;
+        dr += on ? t : 0.0;
+    }
+    return on;
+}
+
 template <int D, bool GAS, bool FLOW>
 __device__ __forceinline__ void pair_range(const Consts &c, const Roles &R, const Scratch &S,
                                            size_t cap, int base, int ipt, int n, double &soa,
@@ -156,38 +195,11 @@ __device__ __forceinline__ void pair_range(const Consts &c, const Roles &R, cons
 #pragma unroll
             for (int u = 0; u < kGather; ++u) {
                 const int j = js[u];
-                const double rj = ps[u].r;
-                const double radii = ri + rj;
-                const double m = sq_len(d[u]);
-                const bool on = j >= 0 && radii * radii >= m;
+                const bool on = add_pair<D, GAS>(f0, i, ri, risq, inv_ri, j, ps[u].r, d[u], acc,
+                                                 ovl, dr);
                 if (FLOW && j >= 0 && (j < i || on)) {
 #pragma unroll
                     for (int a = 0; a < D; ++a) fv[a] += field<double>(R.v[a])[j];
-                }
-                const double rs = rsq_nr(m);
-                const double s = rs - rcp_nr(radii);
-#pragma unroll
-                for (int a = 0; a < D; ++a) {
-                    const double t = d[u][a] * f0 * s;
-                    acc[a] += on ? t : 0.0;
-                }
-                if (GAS) {
-                    const double rjsq = rj * rj;
-                    const double r1sq = i < j ? risq : rjsq;  // of the smaller index
-                    const double r2sq = i < j ? rjsq : risq;
-                    double oa = 0.5 * (r2sq - r1sq + m);
-                    oa *= oa;
-                    oa *= rs * rs;  // / m
-                    oa = fabs(r2sq - oa);
-                    if (m < r1sq || m < r2sq) oa = r1sq < r2sq ? r1sq : r2sq;
-                    if (3 == D) {
-                        oa *= kPi;
-                    } else {
-                        oa = 2.0 * sqrt(oa);
-                    }
-                    const double t = oa * (rcp_nr(rj) - inv_ri);
-                    ovl += on ? oa : 0.0;
-                    dr += on ? t : 0.0;
                 }
             }
         });
@@ -201,23 +213,41 @@ __device__ __forceinline__ void pair_range(const Consts &c, const Roles &R, cons
     }
 }
 
-// Four consecutive slots q0..q0+3 of a foam's block partials, reduced in one
-// pass over the records (each thread takes blocks t, t + kBlock, ... in
-// order), and the integer slot qi of the int partials summed alongside when
-// qi >= 0.  Bit k of `dmax` makes slot q0 + k a maximum (from 0), else a
-// sum.  The results are defined in thread 0 only.
-__device__ __forceinline__ void reduce_parts4(const double *part, const int32_t *part_i, int nb,
-                                              int q0, unsigned dmax, int qi, double (&r)[4],
-                                              int &ri) {
+// Block b's sums of S_A, S_Ar, S_OA, S_OAr; quad: the pair kernel's as
+// k_pair_quad left them, four a block, added in the order of the block's waves.
+__device__ __forceinline__ void block_sums(const double *part, const double *quad, int b,
+                                           double (&v)[4]) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) v[k] = part[b * kPartD + k];
+    if (quad) {
+        v[2] = v[3] = 0.0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            v[2] += quad[8 * b + 2 * w];
+            v[3] += quad[8 * b + 2 * w + 1];
+        }
+    } else {
+        v[2] = part[b * kPartD + 2];
+        v[3] = part[b * kPartD + 3];
+    }
+}
+
+// One value quadruple per block, read(b, v), reduced in one pass (each thread
+// takes blocks t, t + kBlock, ... in order), and the integer slot 0 of the int
+// partials summed alongside if part_i.  Bit k of `dmax` makes value k a maximum
+// (from 0), else a sum.  The results are defined in thread 0 only.
+template <typename Read>
+__device__ __forceinline__ void reduce_parts4(Read &&read, const int32_t *part_i, int nb,
+                                              unsigned dmax, double (&r)[4], int &ri) {
     double a[4] = {0.0, 0.0, 0.0, 0.0};
     int ai = 0;
 #pragma unroll 2
     for (int b = threadIdx.x; b < nb; b += kBlock) {
-        const double *p = part + b * kPartD + q0;
-        const double v[4] = {p[0], p[1], p[2], p[3]};
+        double v[4];
+        read(b, v);
 #pragma unroll
         for (int k = 0; k < 4; ++k) a[k] = (dmax >> k) & 1u ? fmax(a[k], v[k]) : a[k] + v[k];
-        if (qi >= 0) ai += part_i[b * kPartI + qi];
+        if (part_i) ai += part_i[b * kPartI];
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) r[k] = a[k];
@@ -265,16 +295,165 @@ k_pair(Foam *foams, const int2 *bt, uint32_t flags) {
     }
 }
 
+// Lane U's double, of each quad of lanes.
+template <int U>
+__device__ __forceinline__ double quad_lane(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x55 * U, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x55 * U, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// acc + the quad's four values, in the lanes' order.
+__device__ __forceinline__ double quad_add(double acc, double v) {
+    acc += quad_lane<0>(v);
+    acc += quad_lane<1>(v);
+    acc += quad_lane<2>(v);
+    return acc + quad_lane<3>(v);
+}
+
+// Bubble i's pairs by four lanes, lane u of them taking list entries u, u + 4,
+// ..., two at a time; every lane adds all four's terms in list order, the
+// order (and so the bits) of pair_range.  i >= n: nothing.
+template <int D, bool GAS, bool FLOW>
+__device__ __forceinline__ void pair_quad(const Consts &c, const Roles &R, const Scratch &S,
+                                          size_t cap, int i, int n, double &soa, double &soar) {
+    if (i >= n) return;
+    const auto p4 = gmem(S.p4);
+    const auto nbr = gmem(S.nbr);
+    const int u = (int)(threadIdx.x & 3);
+    const double f0 = c.f0;
+    double near[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) near[a] = c.wall[a] ? __builtin_inf() : 0.49 * c.interval[a];
+    const D4 pi = load_rec(p4 + i);
+    const double inv_ri = 1.0 / pi.r, risq = pi.r * pi.r;
+    double acc[3] = {0.0, 0.0, 0.0};
+    double fv[3] = {0.0, 0.0, 0.0};
+    double ovl = 0.0, dr = 0.0;
+    const int m_nn = S.nn[i];
+    for (int q0 = 0; q0 < m_nn; q0 += 8) {
+        int js[2];
+        D4 ps[2];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const int q = q0 + 4 * w + u;
+            const int j = nbr[(size_t)min(q, m_nn - 1) * cap + i];
+            js[w] = q < m_nn ? j : -1;
+        }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) ps[w] = load_rec(p4 + (js[w] >= 0 ? js[w] : i));
+        double d[2][3];
+        bool far = false;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            d[w][0] = pi.x - ps[w].x;
+            d[w][1] = pi.y - ps[w].y;
+            d[w][2] = 3 == D ? pi.z - ps[w].z : 0.0;
+#pragma unroll
+            for (int a = 0; a < D; ++a) far = far || fabs(d[w][a]) > near[a];
+        }
+        if (__builtin_amdgcn_ballot_w64(far) != 0ull) {
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+                wrapped_diff<D>(c, pi.x, pi.y, pi.z, ps[w].x, ps[w].y, ps[w].z, d[w]);
+        }
+        double t[2][3] = {}, to[2] = {}, tr[2] = {}, tv[2][3];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const bool on = add_pair<D, GAS>(f0, i, pi.r, risq, inv_ri, js[w], ps[w].r, d[w], t[w],
+                                             to[w], tr[w]);
+            if (FLOW) {
+                const bool count = js[w] >= 0 && (js[w] < i || on);
+#pragma unroll
+                for (int a = 0; a < D; ++a) tv[w][a] = count ? field<double>(R.v[a])[js[w]] : 0.0;
+            }
+        }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                acc[a] = quad_add(acc[a], t[w][a]);
+                if (FLOW) fv[a] = quad_add(fv[a], tv[w][a]);
+            }
+            if (GAS) {
+                ovl = quad_add(ovl, to[w]);
+                dr = quad_add(dr, tr[w]);
+            }
+        }
+    }
+    if (FLOW) add_flow<D>(c, pi, S.deg[i], fv, acc);
+    if (0 == u) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) field<double>(R.vp[a])[i] = acc[a];
+        field<double>(R.vp[3])[i] = dr;
+        field<double>(S.ov)[i] = ovl;
+    }
+    soa = ovl;
+    soar = ovl * inv_ri;
+}
+
+// The pair kernel of launches of up to kQuadBlocks blocks with one bubble a
+// thread: a workgroup takes 64 bubbles, four lanes each.  k_pair is bound there
+// by each wave's chain of loads and FP64 operations, list entry after list
+// entry, with few waves to overlap it; here a lane evaluates a quarter of the
+// pairs, and a wave waits for the longest of 16 lists instead of 64.  us a
+// launch, k_pair / this: 2D 1e3 6.9 / 3.8, 3e4 7.5 / 5.1, 2e5 12.7 / 11.7; 3D
+// 1e3 13.1 / 6.4, 3e4 15.3 / 7.8, 2e5 26.5 / 21.6; 8 foams of 1e4 17.4 / 10.9,
+// 128 of 2e3 30.7 / 26.9.  Beyond, the additions of every term in four lanes
+// cost more: 2D 5e5 23.5 / 27.4, 3D 42.8 / 46.5, 1e6 75.6 / 86.6.  The sums
+// leave as those of k_pair's waves, two for each 64 bubbles, at quad_parts().
+template <bool FLOW>
+__global__ __launch_bounds__(kBlock) void k_pair_quad(Foam *foams, const int2 *bt,
+                                                      uint32_t flags) {
+    const int2 e = bt ? bt[blockIdx.x >> 2] : make_int2(0, 0);
+    Foam *F = bt ? foams + e.x : touch_header(foams);
+    if (standing(F->d)) return;
+    const int part = bt ? 4 * xcd_remap(e.y, F->nblk) + (int)(blockIdx.x & 3)
+                        : xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    const int n = F->d.count;
+    const Consts c = F->c;
+    const Roles R = F->r;
+    const Scratch S = F->s;
+    const size_t cap = (size_t)F->cap;
+    const int i = part * 64 + (int)(threadIdx.x >> 2);
+    double soa = 0.0, soar = 0.0;
+    const bool gas = (flags & kGas) != 0;
+    if (3 == c.dim) {
+        if (gas) pair_quad<3, true, FLOW>(c, R, S, cap, i, n, soa, soar);
+        else pair_quad<3, false, FLOW>(c, R, S, cap, i, n, soa, soar);
+    } else {
+        if (gas) pair_quad<2, true, FLOW>(c, R, S, cap, i, n, soa, soar);
+        else pair_quad<2, false, FLOW>(c, R, S, cap, i, n, soa, soar);
+    }
+    __shared__ double s_sum[2][64];
+    if (0 == (threadIdx.x & 3)) {
+        s_sum[0][threadIdx.x >> 2] = soa;
+        s_sum[1][threadIdx.x >> 2] = soar;
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const double a = wave_sum(s_sum[0][threadIdx.x]), ar = wave_sum(s_sum[1][threadIdx.x]);
+        if (0 == threadIdx.x) {
+            double *const p = quad_parts(S) + 2 * (size_t)part;
+            p[0] = a;
+            p[1] = ar;
+        }
+    }
+}
+
 // One block per foam: S_A, S_Ar, S_OA, S_OAr from the predictor and pair
 // partials, in a fixed order.  (A separate launch: on MI355X the eight XCD
 // L2 caches are not coherent, so an in-kernel last-block reduction would
 // need an agent-scope release -- an L2 write-back -- in every block.)
-__global__ __launch_bounds__(kBlock) void k_sums(Foam *foams) {
+__global__ __launch_bounds__(kBlock) void k_sums(Foam *foams, bool quad) {
     Foam *F = touch_header(foams + blockIdx.x);
     if (standing(F->d)) return;
     double r[4];
     int none;
-    reduce_parts4(F->s.part, F->s.part_i, F->nblk, 0, 0u, -1, r, none);
+    const double *const part = F->s.part, *const q = quad ? quad_parts(F->s) : nullptr;
+    reduce_parts4([&](int b, double (&v)[4]) { block_sums(part, q, b, v); }, nullptr, F->nblk, 0u,
+                  r, none);
     if (threadIdx.x == 0) {
         F->d.s_a = r[0];
         F->d.s_ar = r[1];
@@ -289,17 +468,15 @@ __global__ __launch_bounds__(kBlock) void k_sums(Foam *foams) {
 // again in every block of the corrector costs it under a microsecond up to
 // two rounds; the launch of k_sums it replaces costs 2.5.  In a batch the
 // launch is the cheaper one: 256 foams' correctors took 36 us longer.
-__device__ __forceinline__ void wave_foam_sums(const double *__restrict__ part, int nb,
+__device__ __forceinline__ void wave_foam_sums(const double *__restrict__ part,
+                                               const double *__restrict__ quad, int nb,
                                                double (&r)[4]) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) r[k] = 0.0;
     for (int b0 = 0; b0 < nb; b0 += 64) {
         const int b = b0 + (int)(threadIdx.x & 63);
         double v[4] = {0.0, 0.0, 0.0, 0.0};
-        if (b < nb) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) v[k] = part[b * kPartD + k];
-        }
+        if (b < nb) block_sums(part, quad, b, v);
 #pragma unroll
         for (int k = 0; k < 4; ++k) r[k] += wave_sum(v[k]);
     }
@@ -533,7 +710,7 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
     const int base = cx.lb * kBlock * ipt;
     if (flags & kOwnSums) {
         double r[4];
-        wave_foam_sums(S.part, F->nblk, r);
+        wave_foam_sums(S.part, flags & kQuad ? quad_parts(S) : nullptr, F->nblk, r);
         dyn.s_a = r[0];
         dyn.s_ar = r[1];
         dyn.s_oa = r[2];
@@ -579,7 +756,13 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
     // deletion count
     double r[4];
     int nd;
-    reduce_parts4(F->s.part, F->s.part_i, F->nblk, 4, 0xeu, 0, r, nd);
+    const double *const part = F->s.part;
+    reduce_parts4(
+        [&](int b, double (&v)[4]) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = part[b * kPartD + 4 + k];
+        },
+        F->s.part_i, F->nblk, 0xeu, r, nd);
     if (threadIdx.x == 0) {
         CorrAcc t;
         t.s_v = r[0];
@@ -604,6 +787,15 @@ void launch_predict(const Grid &g, uint32_t flags) {
 }
 
 void launch_pair(const Grid &g, uint32_t flags) {
+    if (g.quad) {
+        if (flags & kFlow)
+            hipLaunchKernelGGL(k_pair_quad<true>, dim3(4 * g.nb_bub), dim3(kBlock), 0, g.stream,
+                               g.foams, g.bt_bub, flags);
+        else
+            hipLaunchKernelGGL(k_pair_quad<false>, dim3(4 * g.nb_bub), dim3(kBlock), 0, g.stream,
+                               g.foams, g.bt_bub, flags);
+        return;
+    }
     if (flags & kFlow)
         hipLaunchKernelGGL(k_pair<true>, dim3(g.nb_bub), dim3(kBlock), 0, g.stream, g.foams,
                            g.bt_bub, flags);
@@ -613,7 +805,8 @@ void launch_pair(const Grid &g, uint32_t flags) {
 }
 
 void launch_sums(const Grid &g) {
-    if (g.big) hipLaunchKernelGGL(k_sums, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams);
+    if (g.big)
+        hipLaunchKernelGGL(k_sums, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams, g.quad);
 }
 
 // AB2 bootstrap of init (reference src/simulator.cu:739-787): the Euler step
@@ -684,6 +877,7 @@ void launch_bootstrap(const Grid &g, bool mixed) {
 void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control) {
     const dim3 grid(g.nb_bub), block(kBlock);
     if (!g.big) flags |= kOwnSums;
+    if (g.quad) flags |= kQuad;
     if (mixed) {
         if (g.walls)
             hipLaunchKernelGGL((k_correct<true, true>), grid, block, 0, g.stream, g.foams,
