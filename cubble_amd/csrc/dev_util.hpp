@@ -399,6 +399,52 @@ __device__ __forceinline__ void for_neighbours(const int *__restrict__ nbr_,
     }
 }
 
+// ---- four lanes a bubble ----
+// Lane U's double, of each quad of lanes.
+template <int U>
+__device__ __forceinline__ double quad_lane(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x55 * U, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x55 * U, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// acc + the quad's four values, in the lanes' order.
+__device__ __forceinline__ double quad_add(double acc, double v) {
+    acc += quad_lane<0>(v);
+    acc += quad_lane<1>(v);
+    acc += quad_lane<2>(v);
+    return acc + quad_lane<3>(v);
+}
+
+__device__ __forceinline__ float quad_add_f(float acc, float v) {
+    const int b = __float_as_int(v);
+    acc += __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x00, 0xf, 0xf, true));
+    acc += __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0x55, 0xf, 0xf, true));
+    acc += __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0xaa, 0xf, 0xf, true));
+    return acc + __int_as_float(__builtin_amdgcn_update_dpp(0, b, 0xff, 0xf, 0xf, true));
+}
+
+// The sums of a workgroup's 64 bubbles (lane 0 of each quad holds its bubble's)
+// to the foam's record `part` of quad_parts(): the reduction of one wave with
+// one bubble a lane.
+__device__ __forceinline__ void quad_store(const Scratch &S, int part, double soa, double soar) {
+    __shared__ double s_sum[2][64];
+    if (0 == (threadIdx.x & 3)) {
+        s_sum[0][threadIdx.x >> 2] = soa;
+        s_sum[1][threadIdx.x >> 2] = soar;
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const double a = wave_sum(s_sum[0][threadIdx.x]), ar = wave_sum(s_sum[1][threadIdx.x]);
+        if (0 == threadIdx.x) {
+            double *const p = quad_parts(S) + 2 * (size_t)part;
+            p[0] = a;
+            p[1] = ar;
+        }
+    }
+}
+
 // ---- fixed-point positions of the mixed-precision neighbour record ------
 // Code of coordinate x on axis (lb, L, wall): periodic axes take
 // round((x - lb) 2^32 / L) modulo 2^32, as a signed 32-bit value offset by

@@ -465,15 +465,19 @@ Grid Engine::grid() const {
     g.nfoams = (int)foams.size();
     g.stream = stream;
     g.walls = g.big = false;
-    g.quad = CUBBLE_PREC_FP64 == precision && nb_bub_ <= kQuadBlocks;
     g.search_threads = 64;
+    g.quad = true;
+    bool all3 = true;
     for (const FoamRec &r : foams) {
         for (int a = 0; a < r.h.c.dim; ++a) g.walls = g.walls || r.h.c.wall[a] != 0;
+        all3 = all3 && 3 == r.h.c.dim;
         g.quad = g.quad && 1 == r.h.ipt;
         g.big = g.big || r.h.nblk > kFuseBlocks;
         g.search_threads =
             std::max(g.search_threads, std::min(kBlock, (r.h.stile + 63) / 64 * 64));
     }
+    g.quad = g.quad && nb_bub_ <= (CUBBLE_PREC_MIXED != precision ? kQuadBlocks
+                                   : all3 ? kQuadMixed3 : kQuadMixed2);
     return g;
 }
 

@@ -23,7 +23,10 @@ constexpr int kMaxBlocks = 2048;    // bubble-space blocks per foam (partials)
 constexpr int kNumXcd = 8;          // MI355X: 8 XCDs, workgroups round-robin
 constexpr int kFuseBlocks = 128;    // launches of foams of at most this many blocks sum their
                                     // partials in k_correct
-constexpr int kQuadBlocks = 1024;   // FP64 launches of at most this many blocks use k_pair_quad
+// Launches of at most this many blocks, one bubble a thread, take four lanes a
+// bubble in the pair kernel: FP64, mixed with 3D foams only, mixed with 2D ones
+// (a 2D list is half as long, and FP32 leaves less to overlap).
+constexpr int kQuadBlocks = 1024, kQuadMixed3 = 400, kQuadMixed2 = 128;
 constexpr int kSearchParts = 64;    // records the search workgroups add their totals to
 constexpr int kPartD = 8;           // doubles per block partial record
 constexpr int kPartI = 4;           // ints per block partial record

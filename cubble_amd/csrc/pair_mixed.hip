@@ -105,12 +105,38 @@ struct MixedOut {
     float acc[3], fv[3], ovl, dr;
 };
 
-// The terms of bubble i's pairs, one call per neighbour j.  EXACT = false
-// evaluates the pair in FP32 from code differences; EXACT = true takes the
-// values and decisions of a pair that needs them from the FP64 predictions
-// (pi, bubble i's), with everything else the same.  A call adds the pair's
-// terms to o and returns whether the pair needs FP64 values: nearly
-// coincident centres, near-tangent in 2D, or near a branch point.
+// One pair's part of a bubble's sums: the relative coordinate dd, the velocity
+// per unit of it w, the overlap area g in units of area_unit<D>() and the
+// difference of inverse radii rd.  w and g are 0 for a pair that does not
+// overlap.  special: the pair needs FP64 values.
+struct MixedTerm {
+    float dd[3], w, g, rd;
+    bool on, special;
+};
+
+template <int D>
+__device__ __forceinline__ constexpr float area_unit() {
+    return 3 == D ? (float)kPi : 2.0f;
+}
+
+// The terms added, each product with its sum rounded once.
+template <int D, bool GAS>
+__device__ __forceinline__ void add_term(const MixedTerm &t, MixedOut &o) {
+#pragma unroll
+    for (int a = 0; a < D; ++a) o.acc[a] = fmaf(t.dd[a], t.w, o.acc[a]);
+    if (GAS) {
+        o.ovl = fmaf(area_unit<D>(), t.g, o.ovl);
+        o.dr = fmaf(t.rd, area_unit<D>() * t.g, o.dr);
+    }
+}
+
+// The terms of bubble i's pairs, one call per neighbour j (j < 0: none, qj any
+// record).  EXACT = false evaluates the pair in FP32 from code differences;
+// EXACT = true takes the values and decisions of a pair that needs them from
+// the FP64 predictions (pi, bubble i's), with everything else the same.  A
+// pair is special when it needs FP64 values: nearly coincident centres,
+// near-tangent in 2D, or near a branch point.  Without a branch, so that the
+// chains of several pairs overlap.
 template <int D, bool GAS, bool FLOW, bool EXACT>
 struct MixedPair {
     const Consts &c;
@@ -143,66 +169,72 @@ struct MixedPair {
         if (EXACT) pi = predicted<D, GAS, float>(R, h, i);
     }
 
-    __device__ __forceinline__ bool operator()(int j, const Q4 &qj, MixedOut &o) const {
-        const float pi_f = (float)kPi;
+    template <bool BRANCH>
+    __device__ __forceinline__ MixedTerm term(int j, const Q4 &qj) const {
+#pragma clang fp contract(off)
+        MixedTerm t;
         const float rj_f = qj.r;
         // code differences are exact integers; one rounding to FP32 each
-        float dd[3] = {(float)fixed_diff(qi.x, qj.x) * step[0],
-                       (float)fixed_diff(qi.y, qj.y) * step[1],
-                       D == 3 ? (float)fixed_diff(qi.z, qj.z) * step[2] : 0.f};
-        float m = dd[0] * dd[0] + dd[1] * dd[1] + dd[2] * dd[2];
+        t.dd[0] = (float)fixed_diff(qi.x, qj.x) * step[0];
+        t.dd[1] = (float)fixed_diff(qi.y, qj.y) * step[1];
+        t.dd[2] = D == 3 ? (float)fixed_diff(qi.z, qj.z) * step[2] : 0.f;
+        float m = fmaf(t.dd[0], t.dd[0], t.dd[1] * t.dd[1]);
+        if (3 == D) m = fmaf(t.dd[2], t.dd[2], m);
         const float rad = ri_f + rj_f;
-        float over = rad * rad - m;
+        float over = fmaf(rad, rad, -m);
         // a centre inside the other bubble: |d|^2 < r1^2 or r2^2, that is
         // below the larger square; the product form of the area is symmetric
         // in the radii, so their order does not matter
         const float sq_i = ri_f * ri_f, sq_j = rj_f * rj_f;
         const float big = fmaxf(sq_i, sq_j);
-        // pairs the FP32 values do not settle (each test evaluated: a wave
-        // rarely skips one, so no branches)
+        // pairs the FP32 values do not settle
         bool special = m < close2;
         if (FLOW)
-            special |= j > i && fabsf(over) <= band_abs * rad + kBranchBand * (rad * rad);
+            special |= j > i && fabsf(over) <= fmaf(kBranchBand, rad * rad, band_abs * rad);
         if (GAS && D == 2) {
-            const float t = fmaf(kTangentR, rad, tangent_s);
-            special |= fabsf(over) <= t * t;
+            const float tn = fmaf(kTangentR, rad, tangent_s);
+            special |= fabsf(over) <= tn * tn;
         }
         // (the inside band uses max(r1, r2) <= (big + 1) / 2: one FMA)
         if (GAS) special |= fabsf(m - big) <= fmaf(big, inside_k1, inside_k0);
+        special = special && j >= 0;
         bool overlap = over >= 0.f;
         bool inside = m < big;
         if (EXACT && special) {
             const ExactPair e = exact_pair<D, GAS>(c, R, h, pi, i, j);
 #pragma unroll
-            for (int a = 0; a < 3; ++a) dd[a] = e.dd[a];
+            for (int a = 0; a < 3; ++a) t.dd[a] = e.dd[a];
             m = e.m;
             over = e.over;
             overlap = e.overlap;
             inside = e.inside;
         }
-        if (FLOW && (j < i || overlap)) {
-#pragma unroll
-            for (int a = 0; a < D; ++a) o.fv[a] += field<float>(R.v[a])[j];
-        }
-        if (overlap) {
+        overlap = overlap && j >= 0;
+        t.w = t.g = t.rd = 0.f;
+        if (!BRANCH || overlap) {
             const float rs = __builtin_amdgcn_rsqf(m);
             const float s = rs - __builtin_amdgcn_rcpf(rad);
-#pragma unroll
-            for (int a = 0; a < D; ++a) o.acc[a] += dd[a] * (f0 * s);
+            t.w = overlap ? s * f0 : 0.f;
             if (GAS) {
-                float a2;
-                if (inside) {
-                    a2 = fminf(sq_i, sq_j);
-                } else {
+                float a2 = fminf(sq_i, sq_j);
+                if (!BRANCH || !inside) {
                     const float dl = ri_f - rj_f;
-                    a2 = fabsf(over * (m - dl * dl) * (0.25f * rs * rs));
+                    const float out = fabsf(over * fmaf(-dl, dl, m) * (0.25f * rs * rs));
+                    a2 = inside ? a2 : out;
                 }
-                const float oa = 3 == D ? a2 * pi_f : 2.0f * __builtin_amdgcn_sqrtf(a2);
-                o.ovl += oa;
-                o.dr += oa * (__builtin_amdgcn_rcpf(rj_f) - inv_ri);
+                const float g = 3 == D ? a2 : __builtin_amdgcn_sqrtf(a2);
+                t.g = overlap ? g : 0.f;
+                t.rd = __builtin_amdgcn_rcpf(rj_f) - inv_ri;
             }
         }
-        return special;
+        t.on = overlap;
+        t.special = special;
+        return t;
+    }
+
+    // Whether pair (i, j) counts in the neighbour-velocity sum of the flow.
+    __device__ __forceinline__ bool flows(int j, const MixedTerm &t) const {
+        return FLOW && j >= 0 && (j < i || t.on);
     }
 };
 
@@ -250,14 +282,139 @@ __device__ __forceinline__ void mixed_block(const Consts &c, const Roles &R, con
         for_neighbours(S.nbr, S.q4, cap, i, S.nn[i],
                        [&](const int(&js)[kGather], const Q4(&qs)[kGather]) {
 #pragma unroll
-                           for (int u = 0; u < kGather; ++u)
-                               if (js[u] >= 0) near = pair(js[u], qs[u], o) || near;
+                           for (int u = 0; u < kGather; ++u) {
+                               if (js[u] < 0) continue;
+                               const MixedTerm t = pair.template term<true>(js[u], qs[u]);
+                               if (pair.flows(js[u], t)) {
+#pragma unroll
+                                   for (int a = 0; a < D; ++a)
+                                       o.fv[a] += field<float>(R.v[a])[js[u]];
+                               }
+                               add_term<D, GAS>(t, o);
+                               near = near || t.special;
+                           }
                        });
         store_mixed<D, GAS, FLOW>(c, R, S, h, i, o, near);
         near_any = near_any || near;
         soa += (double)o.ovl;
         soar += (double)o.ovl * (1.0 / (double)qi.r);
     }
+}
+
+// Lane U's term, of each quad of lanes, but for its flags.
+template <int D, int U>
+__device__ __forceinline__ MixedTerm quad_term(const MixedTerm &t) {
+    auto lane = [](float v) {
+        return __int_as_float(
+            __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x55 * U, 0xf, 0xf, true));
+    };
+    MixedTerm o;
+#pragma unroll
+    for (int a = 0; a < D; ++a) o.dd[a] = lane(t.dd[a]);
+    o.w = lane(t.w);
+    o.g = lane(t.g);
+    o.rd = lane(t.rd);
+    return o;
+}
+
+// Bubble i's pairs by four lanes, lane u of them taking list entries u, u + 4,
+// ..., two at a time; every lane adds all four's terms in list order, with the
+// roundings of mixed_block.  i >= n: nothing.
+template <int D, bool GAS, bool FLOW>
+__device__ __forceinline__ void mixed_quad(const Consts &c, const Roles &R, const Scratch &S,
+                                           size_t cap, int i, int n, double h, double &soa,
+                                           double &soar, bool &near_any) {
+    if (i >= n) return;
+    const auto q4 = gmem(S.q4);
+    const auto nbr = gmem(S.nbr);
+    const int u = (int)(threadIdx.x & 3);
+    float step[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) step[a] = fixed_step(c.interval[a], c.wall[a] != 0);
+    const Q4 qi = load_rec(q4 + i);
+    const MixedPair<D, GAS, FLOW, false> pair(c, R, h, step, i, qi);
+    MixedOut o;
+    zero_out(o);
+    bool near = false;
+    const int m_nn = S.nn[i];
+    for (int q0 = 0; q0 < m_nn; q0 += 8) {
+        int js[2];
+        Q4 qs[2];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const int q = q0 + 4 * w + u;
+            const int j = nbr[(size_t)min(q, m_nn - 1) * cap + i];
+            js[w] = q < m_nn ? j : -1;
+        }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) qs[w] = load_rec(q4 + (js[w] >= 0 ? js[w] : i));
+        MixedTerm t[2];
+        float tv[2][3];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            t[w] = pair.template term<false>(js[w], qs[w]);
+            near = near || t[w].special;
+            if (FLOW) {
+                const bool count = pair.flows(js[w], t[w]);
+#pragma unroll
+                for (int a = 0; a < D; ++a) tv[w][a] = count ? field<float>(R.v[a])[js[w]] : 0.f;
+            }
+        }
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            add_term<D, GAS>(quad_term<D, 0>(t[w]), o);
+            add_term<D, GAS>(quad_term<D, 1>(t[w]), o);
+            add_term<D, GAS>(quad_term<D, 2>(t[w]), o);
+            add_term<D, GAS>(quad_term<D, 3>(t[w]), o);
+            if (FLOW) {
+#pragma unroll
+                for (int a = 0; a < D; ++a) o.fv[a] = quad_add_f(o.fv[a], tv[w][a]);
+            }
+        }
+    }
+    // any of the four
+    const unsigned long long mask = __builtin_amdgcn_ballot_w64(near);
+    near = (mask >> (threadIdx.x & 60) & 15ull) != 0ull;
+    if (0 == u) store_mixed<D, GAS, FLOW>(c, R, S, h, i, o, near);
+    near_any = near;
+    soa = (double)o.ovl;
+    soar = (double)o.ovl * (1.0 / (double)qi.r);
+}
+
+// The pair kernel of small launches, as k_pair_quad.  us a launch, k_pair_mixed
+// / this: 3D 1e3 7.8 / 4.7, 3e4 8.6 / 5.4, 6e4 8.9 / 7.2, 1e5 9.3 / 9.2 when just
+// seeded (and after 2000 steps, when some lists are long, 18.6 -> 17.1 ms a run
+// of 300 steps), 2e5 11.8 / 13.9; 2D 3e4 5.1 / 4.2, 6e4 5.2 / 5.1, 1e5 5.7 / 6.2.
+template <bool FLOW>
+__global__ __launch_bounds__(kBlock) void k_pair_mixed_quad(Foam *foams, const int2 *bt,
+                                                            uint32_t flags) {
+    const int2 e = bt ? bt[blockIdx.x >> 2] : make_int2(0, 0);
+    Foam *F = bt ? foams + e.x : touch_header(foams);
+    if (standing(F->d)) return;
+    const int part = bt ? 4 * xcd_remap(e.y, F->nblk) + (int)(blockIdx.x & 3)
+                        : xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    const int n = F->d.count;
+    const double h = 0.5 * F->d.dt;
+    const Consts c = F->c;
+    const Roles R = F->r;
+    const Scratch S = F->s;
+    const size_t cap = (size_t)F->cap;
+    const int i = part * 64 + (int)(threadIdx.x >> 2);
+    double soa = 0.0, soar = 0.0;
+    bool near = false;
+    const bool gas = (flags & kGas) != 0;
+    if (3 == c.dim) {
+        if (gas) mixed_quad<3, true, FLOW>(c, R, S, cap, i, n, h, soa, soar, near);
+        else mixed_quad<3, false, FLOW>(c, R, S, cap, i, n, h, soa, soar, near);
+    } else {
+        if (gas) mixed_quad<2, true, FLOW>(c, R, S, cap, i, n, h, soa, soar, near);
+        else mixed_quad<2, false, FLOW>(c, R, S, cap, i, n, h, soa, soar, near);
+    }
+    quad_store(S, part, soa, soar);
+    // the block's mark, a byte of it for each 64 bubbles
+    const bool any = __syncthreads_or(near) != 0;
+    if (0 == threadIdx.x)
+        reinterpret_cast<uint8_t *>(S.part_i + (part >> 2) * kPartI + 2)[part & 3] = any ? 1 : 0;
 }
 
 // Flagged bubble i (wave-uniform) summed again by the whole wave, the values
@@ -276,7 +433,12 @@ __device__ __forceinline__ float exact_bubble_wave(const Consts &c, const Roles 
     const int m_nn = S.nn[i];
     for (int q = (int)(threadIdx.x & 63); q < m_nn; q += 64) {
         const int j = gmem(S.nbr)[(size_t)q * cap + i];
-        pair(j, load_rec(gmem(S.q4) + j), o);
+        const MixedTerm t = pair.template term<true>(j, load_rec(gmem(S.q4) + j));
+        if (pair.flows(j, t)) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) o.fv[a] += field<float>(R.v[a])[j];
+        }
+        add_term<D, GAS>(t, o);
     }
 #pragma unroll
     for (int a = 0; a < D; ++a) {
@@ -373,7 +535,7 @@ __device__ __forceinline__ void mixed_block_dispatch(const Foam *F, int lb, uint
 // flag in the sign of its stored overlap sum, and its wave sets a bit in the
 // block's mark (block partial slot 2).
 template <bool FLOW>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FLOW ? 1 : 8, 8))) void
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FLOW ? 6 : 8, 8))) void
 k_pair_mixed(Foam *foams, const int2 *bt, uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
@@ -408,6 +570,17 @@ __global__ __launch_bounds__(kBlock) void k_fix_mixed(Foam *foams, const int2 *b
     double soa = 0.0, soar = 0.0;
     bool near = false;
     mixed_block_dispatch<FLOW, true>(F, cx.lb, flags, soa, soar, near);
+    if (flags & kQuad) {
+        // (one bubble a thread)
+        soa = wave_sum(soa);
+        soar = wave_sum(soar);
+        if (0 == (threadIdx.x & 63)) {
+            double *const p = quad_parts(F->s) + 8 * (size_t)cx.lb + 2 * (threadIdx.x >> 6);
+            p[0] = soa;
+            p[1] = soar;
+        }
+        return;
+    }
     double sums[2] = {soa, soar};
     int none = 0;
     block_reduce_t0(sums, 0u, none);
@@ -418,18 +591,28 @@ __global__ __launch_bounds__(kBlock) void k_fix_mixed(Foam *foams, const int2 *b
 }
 
 void launch_pair_mixed(const Grid &g, uint32_t flags, bool fix) {
+    const dim3 grid(g.nb_bub), quad(4 * g.nb_bub), block(kBlock);
+    if (g.quad) flags |= kQuad;
     if (flags & kFlow) {
-        hipLaunchKernelGGL(k_pair_mixed<true>, dim3(g.nb_bub), dim3(kBlock), 0, g.stream, g.foams,
-                           g.bt_bub, flags);
+        if (g.quad)
+            hipLaunchKernelGGL(k_pair_mixed_quad<true>, quad, block, 0, g.stream, g.foams,
+                               g.bt_bub, flags);
+        else
+            hipLaunchKernelGGL(k_pair_mixed<true>, grid, block, 0, g.stream, g.foams, g.bt_bub,
+                               flags);
         if (fix)
-            hipLaunchKernelGGL(k_fix_mixed<true>, dim3(g.nb_bub), dim3(kBlock), 0, g.stream,
-                               g.foams, g.bt_bub, flags);
+            hipLaunchKernelGGL(k_fix_mixed<true>, grid, block, 0, g.stream, g.foams, g.bt_bub,
+                               flags);
     } else {
-        hipLaunchKernelGGL(k_pair_mixed<false>, dim3(g.nb_bub), dim3(kBlock), 0, g.stream,
-                           g.foams, g.bt_bub, flags);
+        if (g.quad)
+            hipLaunchKernelGGL(k_pair_mixed_quad<false>, quad, block, 0, g.stream, g.foams,
+                               g.bt_bub, flags);
+        else
+            hipLaunchKernelGGL(k_pair_mixed<false>, grid, block, 0, g.stream, g.foams, g.bt_bub,
+                               flags);
         if (fix)
-            hipLaunchKernelGGL(k_fix_mixed<false>, dim3(g.nb_bub), dim3(kBlock), 0, g.stream,
-                               g.foams, g.bt_bub, flags);
+            hipLaunchKernelGGL(k_fix_mixed<false>, grid, block, 0, g.stream, g.foams, g.bt_bub,
+                               flags);
     }
 }
 

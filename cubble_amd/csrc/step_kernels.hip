@@ -295,23 +295,6 @@ k_pair(Foam *foams, const int2 *bt, uint32_t flags) {
     }
 }
 
-// Lane U's double, of each quad of lanes.
-template <int U>
-__device__ __forceinline__ double quad_lane(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x55 * U, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x55 * U, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
-// acc + the quad's four values, in the lanes' order.
-__device__ __forceinline__ double quad_add(double acc, double v) {
-    acc += quad_lane<0>(v);
-    acc += quad_lane<1>(v);
-    acc += quad_lane<2>(v);
-    return acc + quad_lane<3>(v);
-}
-
 // Bubble i's pairs by four lanes, lane u of them taking list entries u, u + 4,
 // ..., two at a time; every lane adds all four's terms in list order, the
 // order (and so the bits) of pair_range.  i >= n: nothing.
@@ -426,20 +409,7 @@ __global__ __launch_bounds__(kBlock) void k_pair_quad(Foam *foams, const int2 *b
         if (gas) pair_quad<2, true, FLOW>(c, R, S, cap, i, n, soa, soar);
         else pair_quad<2, false, FLOW>(c, R, S, cap, i, n, soa, soar);
     }
-    __shared__ double s_sum[2][64];
-    if (0 == (threadIdx.x & 3)) {
-        s_sum[0][threadIdx.x >> 2] = soa;
-        s_sum[1][threadIdx.x >> 2] = soar;
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        const double a = wave_sum(s_sum[0][threadIdx.x]), ar = wave_sum(s_sum[1][threadIdx.x]);
-        if (0 == threadIdx.x) {
-            double *const p = quad_parts(S) + 2 * (size_t)part;
-            p[0] = a;
-            p[1] = ar;
-        }
-    }
+    quad_store(S, part, soa, soar);
 }
 
 // One block per foam: S_A, S_Ar, S_OA, S_OAr from the predictor and pair

@@ -32,19 +32,20 @@ def _outputs(sim, st, sc, ip):
 # around the 64 bubbles of a workgroup and the 256 of a block, lists of more
 # than 8 and (a large bubble) more than 64 entries, gas exchange off, flow and
 # walls
+@pytest.mark.parametrize("precision", [ca.PREC_FP64, ca.PREC_MIXED])
 @pytest.mark.parametrize("dim,n,gas,flow,walls,big", [
     (2, 5, True, False, False, 0.0), (2, 63, True, False, False, 0.0),
     (3, 64, True, False, False, 0.0), (2, 65, False, False, True, 0.0),
     (3, 257, True, False, True, 0.0), (2, 3001, True, True, True, 0.0),
     (3, 3000, True, True, False, 0.0), (3, 5000, False, False, False, 0.0),
     (2, 4000, True, False, False, 9.0), (3, 4000, True, True, False, 5.0)])
-def test_four_lanes_a_bubble(dim, n, gas, flow, walls, big):
-    print(f"pair quad dim={dim} n={n} gas={gas} flow={flow} walls={walls} big={big}", flush=True)
+def test_four_lanes_a_bubble(precision, dim, n, gas, flow, walls, big):
+    print(f"pair quad precision={precision} dim={dim} n={n} gas={gas} flow={flow} walls={walls} big={big}", flush=True)
     over = {"wall": (0, 1, 0)} if walls else {}
     if flow:
         over.update(flow=1, flow_vel=(0.01, 0.0, 0.0), flow_lbb=(0.0, 0.3, 0.0),
                     flow_tfr=(0.4, 0.7, 1.0))
-    cfg = config(dim, n, seed=100 + n, **over)
+    cfg = config(dim, n, seed=100 + n, precision=precision, **over)
     ip = ca.IntegrationParams(gas, flow, True)
     one, st, sc = _attempt(cfg, 1, ip, big)
     two, _, _ = _attempt(cfg, 2, ip)
@@ -61,11 +62,13 @@ def test_four_lanes_a_bubble(dim, n, gas, flow, walls, big):
     two.close()
 
 
-def test_several_foams_in_a_small_launch():
+@pytest.mark.parametrize("precision", [ca.PREC_FP64, ca.PREC_MIXED])
+def test_several_foams_in_a_small_launch(precision):
     """A foam's run does not depend on the foams beside it: each alone, and the
     three in one launch of few blocks and of many."""
-    cfgs = [config(2, 700, seed=7), config(3, 1500, seed=8), config(2, 300, seed=9)]
-    large = config(3, 1024 * 256 + 1, seed=10)
+    cfgs = [config(d, n, seed=s, precision=precision)
+            for d, n, s in ((2, 700, 7), (3, 1500, 8), (2, 300, 9))]
+    large = config(3, 1024 * 256 + 1, seed=10, precision=precision)
     ip = ca.IntegrationParams()
     alone = []
     for c in cfgs:
