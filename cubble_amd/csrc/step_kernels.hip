@@ -590,64 +590,72 @@ __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, c
     }
 }
 
-// dt controller and commit: reference src/simulator.cu:239-246, :258-321.
-// Returns whether the step removes bubbles.
-__device__ bool control(Foam *F, uint32_t flags, const CorrAcc &a) {
+// dt controller and commit: reference src/simulator.cu:239-246, :258-321, by
+// one thread, from copies of the header's parts that were read before (the
+// pointers' rotation in place took a load's time for each buffer: a load does
+// not pass the stores before it).  Returns whether the step removes bubbles.
+__device__ __forceinline__ bool control(Foam *F, const Dyn &was, const Roles &R, uint32_t flags,
+                                        const CorrAcc &a) {
     Dyn &d = F->d;
     const Consts &c = F->c;
+    const double tol = c.tol, skin = c.skin;
+    const int dim = c.dim;
+    const bool too_large = a.max_err > tol;
+    const bool increase = a.max_err < 0.45 * tol && was.dt < 10;
+    double ndt = was.dt;
+    if (too_large) {
+        ndt = was.dt * 0.37;
+    } else if (increase) {
+        ndt = was.dt * 1.269;
+    }
     d.s_v = a.s_v;
     d.max_err = a.max_err;
     d.max_r = a.max_r;
     d.max_exp = a.max_exp;
     d.n_del = a.n_del;
-    d.attempts += 1;
-    const double dt = d.dt;
-    const bool too_large = a.max_err > c.tol;
-    const bool increase = a.max_err < 0.45 * c.tol && dt < 10;
-    double ndt = dt;
-    if (too_large) {
-        ndt = dt * 0.37;
-    } else if (increase) {
-        ndt = dt * 1.269;
-    }
+    d.attempts = was.attempts + 1;
     d.dt = ndt;
     d.accepted = too_large ? 0 : 1;
-    d.need_remove = 0;  // the last one is done
-    if (too_large || !(flags & kCommit)) return false;
+    if (too_large || !(flags & kCommit)) {
+        d.need_remove = 0;  // the last one is done
+        return false;
+    }
     const bool gas = (flags & kGas) != 0;
-    Roles &R = F->r;
+    Roles &W = F->r;
     for (int k = 0; k < 4; ++k) {
-        if (2 == k && 2 == c.dim) continue;
+        if (2 == k && 2 == dim) continue;
         if (3 == k && !gas) continue;
-        void *t = R.vo[k];
-        R.vo[k] = R.v[k];
-        R.v[k] = R.vp[k];
-        R.vp[k] = t;
-        double *u = R.x[k];
-        R.x[k] = R.xp[k];
-        R.xp[k] = u;
+        W.vo[k] = R.v[k];
+        W.v[k] = R.vp[k];
+        W.vp[k] = R.vo[k];
+        W.x[k] = R.xp[k];
+        W.xp[k] = R.x[k];
     }
     if (flags & kPath) {
-        double *t = R.path;
-        R.path = R.path_new;
-        R.path_new = t;
+        W.path = R.path_new;
+        W.path_new = R.path;
     }
-    d.steps += 1;
-    d.bubble_steps += (double)d.count;
-    d.time_frac += ndt;
-    const uint64_t whole = (uint64_t)d.time_frac;
-    d.time_int += whole;
-    d.time_frac = d.time_frac - (double)whole;
-    if (gas) {
-        d.max_r_cell = a.max_r;
-        d.need_remove = a.n_del > 0 ? 1 : 0;
-    }
-    d.need_search = a.max_exp >= 0.5 * c.skin ? 1 : 0;
-    d.ts_min = fmin(d.ts_min, ndt);
-    d.ts_max = fmax(d.ts_max, ndt);
-    d.ts_sum += ndt;
-    if (stop_reached(d)) d.halt = 1;
-    return d.need_remove != 0;
+    // the stop rules look at the new state
+    Dyn now = was;
+    now.max_r = a.max_r;
+    now.steps = was.steps + 1;
+    const double frac = was.time_frac + ndt;
+    const uint64_t whole = (uint64_t)frac;
+    now.time_int = was.time_int + whole;
+    now.time_frac = frac - (double)whole;
+    d.steps = now.steps;
+    d.bubble_steps = was.bubble_steps + (double)was.count;
+    d.time_int = now.time_int;
+    d.time_frac = now.time_frac;
+    const bool removes = gas && a.n_del > 0;
+    if (gas) d.max_r_cell = a.max_r;
+    d.need_remove = removes ? 1 : 0;
+    d.need_search = a.max_exp >= 0.5 * skin ? 1 : 0;
+    d.ts_min = fmin(was.ts_min, ndt);
+    d.ts_max = fmax(was.ts_max, ndt);
+    d.ts_sum = was.ts_sum + ndt;
+    if (stop_reached(now)) d.halt = 1;
+    return removes;
 }
 
 template <int D, bool M, bool W>
@@ -721,7 +729,9 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
         return;
     }
     __shared__ int s_del;
-    const int n = F->d.count;
+    const Dyn was = F->d;
+    const Roles R = F->r;
+    const int n = was.count;
     // the volume sum, the maxima of error, radius and expansion, the
     // deletion count
     double r[4];
@@ -740,7 +750,7 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
         t.max_r = r[2];
         t.max_exp = r[3];
         t.n_del = nd;
-        s_del = control(F, flags, t) ? nd : 0;
+        s_del = control(F, was, R, flags, t) ? nd : 0;
     }
     __syncthreads();
     if (s_del > 0) plan_removal(F, n, s_del);
