@@ -185,7 +185,6 @@ enum Flags : uint32_t {
     kPath = 2u,
     kCommit = 4u,
     kFlow = 8u,
-    kOwnSums = 16u,  // the corrector forms the foam's sums itself
     kQuad = 64u,     // the pair kernel was k_pair_quad
     kApply = 32u,    // the predictor carries out the removal of the attempt before
 };

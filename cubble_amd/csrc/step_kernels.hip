@@ -499,26 +499,55 @@ struct CorrAcc {
     int n_del;
 };
 
+// What the gas exchange takes from a foam's sums, the same for every bubble.
+struct GasSums {
+    double inv_rho, flux;
+};
+
+__device__ __forceinline__ GasSums gas_sums(const Consts &c, int n, double s_a, double s_ar,
+                                            double s_oa, double s_oar) {
+    return GasSums{(s_ar - s_oar) / (s_a - s_oa), c.kappa * c.avg_area_in * n / s_a};
+}
+
 // MIXED: no FP64 predicted record is stored (recompute it) and velocities
 // are FP32.  WALLS false: no foam of the launch has a wall (the wall code,
-// and its registers, compiled out).
-template <int D, bool GAS, bool PATH, bool MIXED, bool WALLS>
+// and its registers, compiled out).  sums() gives the foam's GasSums; it is
+// called behind the loads of the first bubble.
+template <int D, bool GAS, bool PATH, bool MIXED, bool WALLS, bool OWN, typename Sums>
 __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, const Scratch &S,
-                                              const Dyn &dyn, int base, int ipt, int n,
+                                              double dt, int base, int ipt, int n, Sums &&sums,
                                               CorrAcc &a) {
     typedef typename std::conditional<MIXED, float, double>::type V;
-    const double h = 0.5 * dyn.dt;
+    const double h = 0.5 * dt;
     const bool walls = WALLS && (c.wall[0] || c.wall[1] || (3 == D && c.wall[2]));
-    const double inv_rho = (dyn.s_ar - dyn.s_oar) / (dyn.s_a - dyn.s_oa);
-    const double flux = c.kappa * c.avg_area_in * n / dyn.s_a;  // same for every bubble
+    GasSums gs{0.0, 0.0};
     for (int k = 0; k < ipt; ++k) {
         const int i = base + k * kBlock + (int)threadIdx.x;
-        if (i >= n) break;
-        const D4 pp = MIXED ? predicted<D, GAS, V>(R, h, i) : S.p4[i];
+        const bool valid = i < n;
+        if ((!OWN || k > 0) && !valid) break;  // (OWN: whole waves call sums())
+        const int at = valid ? i : 0;
+        const D4 pp = MIXED ? predicted<D, GAS, V>(R, h, at) : S.p4[at];
         const double pv[3] = {pp.x, pp.y, pp.z};
-        double vp[3];
+        double vp[3], xo[3], v[3], sv[4];
 #pragma unroll
-        for (int q = 0; q < D; ++q) vp[q] = (double)field<V>(R.vp[q])[i];
+        for (int q = 0; q < D; ++q) {
+            vp[q] = (double)field<V>(R.vp[q])[at];
+            xo[q] = R.x[q][at];
+            v[q] = (double)field<V>(R.v[q])[at];
+            sv[q] = (double)field<V>(R.saved[q])[at];
+        }
+        double ov = 0.0, vpr = 0.0, ro = 0.0, vr0 = 0.0;
+        if (GAS) {
+            ov = (double)field<V>(S.ov)[at];
+            vpr = (double)field<V>(R.vp[3])[at];
+            ro = R.x[3][at];
+            vr0 = (double)field<V>(R.v[3])[at];
+            sv[3] = (double)field<V>(R.saved[3])[at];
+        }
+        const double path = PATH ? R.path[at] : 0.0;
+        const double err = (double)field<V>(R.err)[at];
+        if (0 == k) gs = sums();
+        if (OWN && !valid) break;
         if (walls) {
             double vz = 3 == D ? vp[2] : 0.0;
             add_wall_velocity<D>(c, pp.x, pp.y, pp.z, pp.r, vp[0], vp[1], vz);
@@ -530,16 +559,15 @@ __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, c
             }
         }
         double e = 0.0, dist = 0.0;
-        double xo[3], xc[3];
+        double xc[3];
 #pragma unroll
         for (int q = 0; q < D; ++q) {
             const double pred = pv[q];
-            xo[q] = R.x[q][i];
-            const double corr = xo[q] + h * ((double)field<V>(R.v[q])[i] + vp[q]);
+            const double corr = xo[q] + h * (v[q] + vp[q]);
             xc[q] = corr;
             stream_store(R.xp[q] + i, corr);
             e = fmax(e, fabs(pred - corr));
-            const double t = corr - (double)field<V>(R.saved[q])[i];
+            const double t = corr - sv[q];
             dist += t * t;
         }
         dist = sqrt(dist);
@@ -548,17 +576,17 @@ __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, c
             double r = pp.r;
             double area = 2.0 * kPi * r;
             if (3 == D) area *= 2.0 * r;
-            double vr = inv_rho - rcp_nr(r);
-            vr *= flux * (area - (double)field<V>(S.ov)[i]);
-            vr += (double)field<V>(R.vp[3])[i];
+            double vr = gs.inv_rho - rcp_nr(r);
+            vr *= gs.flux * (area - ov);
+            vr += vpr;
             vr *= c.k_param * rcp_nr(area);
             stream_store(field<V>(R.vp[3]) + i, (V)vr);
             vr = (double)(V)vr;  // the stored value drives the corrector
             const double pred = r;
-            const double corr = R.x[3][i] + h * ((double)field<V>(R.v[3])[i] + vr);
+            const double corr = ro + h * (vr0 + vr);
             stream_store(R.xp[3] + i, corr);
             e = fmax(e, fabs(pred - corr));
-            dist += corr - (double)field<V>(R.saved[3])[i];
+            dist += corr - sv[3];
             r = corr;
             if (r > c.min_rad) {
                 double vol = r * r;
@@ -583,9 +611,9 @@ __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, c
                 t = xo[2] - xc[2];
                 pd += t * t;
             }
-            stream_store(R.path_new + i, R.path[i] + sqrt(pd));
+            stream_store(R.path_new + i, path + sqrt(pd));
         }
-        stream_store(field<V>(R.err) + i, (V)fmax(e, (double)field<V>(R.err)[i]));
+        stream_store(field<V>(R.err) + i, (V)fmax(e, err));
         a.max_err = fmax(a.max_err, e);
     }
 }
@@ -658,24 +686,26 @@ __device__ __forceinline__ bool control(Foam *F, const Dyn &was, const Roles &R,
     return removes;
 }
 
-template <int D, bool M, bool W>
+template <int D, bool M, bool W, bool OWN, typename Sums>
 __device__ __forceinline__ void correct_dispatch(const Consts &c, const Roles &R, const Scratch &S,
-                                                 const Dyn &dyn, int base, int ipt, int n,
-                                                 uint32_t flags, CorrAcc &a) {
+                                                 double dt, int base, int ipt, int n,
+                                                 uint32_t flags, Sums &&sums, CorrAcc &a) {
     const bool gas = (flags & kGas) != 0, path = (flags & kPath) != 0;
     if (gas) {
-        if (path) correct_range<D, true, true, M, W>(c, R, S, dyn, base, ipt, n, a);
-        else correct_range<D, true, false, M, W>(c, R, S, dyn, base, ipt, n, a);
+        if (path) correct_range<D, true, true, M, W, OWN>(c, R, S, dt, base, ipt, n, sums, a);
+        else correct_range<D, true, false, M, W, OWN>(c, R, S, dt, base, ipt, n, sums, a);
     } else {
-        if (path) correct_range<D, false, true, M, W>(c, R, S, dyn, base, ipt, n, a);
-        else correct_range<D, false, false, M, W>(c, R, S, dyn, base, ipt, n, a);
+        if (path) correct_range<D, false, true, M, W, OWN>(c, R, S, dt, base, ipt, n, sums, a);
+        else correct_range<D, false, false, M, W, OWN>(c, R, S, dt, base, ipt, n, sums, a);
     }
 }
 
 // One kernel per precision (MIXED: FP32 velocity buffers, recomputed
-// prediction) and per wall presence (WALLS: some foam of the launch has a
-// wall), so that none pays the registers of another.
-template <bool MIXED, bool WALLS>
+// prediction), per wall presence (WALLS: some foam of the launch has a
+// wall) and per place of the foam's sums (OWN: formed here, behind the block's
+// own loads; else k_sums formed them), so that none pays the registers of
+// another.
+template <bool MIXED, bool WALLS, bool OWN>
 __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt, uint32_t flags) {
     const Ctx cx = bubble_ctx(foams, bt);
     Foam *F = cx.F;
@@ -684,15 +714,12 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
     const Consts c = F->c;
     const Roles R = F->r;
     const Scratch S = F->s;
-    Dyn dyn = F->d;
+    const double dt = F->d.dt;
     const int base = cx.lb * kBlock * ipt;
-    if (flags & kOwnSums) {
+    auto sums = [&]() {
+        if (!OWN) return gas_sums(c, n, F->d.s_a, F->d.s_ar, F->d.s_oa, F->d.s_oar);
         double r[4];
         wave_foam_sums(S.part, flags & kQuad ? quad_parts(S) : nullptr, F->nblk, r);
-        dyn.s_a = r[0];
-        dyn.s_ar = r[1];
-        dyn.s_oa = r[2];
-        dyn.s_oar = r[3];
         // for the host; the other blocks use their own
         if (0 == cx.lb && 0 == threadIdx.x) {
             F->d.s_a = r[0];
@@ -700,10 +727,13 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
             F->d.s_oa = r[2];
             F->d.s_oar = r[3];
         }
-    }
+        return gas_sums(c, n, r[0], r[1], r[2], r[3]);
+    };
     CorrAcc a{0.0, 0.0, 0.0, 0.0, 0};
-    if (3 == c.dim) correct_dispatch<3, MIXED, WALLS>(c, R, S, dyn, base, ipt, n, flags, a);
-    else correct_dispatch<2, MIXED, WALLS>(c, R, S, dyn, base, ipt, n, flags, a);
+    if (3 == c.dim)
+        correct_dispatch<3, MIXED, WALLS, OWN>(c, R, S, dt, base, ipt, n, flags, sums, a);
+    else
+        correct_dispatch<2, MIXED, WALLS, OWN>(c, R, S, dt, base, ipt, n, flags, sums, a);
     // the volume sum, then the maxima of error, radius and expansion
     double r4[4] = {a.s_v, a.max_err, a.max_r, a.max_exp};
     int nd = a.n_del;
@@ -856,22 +886,16 @@ void launch_bootstrap(const Grid &g, bool mixed) {
 
 void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control) {
     const dim3 grid(g.nb_bub), block(kBlock);
-    if (!g.big) flags |= kOwnSums;
     if (g.quad) flags |= kQuad;
-    if (mixed) {
-        if (g.walls)
-            hipLaunchKernelGGL((k_correct<true, true>), grid, block, 0, g.stream, g.foams,
-                               g.bt_bub, flags);
-        else
-            hipLaunchKernelGGL((k_correct<true, false>), grid, block, 0, g.stream, g.foams,
-                               g.bt_bub, flags);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, g.stream, g.foams, g.bt_bub, flags);
+    };
+    if (g.big) {
+        if (mixed) g.walls ? launch(k_correct<true, true, false>) : launch(k_correct<true, false, false>);
+        else g.walls ? launch(k_correct<false, true, false>) : launch(k_correct<false, false, false>);
     } else {
-        if (g.walls)
-            hipLaunchKernelGGL((k_correct<false, true>), grid, block, 0, g.stream, g.foams,
-                               g.bt_bub, flags);
-        else
-            hipLaunchKernelGGL((k_correct<false, false>), grid, block, 0, g.stream, g.foams,
-                               g.bt_bub, flags);
+        if (mixed) g.walls ? launch(k_correct<true, true, true>) : launch(k_correct<true, false, true>);
+        else g.walls ? launch(k_correct<false, true, true>) : launch(k_correct<false, false, true>);
     }
     if (control)
         hipLaunchKernelGGL(k_control, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams, flags);
