@@ -57,11 +57,14 @@ struct Tuning {
 };
 
 // Attempts between two search phases of a captured run.  A search is needed
-// every 20 to 80 steps (14 in the first steps after seeding), and its seven
+// every 20 to 80 steps (14 in the first steps after seeding), and its eight
 // launches cost 1.5 to 4.5 us each when no foam needs them; a foam that does
 // stands still until the next phase, which costs it the few idle launches of
-// the attempts between.
-constexpr int kSearchEvery = 8;
+// the attempts between.  Runs at 8 / 12 / 16: 2D 1e3 5.91 / 5.91 / 5.66 ms, 1e4
+// 8.73 / 8.73 / 8.42, 3D 1e5 16.9 / 16.9 / 16.75, 1e6 20.6 / 20.7 / 20.5, 256
+// foams 32.7 / 32.8 / 32.1 (a graph holds 16 attempts by default, and ends with
+// a phase).
+constexpr int kSearchEvery = 16;
 
 // Launches of at most this many blocks carry out removals in the predictor: a
 // launch for them costs 2.5 us an attempt (2D 1e4: 10.9 ms with it, 10.4
