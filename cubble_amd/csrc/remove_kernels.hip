@@ -31,7 +31,16 @@ namespace cubble_amd {
 // own.
 __global__ __launch_bounds__(kBlock) void k_rm_plan(Foam *foams) {
     Foam *F = foams + blockIdx.x;
-    if (F->d.need_remove) plan_removal(F, F->d.count, F->d.n_del);
+    if (!F->d.need_remove) return;
+    __shared__ DeletedBlocks s_blocks;
+    if (0 == threadIdx.x) s_blocks.m = 0;
+    __syncthreads();
+    for (int b = threadIdx.x; b < F->nblk; b += kBlock) {
+        const int c = F->s.part_i[b * kPartI];
+        if (c > 0) s_blocks.add(b, c);
+    }
+    __syncthreads();
+    plan_removal(F, s_blocks, F->d.count, F->d.n_del);
 }
 
 // Removals of the last attempt before a search phase, and of foams that stand

@@ -234,11 +234,12 @@ __device__ __forceinline__ void block_sums(const double *part, const double *qua
 
 // One value quadruple per block, read(b, v), reduced in one pass (each thread
 // takes blocks t, t + kBlock, ... in order), and the integer slot 0 of the int
-// partials summed alongside if part_i.  Bit k of `dmax` makes value k a maximum
+// partials summed alongside, their non-zero ones given to found(b, count), if
+// part_i.  Bit k of `dmax` makes value k a maximum
 // (from 0), else a sum.  The results are defined in thread 0 only.
-template <typename Read>
-__device__ __forceinline__ void reduce_parts4(Read &&read, const int32_t *part_i, int nb,
-                                              unsigned dmax, double (&r)[4], int &ri) {
+template <typename Read, typename Found>
+__device__ __forceinline__ void reduce_parts4(Read &&read, const int32_t *part_i, Found &&found,
+                                              int nb, unsigned dmax, double (&r)[4], int &ri) {
     double a[4] = {0.0, 0.0, 0.0, 0.0};
     int ai = 0;
 #pragma unroll 2
@@ -247,7 +248,11 @@ __device__ __forceinline__ void reduce_parts4(Read &&read, const int32_t *part_i
         read(b, v);
 #pragma unroll
         for (int k = 0; k < 4; ++k) a[k] = (dmax >> k) & 1u ? fmax(a[k], v[k]) : a[k] + v[k];
-        if (part_i) ai += part_i[b * kPartI];
+        if (part_i) {
+            const int c = part_i[b * kPartI];
+            if (c > 0) found(b, c);
+            ai += c;
+        }
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) r[k] = a[k];
@@ -422,8 +427,8 @@ __global__ __launch_bounds__(kBlock) void k_sums(Foam *foams, bool quad) {
     double r[4];
     int none;
     const double *const part = F->s.part, *const q = quad ? quad_parts(F->s) : nullptr;
-    reduce_parts4([&](int b, double (&v)[4]) { block_sums(part, q, b, v); }, nullptr, F->nblk, 0u,
-                  r, none);
+    reduce_parts4([&](int b, double (&v)[4]) { block_sums(part, q, b, v); }, nullptr,
+                  [](int, int) {}, F->nblk, 0u, r, none);
     if (threadIdx.x == 0) {
         F->d.s_a = r[0];
         F->d.s_ar = r[1];
@@ -759,6 +764,9 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
         return;
     }
     __shared__ int s_del;
+    __shared__ DeletedBlocks s_blocks;
+    if (0 == threadIdx.x) s_blocks.m = 0;
+    __syncthreads();
     const Dyn was = F->d;
     const Roles R = F->r;
     const int n = was.count;
@@ -772,7 +780,7 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
 #pragma unroll
             for (int k = 0; k < 4; ++k) v[k] = part[b * kPartD + 4 + k];
         },
-        F->s.part_i, F->nblk, 0xeu, r, nd);
+        F->s.part_i, [&](int b, int c) { s_blocks.add(b, c); }, F->nblk, 0xeu, r, nd);
     if (threadIdx.x == 0) {
         CorrAcc t;
         t.s_v = r[0];
@@ -783,7 +791,8 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
         s_del = control(F, was, R, flags, t) ? nd : 0;
     }
     __syncthreads();
-    if (s_del > 0) plan_removal(F, n, s_del);
+    nd = s_del;
+    if (nd > 0) plan_removal(F, s_blocks, n, nd);
 }
 
 // ---------------------------------------------------------------- launches
