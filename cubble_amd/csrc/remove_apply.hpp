@@ -90,54 +90,94 @@ __device__ __forceinline__ void filter_list(const Scratch &S, size_t cap, int nn
     S.nn[i] = out;
 }
 
+// Bubble i's own list of at most 16 entries, filtered by 16 lanes (g: which of
+// the wave's four groups).  j: this lane's entry, -1 past the end.
+__device__ __forceinline__ void filter_short(const Scratch &S, size_t cap, int nnew, int i, int j,
+                                             int g) {
+    const int lane = (int)(threadIdx.x & 15);
+    const bool keep = j >= 0 && !S.del[j];
+    const bool moved = keep && j >= nnew;
+    const int jj = moved ? S.moved_to[j - nnew] : j;
+    const unsigned kept = (unsigned)(__builtin_amdgcn_ballot_w64(keep) >> (16 * g)) & 0xffffu;
+    int pos = __popc(kept & ((1u << lane) - 1u));
+    if (__builtin_amdgcn_ballot_w64(moved)) {
+        pos = 0;
+        for (int k = 0; k < 16; ++k) {
+            const int v = __shfl(jj, 16 * g + k);
+            pos += (kept >> k & 1u) && v < jj ? 1 : 0;
+        }
+    }
+    if (keep) S.nbr[(size_t)pos * cap + i] = jj;
+    if (0 == lane && i >= 0) S.nn[i] = __popc(kept);
+}
+
 // The planned removal on the slots of bubble-space block lb, by its whole
 // workgroup: each thread applies the volume fix to its bubbles; the few holes
-// and marked bubbles are listed in LDS and rebuilt by one wave each.  No block
-// reads a slot that another one writes: the survivors lie past the new count.
-// What bounds it is the rebuild's chain of dependent loads (list, marks, new
-// slots) behind one pass over marks and radii.
+// and marked bubbles are listed in LDS and rebuilt, a marked bubble with a short
+// list by 16 lanes, the others by one wave each.  No block reads a slot that
+// another one writes: the survivors lie past the new count.  What bounds it is
+// the rebuild's chain of dependent loads (list, marks, new slots) behind one
+// pass over marks and radii; the ten or so neighbours of a deleted bubble are
+// in few blocks, so that rebuilt by a wave each they took three such chains.
 __device__ __forceinline__ void apply_removal(const Foam *F, int lb) {
-    __shared__ int s_cnt, s_list[kBlock];
+    // marked bubbles from the front of the list, holes from its back
+    __shared__ int s_cnt, s_holes, s_list[kBlock];
     const Scratch S = F->s;
     double *const r = F->r.x[3];
     const int nnew = F->d.count, h = F->d.n_holes, ipt = F->ipt;
     const double vm = F->d.vol_fix;
     const size_t cap = (size_t)F->cap;
-    const int lane = (int)(threadIdx.x & 63);
+    const int nbr_cap = F->nbr_cap;
+    const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
     for (int k = 0; k < ipt; ++k) {
         const int base = (lb * ipt + k) * kBlock;
         if (base >= nnew) break;  // uniform per block
         const int i = base + (int)threadIdx.x;
-        if (0 == threadIdx.x) s_cnt = 0;
+        if (0 == threadIdx.x) s_cnt = s_holes = 0;
         __syncthreads();
         if (i < nnew) {
             const bool hole = S.del[i] != 0;
             const bool marked = S.dirty[i] != 0;
             if (!hole) r[i] = r[i] * vm;
             if (marked) S.dirty[i] = 0;
-            if (hole || marked) s_list[atomicAdd(&s_cnt, 1)] = hole ? ~i : i;
+            if (hole) s_list[kBlock - 1 - atomicAdd(&s_holes, 1)] = i;
+            else if (marked) s_list[atomicAdd(&s_cnt, 1)] = i;
         }
         __syncthreads();
-        const int cnt = s_cnt;
-        for (int e = threadIdx.x >> 6; e < cnt; e += kWaves) {
-            const int v = uniform_i(s_list[e]);
-            const bool hole = v < 0;
-            const int b = hole ? ~v : v;
-            int src = b;
-            if (hole) {  // the k-th entry of the deletion list is the k-th hole
-                for (int k0 = 0; k0 < h; k0 += 64) {
-                    const bool in = k0 + lane < h;
-                    const int d = in ? S.del_list[k0 + lane] : -1;
-                    const int s = in ? S.plan_src[k0 + lane] : -1;
-                    const unsigned long long at = __builtin_amdgcn_ballot_w64(d == b);
-                    if (at) {
-                        src = __builtin_amdgcn_readlane(s, __builtin_ctzll(at));
-                        break;
-                    }
+        const int cnt = s_cnt, holes = s_holes;
+        // the last waves first: the marked bubbles go to the first
+        for (int e = kWaves - 1 - wave; e < holes; e += kWaves) {
+            const int b = uniform_i(s_list[kBlock - 1 - e]);
+            int src = b;  // the k-th entry of the deletion list is the k-th hole
+            for (int k0 = 0; k0 < h; k0 += 64) {
+                const bool in = k0 + lane < h;
+                const int d = in ? S.del_list[k0 + lane] : -1;
+                const int s = in ? S.plan_src[k0 + lane] : -1;
+                const unsigned long long at = __builtin_amdgcn_ballot_w64(d == b);
+                if (at) {
+                    src = __builtin_amdgcn_readlane(s, __builtin_ctzll(at));
+                    break;
                 }
-                move_state(F, b, src, vm);
             }
+            move_state(F, b, src, vm);
             filter_list(S, cap, nnew, b, src);
+        }
+        // (a wave's four groups together: the ballots need them)
+        for (int e0 = 4 * wave; e0 < cnt; e0 += kBlock / 16) {
+            const int e = e0 + (lane >> 4), q = lane & 15;
+            const int b = e < cnt ? s_list[e] : -1;
+            int j = -1, m = 0;
+            if (b >= 0) {
+                j = S.nbr[(size_t)min(q, nbr_cap - 1) * cap + b];
+                m = S.nn[b];
+            }
+            const bool brief = m <= 16;
+            filter_short(S, cap, nnew, brief ? b : -1, brief && q < m ? j : -1, lane >> 4);
+            for (unsigned long long t = __builtin_amdgcn_ballot_w64(!brief && 0 == q); t;
+                 t &= t - 1ull) {
+                const int v = __builtin_amdgcn_readlane(b, __builtin_ctzll(t));
+                filter_list(S, cap, nnew, v, v);
+            }
         }
         __syncthreads();
     }
