@@ -41,17 +41,21 @@ __device__ __forceinline__ double cells_range(const Consts &c, const Roles &R, c
         const bool valid = i < n;
         int cid = -1;
         if (valid) {
+            // (all loads before a store, which they would not pass)
             double p[3] = {0.0, 0.0, 0.0};
 #pragma unroll
+            for (int q = 0; q < D; ++q) p[q] = R.x[q][i];
+            rmax = fmax(rmax, R.x[3][i]);
+#pragma unroll
             for (int q = 0; q < D; ++q) {
-                double xv = R.x[q][i];
-                if (!c.wall[q]) {
-                    const int mult = xv < c.lbb[q] ? 1 : (xv > c.tfr[q] ? -1 : 0);
-                    xv = xv + (c.tfr[q] - c.lbb[q]) * (double)mult;
-                    R.x[q][i] = xv;
-                    if (mult) R.wc[q][i] -= mult;
+                const double xv = p[q];
+                const int mult = c.wall[q] || (xv >= c.lbb[q] && xv <= c.tfr[q]) ? 0
+                                 : xv < c.lbb[q] ? 1 : (xv > c.tfr[q] ? -1 : 0);
+                if (mult) {
+                    p[q] = xv + (c.tfr[q] - c.lbb[q]) * (double)mult;
+                    R.x[q][i] = p[q];
+                    R.wc[q][i] -= mult;
                 }
-                p[q] = xv;
             }
             int id[3] = {0, 0, 0};
 #pragma unroll
@@ -61,7 +65,6 @@ __device__ __forceinline__ double cells_range(const Consts &c, const Roles &R, c
             }
             cid = id[2] * cd[0] * cd[1] + id[1] * cd[0] + id[0];
             S.cell_of[i] = cid;
-            rmax = fmax(rmax, R.x[3][i]);
         }
         const WaveRuns wr = wave_runs(cid, valid);
         if (valid && (int)(threadIdx.x & 63) == wr.head) atomicAdd(&S.cell_count[cid], wr.len);
@@ -172,6 +175,23 @@ __device__ __forceinline__ void reorder_range(const Roles &R, const Scratch &S, 
     for (int k = 0; k < ipt; ++k) {
         const int i = base + k * kBlock + (int)threadIdx.x;
         if (i >= n) break;
+        // the whole state before any store (which the loads would not pass),
+        // and before the chain to the new slot
+        double xs[4] = {0.0, 0.0, 0.0, 0.0};
+        V v[4], vo[4];
+        int wc[3];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (2 == q && 2 == D) continue;
+            xs[q] = R.x[q][i];
+            v[q] = field<V>(R.v[q])[i];
+            vo[q] = field<V>(R.vo[q])[i];
+        }
+        const double path = R.path[i];
+        const V err = field<V>(R.err)[i];
+#pragma unroll
+        for (int q = 0; q < D; ++q) wc[q] = R.wc[q][i];
+        const int idx = R.idx[i];
         const int c = S.cell_of[i];
         const int s0 = S.cell_start[c], s1 = S.cell_start[c + 1];
         // rank among the cell's members by old index; the members are loaded
@@ -186,23 +206,20 @@ __device__ __forceinline__ void reorder_range(const Roles &R, const Scratch &S, 
             for (int u = 0; u < 8; ++u) rank += mb[u] < i ? 1 : 0;
         }
         const int np = s0 + rank;
-        double xs[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             if (2 == q && 2 == D) continue;
-            const double xv = R.x[q][i];
-            xs[q] = xv;
-            R.xp[q][np] = xv;
-            field<V>(R.saved[q])[np] = (V)xv;
-            field<V>(R.vp[q])[np] = field<V>(R.v[q])[i];
-            field<V>(R.vs[q])[np] = field<V>(R.vo[q])[i];
+            R.xp[q][np] = xs[q];
+            field<V>(R.saved[q])[np] = (V)xs[q];
+            field<V>(R.vp[q])[np] = v[q];
+            field<V>(R.vs[q])[np] = vo[q];
         }
         S.x4[np] = D4{xs[0], xs[1], xs[2], xs[3]};
-        R.path_new[np] = R.path[i];
-        field<V>(R.err_alt)[np] = field<V>(R.err)[i];
+        R.path_new[np] = path;
+        field<V>(R.err_alt)[np] = err;
 #pragma unroll
-        for (int q = 0; q < D; ++q) R.wc_alt[q][np] = R.wc[q][i];
-        R.idx_alt[np] = R.idx[i];
+        for (int q = 0; q < D; ++q) R.wc_alt[q][np] = wc[q];
+        R.idx_alt[np] = idx;
     }
 }
 
