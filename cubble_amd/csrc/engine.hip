@@ -453,6 +453,7 @@ int Engine::restore(const Snapshot &s) {
 }
 
 Grid Engine::grid() const {
+    clean_ = false;  // whatever the caller launches may halt a foam
     Grid g;
     g.foams = dfoams_;
     const bool one = 1 == foams.size();  // its blocks are the launch's
@@ -481,13 +482,13 @@ Grid Engine::grid() const {
     return g;
 }
 
-void Engine::enqueue_attempt(uint32_t flags) {
+void Engine::enqueue_attempt(uint32_t flags, Dyn *mirror) {
     const Grid g = grid();
     launch_predict(g, flags);
     if (CUBBLE_PREC_MIXED == precision) launch_pair_mixed(g, flags);
     else launch_pair(g, flags);
     launch_sums(g);
-    launch_correct(g, flags, CUBBLE_PREC_MIXED == precision);
+    launch_correct(g, flags, CUBBLE_PREC_MIXED == precision, true, mirror);
 }
 
 void Engine::enqueue_groups(uint32_t flags, int groups) {
@@ -545,6 +546,23 @@ __global__ __launch_bounds__(64) void k_read(const uint64_t *src, uint64_t *dst,
                                              int stride) {
     for (int w = threadIdx.x; w < words; w += 64)
         dst[(size_t)blockIdx.x * words + w] = src[(size_t)blockIdx.x * stride + w];
+}
+
+int Engine::read_mirror(std::vector<Dyn> &out) {
+    E_TRY(hipGetLastError());
+    E_TRY(hipStreamSynchronize(stream));
+    out.resize(foams.size());
+    if (!out.empty()) std::memcpy(out.data(), pinned_, sizeof(Dyn) * out.size());
+    return CUBBLE_OK;
+}
+
+int Engine::attempt(uint32_t flags, std::vector<Dyn> &d) {
+    int rc = clean_ ? CUBBLE_OK : set_limits(0, nullptr);
+    if (rc) return rc;
+    enqueue_attempt(flags, pinned_);
+    rc = read_mirror(d);
+    clean_ = 0 == rc;  // without a commit an attempt halts no foam
+    return rc;
 }
 
 int Engine::read_dyn_all(std::vector<Dyn> &out) {
@@ -712,17 +730,20 @@ int Engine::set_limits(int64_t steps, const std::vector<int64_t> *per_foam) {
 int Engine::lift_limits(std::vector<Dyn> &d) {
     const int rc = set_limits(0, nullptr);
     for (Dyn &x : d) x.halt = x.overflow = x.step_limit = 0;
+    if (0 == rc) clean_ = true;
     return rc;
 }
 
 int Engine::integrate(uint32_t flags, std::vector<Dyn> &d) {
-    int rc = set_limits(1, nullptr);
+    // One foam needs no step limit: the host looks at every attempt.  (Between
+    // calls none is halted, unless a call failed.)
+    const bool one = 1 == foams.size();
+    int rc = one && clean_ ? CUBBLE_OK : set_limits(one ? 0 : 1, nullptr);
     if (rc) return rc;
     for (int tries = 0; tries < 100000; ++tries) {
-        enqueue_attempt(flags);
+        enqueue_attempt(flags, pinned_);
         launch_apply(grid());
-        E_TRY(hipGetLastError());
-        if ((rc = read_dyn_all(d))) return rc;
+        if ((rc = read_mirror(d))) return rc;
         // the search's launches only when some foam needs them
         bool search = false;
         for (const Dyn &x : d) search = search || x.need_search;
@@ -732,7 +753,11 @@ int Engine::integrate(uint32_t flags, std::vector<Dyn> &d) {
             if ((rc = read_dyn_all(d))) return rc;
         }
         if ((rc = settle_read(d))) return rc;
-        if (steps_left(d) == 0) return lift_limits(d);
+        if (one && d[0].accepted && !d[0].halt && !d[0].overflow) {
+            clean_ = true;
+            return CUBBLE_OK;
+        }
+        if (one ? d[0].accepted || steps_left(d) == 0 : steps_left(d) == 0) return lift_limits(d);
     }
     return fail(CUBBLE_E_STATE, "integrate: no accepted step after 100000 attempts");
 }

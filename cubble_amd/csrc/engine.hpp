@@ -123,7 +123,10 @@ class Engine {
     int search_pending();
 
     Grid grid() const;
-    void enqueue_attempt(uint32_t flags);
+    // mirror: as launch_correct's
+    void enqueue_attempt(uint32_t flags, Dyn *mirror = nullptr);
+    // One attempt without its commit, and every foam's scalars after it.
+    int attempt(uint32_t flags, std::vector<Dyn> &d);
     // `groups` attempts with their removals; a search phase after every
     // kSearchEvery of them and at the end
     void enqueue_groups(uint32_t flags, int groups);
@@ -183,6 +186,8 @@ class Engine {
   private:
     int grow_lists(int k, int need, bool rebuild, bool keep = false);
     int pull_headers();
+    // Wait for the stream and take the scalars a launch left in pinned_.
+    int read_mirror(std::vector<Dyn> &out);
     Tuning tuning_;
     Foam *dfoams_ = nullptr;
     int dfoams_cap_ = 0;
@@ -197,6 +202,7 @@ class Engine {
     int graph_groups_ = 0;
     bool graph_walls_ = false, graph_big_ = false, graph_quad_ = false;
     int graph_threads_ = 0;
+    mutable bool clean_ = false;  // no foam is halted or has a step limit
     bool opened_ = false;  // counted among the users of the pinned blocks
     int committed_nf_ = 0;  // foams in the device array at the last commit
 

@@ -37,8 +37,10 @@ void launch_pair_mixed(const Grid &g, uint32_t flags, bool fix = true);
 void launch_sums(const Grid &g);
 // corrector (mixed: the mixed-precision variant, for engines of that
 // precision), then (control) the dt controller / commit and the plan of a
-// removal (one block per foam)
-void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control = true);
+// removal (one block per foam), and the foams' scalars into `mirror` (pinned
+// host memory, one record per foam) if given
+void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control = true,
+                    Dyn *mirror = nullptr);
 
 // The planned removals: move the tail survivors into the holes, filter /
 // remap the neighbour lists and apply the volume fix.  Runs only for foams

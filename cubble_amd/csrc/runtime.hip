@@ -356,11 +356,8 @@ int cubble_step(cubble_sim *s, const cubble_integrate_params *ip, cubble_step_re
     if (!s) return CUBBLE_E_INVALID;
     Engine &e = s->e;
     int rc = CUBBLE_OK;
-    launch_set_flags(e.grid(), -1, -1, 1);
-    e.enqueue_attempt(flags_of(ip));
-    R_TRY(e, hipGetLastError());
     std::vector<Dyn> d;
-    if ((rc = e.read_dyn_all(d))) return rc;
+    if ((rc = e.attempt(flags_of(ip), d))) return rc;
     fill_result(d[0], res);
     return CUBBLE_OK;
 }

@@ -755,8 +755,7 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
 // One block per foam: reduce the corrector partials, then the dt controller
 // and (when committing) the role rotation and the plan of a removal, which
 // the next launch applies.
-__global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags) {
-    Foam *F = touch_header(foams + blockIdx.x);
+__device__ __forceinline__ void control_block(Foam *F, uint32_t flags) {
     if (standing(F->d)) {
         // the removal of its last step is done, or (kApply) waits for the
         // search phase
@@ -793,6 +792,18 @@ __global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags)
     __syncthreads();
     nd = s_del;
     if (nd > 0) plan_removal(F, s_blocks, n, nd);
+}
+
+// mirror: pinned host memory that receives the foams' scalars as they are then
+// (a launch less than reading them afterwards), or null.
+__global__ __launch_bounds__(kBlock) void k_control(Foam *foams, uint32_t flags, Dyn *mirror) {
+    Foam *F = touch_header(foams + blockIdx.x);
+    control_block(F, flags);
+    if (!mirror) return;
+    __syncthreads();
+    for (int w = threadIdx.x; w < (int)(sizeof(Dyn) / 8); w += kBlock)
+        reinterpret_cast<uint64_t *>(mirror + blockIdx.x)[w] =
+            reinterpret_cast<const volatile uint64_t *>(&F->d)[w];
 }
 
 // ---------------------------------------------------------------- launches
@@ -893,7 +904,7 @@ void launch_bootstrap(const Grid &g, bool mixed) {
                        g.bt_bub);
 }
 
-void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control) {
+void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control, Dyn *mirror) {
     const dim3 grid(g.nb_bub), block(kBlock);
     if (g.quad) flags |= kQuad;
     auto launch = [&](auto kernel) {
@@ -907,7 +918,8 @@ void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control) {
         else g.walls ? launch(k_correct<false, true, true>) : launch(k_correct<false, false, true>);
     }
     if (control)
-        hipLaunchKernelGGL(k_control, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams, flags);
+        hipLaunchKernelGGL(k_control, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams, flags,
+                           mirror);
 }
 
 }  // namespace cubble_amd
