@@ -473,7 +473,7 @@ Grid Engine::grid() const {
         for (int a = 0; a < r.h.c.dim; ++a) g.walls = g.walls || r.h.c.wall[a] != 0;
         all3 = all3 && 3 == r.h.c.dim;
         g.quad = g.quad && 1 == r.h.ipt;
-        g.big = g.big || r.h.nblk > kFuseBlocks;
+        g.big = g.big || r.h.nblk > (one ? kFuseBlocks : kFuseBatch);
         g.search_threads =
             std::max(g.search_threads, std::min(kBlock, (r.h.stile + 63) / 64 * 64));
     }

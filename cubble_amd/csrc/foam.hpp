@@ -21,8 +21,11 @@ namespace cubble_amd {
 constexpr int kBlock = 256;         // threads per block, bubble- and cell-space
 constexpr int kMaxBlocks = 2048;    // bubble-space blocks per foam (partials)
 constexpr int kNumXcd = 8;          // MI355X: 8 XCDs, workgroups round-robin
-constexpr int kFuseBlocks = 128;    // launches of foams of at most this many blocks sum their
-                                    // partials in k_correct
+// Foams of at most this many blocks have their partials summed in k_correct: a
+// foam alone, and all foams of a batch.  Every block reads them all: 3D mixed at
+// 391 blocks 4.4 -> 6.5 us a launch for the 3.5 of k_sums and its launch, at 625
+// 5.1 -> 7.3; at 782 (2D FP64) 6.4 -> 11.2, no gain any more.
+constexpr int kFuseBlocks = 640, kFuseBatch = 128;
 // Launches of at most this many blocks, one bubble a thread, take four lanes a
 // bubble in the pair kernel: FP64, mixed with 3D foams only, mixed with 2D ones
 // (a 2D list is half as long, and FP32 leaves less to overlap).

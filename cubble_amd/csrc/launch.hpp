@@ -23,7 +23,7 @@ struct Grid {
     hipStream_t stream;
     bool walls;  // some foam of the launch has a wall
     bool quad;   // the FP64 pair kernel is k_pair_quad: one bubble a thread, few blocks
-    bool big;    // some foam of the launch has more than kFuseBlocks blocks
+    bool big;    // some foam of the launch has more blocks than k_correct sums itself
 };
 
 void launch_predict(const Grid &g, uint32_t flags);
@@ -32,7 +32,7 @@ void launch_pair(const Grid &g, uint32_t flags);
 // a pair needing FP64 values.
 void launch_pair_mixed(const Grid &g, uint32_t flags, bool fix = true);
 // S_A, S_Ar, S_OA, S_OAr from the predictor and pair partials (one block per
-// foam), when some foam of the launch has more than kFuseBlocks blocks;
+// foam), when some foam of the launch has more blocks than k_correct sums;
 // otherwise the corrector forms them
 void launch_sums(const Grid &g);
 // corrector (mixed: the mixed-precision variant, for engines of that

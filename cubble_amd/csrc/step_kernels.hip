@@ -437,23 +437,38 @@ __global__ __launch_bounds__(kBlock) void k_sums(Foam *foams, bool quad) {
     }
 }
 
-// S_A, S_Ar, S_OA, S_OAr of a foam of at most kFuseBlocks <= kBlock blocks, by
-// every wave for itself and without a barrier: 64 block partials per round,
-// the rounds in order -- the waves of k_sums, so the same bits.  Reading them
-// again in every block of the corrector costs it under a microsecond up to
-// two rounds; the launch of k_sums it replaces costs 2.5.  In a batch the
-// launch is the cheaper one: 256 foams' correctors took 36 us longer.
-__device__ __forceinline__ void wave_foam_sums(const double *__restrict__ part,
-                                               const double *__restrict__ quad, int nb,
-                                               double (&r)[4]) {
+// S_A, S_Ar, S_OA, S_OAr of a foam, in every thread of the calling workgroup:
+// the sums of k_sums in its order, so the same bits.  Reading the partials in
+// every block of the corrector costs it under a microsecond up to kFuseBlocks;
+// the launch of k_sums that it replaces costs 2.5 to 3.5.  In a batch the launch
+// is the cheaper one: 256 foams' correctors took 36 us longer.
+// Up to 64 blocks every wave sums for itself, without a barrier.
+__device__ __forceinline__ void block_foam_sums(const double *__restrict__ part,
+                                                const double *__restrict__ quad, int nb,
+                                                double (&r)[4]) {
+    __shared__ double s_sum[kWaves][4];
+    const bool few = nb <= 64;
 #pragma unroll
     for (int k = 0; k < 4; ++k) r[k] = 0.0;
-    for (int b0 = 0; b0 < nb; b0 += 64) {
-        const int b = b0 + (int)(threadIdx.x & 63);
-        double v[4] = {0.0, 0.0, 0.0, 0.0};
-        if (b < nb) block_sums(part, quad, b, v);
+    for (int b = few ? threadIdx.x & 63 : threadIdx.x; b < nb; b += kBlock) {
+        double v[4];
+        block_sums(part, quad, b, v);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) r[k] += wave_sum(v[k]);
+        for (int k = 0; k < 4; ++k) r[k] += v[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[k] = wave_sum(r[k]);
+    if (few) return;
+    if (0 == (threadIdx.x & 63)) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s_sum[threadIdx.x >> 6][k] = r[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        r[k] = 0.0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) r[k] += s_sum[w][k];
     }
 }
 
@@ -529,7 +544,7 @@ __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, c
     for (int k = 0; k < ipt; ++k) {
         const int i = base + k * kBlock + (int)threadIdx.x;
         const bool valid = i < n;
-        if ((!OWN || k > 0) && !valid) break;  // (OWN: whole waves call sums())
+        if ((!OWN || k > 0) && !valid) break;  // (OWN: the whole workgroup calls sums())
         const int at = valid ? i : 0;
         const D4 pp = MIXED ? predicted<D, GAS, V>(R, h, at) : S.p4[at];
         const double pv[3] = {pp.x, pp.y, pp.z};
@@ -724,7 +739,7 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
     auto sums = [&]() {
         if (!OWN) return gas_sums(c, n, F->d.s_a, F->d.s_ar, F->d.s_oa, F->d.s_oar);
         double r[4];
-        wave_foam_sums(S.part, flags & kQuad ? quad_parts(S) : nullptr, F->nblk, r);
+        block_foam_sums(S.part, flags & kQuad ? quad_parts(S) : nullptr, F->nblk, r);
         // for the host; the other blocks use their own
         if (0 == cx.lb && 0 == threadIdx.x) {
             F->d.s_a = r[0];

@@ -72,9 +72,10 @@ def test_removal_filters_long_lists(ora, dim, ipt):
     sim.close()
 
 
-# 255 to 257 blocks of 256 bubbles, and around 128 of them: the corrector forms
-# the foam's sums itself up to there
-@pytest.mark.parametrize("n", [65, 32767, 32768, 32769, 65279, 65536, 65537])
+# 255 to 257 blocks of 256 bubbles, around 128 and around 64 and 640 of them: the
+# corrector forms the sums by waves, by workgroups, or leaves them to a launch
+@pytest.mark.parametrize("n", [65, 16384, 16385, 32767, 32768, 32769, 65279, 65536, 65537,
+                               163840, 163841])
 def test_attempt_around_the_fused_sums(ora, n):
     print(f"fused sums n={n}", flush=True)
     sim = ca.Simulator(config(2, n, seed=70))
