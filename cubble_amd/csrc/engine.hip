@@ -477,8 +477,8 @@ Grid Engine::grid() const {
         g.search_threads =
             std::max(g.search_threads, std::min(kBlock, (r.h.stile + 63) / 64 * 64));
     }
-    g.quad = g.quad && nb_bub_ <= (CUBBLE_PREC_MIXED != precision ? kQuadBlocks
-                                   : all3 ? kQuadMixed3 : kQuadMixed2);
+    g.quad = g.quad && nb_bub_ <= (CUBBLE_PREC_MIXED == precision && all3 ? kQuadMixed3
+                                                                          : kQuadBlocks);
     return g;
 }
 

@@ -27,9 +27,11 @@ constexpr int kNumXcd = 8;          // MI355X: 8 XCDs, workgroups round-robin
 // 5.1 -> 7.3; at 782 (2D FP64) 6.4 -> 11.2, no gain any more.
 constexpr int kFuseBlocks = 640, kFuseBatch = 128;
 // Launches of at most this many blocks, one bubble a thread, take four lanes a
-// bubble in the pair kernel: FP64, mixed with 3D foams only, mixed with 2D ones
-// (a 2D list is half as long, and FP32 leaves less to overlap).
-constexpr int kQuadBlocks = 1024, kQuadMixed3 = 400, kQuadMixed2 = 128;
+// bubble in the pair kernel; mixed ones of 3D foams only up to the second, where
+// the longer lists give the wider kernel less to gain (200 steps, one lane /
+// four: 3D mixed 6e4 6.2 / 5.8 ms, 1e5 7.45 / 7.1, 1.3e5 7.5 / 7.7; 2D mixed 6e4
+// 5.9 / 5.1, 2e5 9.0 / 8.6; 128 foams of 2e3 24.4 / 23.1).
+constexpr int kQuadBlocks = 1024, kQuadMixed3 = 400;
 constexpr int kSearchParts = 64;    // records the search workgroups add their totals to
 constexpr int kPartD = 8;           // doubles per block partial record
 constexpr int kPartI = 4;           // ints per block partial record

@@ -45,11 +45,12 @@
 // difference.)
 //
 // A bubble that met such a pair is flagged (the sign of its stored overlap
-// sum) and its workgroup marked; a second kernel sums each flagged bubble
-// again with one wave, taking those pairs' d, |d|^2, R^2 - |d|^2 and both
-// branch decisions from the FP64 predictions, exactly as the FP64 path
-// evaluates them (rounded once to FP32 where the formula continues in FP32),
-// in parallel over the marked workgroups of every foam.
+// sum) and its workgroup marked; a second kernel (in small launches the
+// workgroup itself) sums each flagged bubble again with one wave, taking those
+// pairs' d, |d|^2, R^2 - |d|^2 and both branch decisions from the FP64
+// predictions, exactly as the FP64 path evaluates them (rounded once to FP32
+// where the formula continues in FP32), in parallel over the marked workgroups
+// of every foam.
 #include "dev_util.hpp"
 #include "launch.hpp"
 
@@ -301,6 +302,42 @@ __device__ __forceinline__ void mixed_block(const Consts &c, const Roles &R, con
     }
 }
 
+// Flagged bubble i (wave-uniform) summed again by the whole wave, the values
+// of the pairs that need them taken from the FP64 predictions: lane l takes
+// list entries l, l + 64, ..., and the lanes' sums are added in a fixed
+// butterfly order (every lane ends with the same sums, independent of
+// timing).  Lane 0 stores the terms; returns the overlap sum.
+template <int D, bool GAS, bool FLOW>
+__device__ __forceinline__ float exact_bubble_wave(const Consts &c, const Roles &R,
+                                                   const Scratch &S, size_t cap, double h,
+                                                   const float step[3], int i) {
+    const Q4 qi = load_rec(gmem(S.q4) + i);
+    const MixedPair<D, GAS, FLOW, true> pair(c, R, h, step, i, qi);
+    MixedOut o;
+    zero_out(o);
+    const int m_nn = S.nn[i];
+    for (int q = (int)(threadIdx.x & 63); q < m_nn; q += 64) {
+        const int j = gmem(S.nbr)[(size_t)q * cap + i];
+        const MixedTerm t = pair.template term<true>(j, load_rec(gmem(S.q4) + j));
+        if (pair.flows(j, t)) {
+#pragma unroll
+            for (int a = 0; a < D; ++a) o.fv[a] += field<float>(R.v[a])[j];
+        }
+        add_term<D, GAS>(t, o);
+    }
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        o.acc[a] = wave_sum_f(o.acc[a]);
+        if (FLOW) o.fv[a] = wave_sum_f(o.fv[a]);
+    }
+    if (GAS) {
+        o.ovl = wave_sum_f(o.ovl);
+        o.dr = wave_sum_f(o.dr);
+    }
+    if (0 == (threadIdx.x & 63)) store_mixed<D, GAS, FLOW>(c, R, S, h, i, o, false);
+    return o.ovl;
+}
+
 // Lane U's term, of each quad of lanes, but for its flags.
 template <int D, int U>
 __device__ __forceinline__ MixedTerm quad_term(const MixedTerm &t) {
@@ -319,24 +356,29 @@ __device__ __forceinline__ MixedTerm quad_term(const MixedTerm &t) {
 
 // Bubble i's pairs by four lanes, lane u of them taking list entries u, u + 4,
 // ..., two at a time; every lane adds all four's terms in list order, with the
-// roundings of mixed_block.  i >= n: nothing.
+// roundings of mixed_block.  Bubbles that met a pair that needs FP64 values are
+// then summed again by a wave each, as k_fix_mixed does.  i >= n: no bubble.  The
+// whole workgroup calls it.
 template <int D, bool GAS, bool FLOW>
 __device__ __forceinline__ void mixed_quad(const Consts &c, const Roles &R, const Scratch &S,
                                            size_t cap, int i, int n, double h, double &soa,
-                                           double &soar, bool &near_any) {
-    if (i >= n) return;
+                                           double &soar) {
+    __shared__ int s_cnt;
+    __shared__ int s_list[64];
+    __shared__ float s_ovl[64];
     const auto q4 = gmem(S.q4);
     const auto nbr = gmem(S.nbr);
     const int u = (int)(threadIdx.x & 3);
     float step[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) step[a] = fixed_step(c.interval[a], c.wall[a] != 0);
-    const Q4 qi = load_rec(q4 + i);
+    const bool valid = i < n;
+    const Q4 qi = load_rec(q4 + (valid ? i : 0));
     const MixedPair<D, GAS, FLOW, false> pair(c, R, h, step, i, qi);
     MixedOut o;
     zero_out(o);
     bool near = false;
-    const int m_nn = S.nn[i];
+    const int m_nn = valid ? S.nn[i] : 0;
     for (int q0 = 0; q0 < m_nn; q0 += 8) {
         int js[2];
         Q4 qs[2];
@@ -372,19 +414,42 @@ __device__ __forceinline__ void mixed_quad(const Consts &c, const Roles &R, cons
             }
         }
     }
-    // any of the four
     const unsigned long long mask = __builtin_amdgcn_ballot_w64(near);
-    near = (mask >> (threadIdx.x & 60) & 15ull) != 0ull;
-    if (0 == u) store_mixed<D, GAS, FLOW>(c, R, S, h, i, o, near);
-    near_any = near;
-    soa = (double)o.ovl;
-    soar = (double)o.ovl * (1.0 / (double)qi.r);
+    const bool flagged = 0 == u && (mask >> (threadIdx.x & 60) & 15ull) != 0ull;
+    if (valid && 0 == u) {
+        store_mixed<D, GAS, FLOW>(c, R, S, h, i, o, false);
+        soa = (double)o.ovl;
+        soar = (double)o.ovl * (1.0 / (double)qi.r);
+    }
+    if (!__syncthreads_or(flagged)) return;
+    if (0 == threadIdx.x) s_cnt = 0;
+    __syncthreads();
+    int slot = -1;
+    if (flagged) {
+        slot = atomicAdd(&s_cnt, 1);
+        s_list[slot] = i;
+    }
+    __syncthreads();
+    const int cnt = s_cnt;
+    for (int k = (int)(threadIdx.x >> 6); k < cnt; k += kWaves) {
+        const float ovl =
+            exact_bubble_wave<D, GAS, FLOW>(c, R, S, cap, h, step, uniform_i(s_list[k]));
+        if (0 == (threadIdx.x & 63)) s_ovl[k] = ovl;
+    }
+    __syncthreads();
+    if (slot >= 0) {
+        soa = (double)s_ovl[slot];
+        soar = (double)s_ovl[slot] * (1.0 / (double)qi.r);
+    }
 }
 
 // The pair kernel of small launches, as k_pair_quad.  us a launch, k_pair_mixed
-// / this: 3D 1e3 7.8 / 4.7, 3e4 8.6 / 5.4, 6e4 8.9 / 7.2, 1e5 9.3 / 9.2 when just
-// seeded (and after 2000 steps, when some lists are long, 18.6 -> 17.1 ms a run
-// of 300 steps), 2e5 11.8 / 13.9; 2D 3e4 5.1 / 4.2, 6e4 5.2 / 5.1, 1e5 5.7 / 6.2.
+// / this without the FP64 pass: 3D 1e3 7.8 / 4.7, 3e4 8.6 / 5.4, 6e4 8.9 / 7.2,
+// 1e5 9.3 / 9.2 when just seeded (and after 2000 steps, when some lists are long,
+// 18.6 -> 17.1 ms a run of 300 steps), 2e5 11.8 / 13.9; 2D 3e4 5.1 / 4.2, 1e5 5.7 /
+// 6.2.  The bubbles that need FP64 values are few, and their workgroup sums them
+// again at once (in 2D 1.3 us, where most workgroups have one): k_fix_mixed's
+// launch took 2.5 to 4.
 template <bool FLOW>
 __global__ __launch_bounds__(kBlock) void k_pair_mixed_quad(Foam *foams, const int2 *bt,
                                                             uint32_t flags) {
@@ -401,56 +466,15 @@ __global__ __launch_bounds__(kBlock) void k_pair_mixed_quad(Foam *foams, const i
     const size_t cap = (size_t)F->cap;
     const int i = part * 64 + (int)(threadIdx.x >> 2);
     double soa = 0.0, soar = 0.0;
-    bool near = false;
     const bool gas = (flags & kGas) != 0;
     if (3 == c.dim) {
-        if (gas) mixed_quad<3, true, FLOW>(c, R, S, cap, i, n, h, soa, soar, near);
-        else mixed_quad<3, false, FLOW>(c, R, S, cap, i, n, h, soa, soar, near);
+        if (gas) mixed_quad<3, true, FLOW>(c, R, S, cap, i, n, h, soa, soar);
+        else mixed_quad<3, false, FLOW>(c, R, S, cap, i, n, h, soa, soar);
     } else {
-        if (gas) mixed_quad<2, true, FLOW>(c, R, S, cap, i, n, h, soa, soar, near);
-        else mixed_quad<2, false, FLOW>(c, R, S, cap, i, n, h, soa, soar, near);
+        if (gas) mixed_quad<2, true, FLOW>(c, R, S, cap, i, n, h, soa, soar);
+        else mixed_quad<2, false, FLOW>(c, R, S, cap, i, n, h, soa, soar);
     }
     quad_store(S, part, soa, soar);
-    // the block's mark, a byte of it for each 64 bubbles
-    const bool any = __syncthreads_or(near) != 0;
-    if (0 == threadIdx.x)
-        reinterpret_cast<uint8_t *>(S.part_i + (part >> 2) * kPartI + 2)[part & 3] = any ? 1 : 0;
-}
-
-// Flagged bubble i (wave-uniform) summed again by the whole wave, the values
-// of the pairs that need them taken from the FP64 predictions: lane l takes
-// list entries l, l + 64, ..., and the lanes' sums are added in a fixed
-// butterfly order (every lane ends with the same sums, independent of
-// timing).  Lane 0 stores the terms; returns the overlap sum.
-template <int D, bool GAS, bool FLOW>
-__device__ __forceinline__ float exact_bubble_wave(const Consts &c, const Roles &R,
-                                                   const Scratch &S, size_t cap, double h,
-                                                   const float step[3], int i) {
-    const Q4 qi = load_rec(gmem(S.q4) + i);
-    const MixedPair<D, GAS, FLOW, true> pair(c, R, h, step, i, qi);
-    MixedOut o;
-    zero_out(o);
-    const int m_nn = S.nn[i];
-    for (int q = (int)(threadIdx.x & 63); q < m_nn; q += 64) {
-        const int j = gmem(S.nbr)[(size_t)q * cap + i];
-        const MixedTerm t = pair.template term<true>(j, load_rec(gmem(S.q4) + j));
-        if (pair.flows(j, t)) {
-#pragma unroll
-            for (int a = 0; a < D; ++a) o.fv[a] += field<float>(R.v[a])[j];
-        }
-        add_term<D, GAS>(t, o);
-    }
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        o.acc[a] = wave_sum_f(o.acc[a]);
-        if (FLOW) o.fv[a] = wave_sum_f(o.fv[a]);
-    }
-    if (GAS) {
-        o.ovl = wave_sum_f(o.ovl);
-        o.dr = wave_sum_f(o.dr);
-    }
-    if (0 == (threadIdx.x & 63)) store_mixed<D, GAS, FLOW>(c, R, S, h, i, o, false);
-    return o.ovl;
 }
 
 // The flagged bubbles of block lb, one wave per flagged bubble, and the
@@ -570,17 +594,6 @@ __global__ __launch_bounds__(kBlock) void k_fix_mixed(Foam *foams, const int2 *b
     double soa = 0.0, soar = 0.0;
     bool near = false;
     mixed_block_dispatch<FLOW, true>(F, cx.lb, flags, soa, soar, near);
-    if (flags & kQuad) {
-        // (one bubble a thread)
-        soa = wave_sum(soa);
-        soar = wave_sum(soar);
-        if (0 == (threadIdx.x & 63)) {
-            double *const p = quad_parts(F->s) + 8 * (size_t)cx.lb + 2 * (threadIdx.x >> 6);
-            p[0] = soa;
-            p[1] = soar;
-        }
-        return;
-    }
     double sums[2] = {soa, soar};
     int none = 0;
     block_reduce_t0(sums, 0u, none);
@@ -592,7 +605,7 @@ __global__ __launch_bounds__(kBlock) void k_fix_mixed(Foam *foams, const int2 *b
 
 void launch_pair_mixed(const Grid &g, uint32_t flags, bool fix) {
     const dim3 grid(g.nb_bub), quad(4 * g.nb_bub), block(kBlock);
-    if (g.quad) flags |= kQuad;
+    fix = fix && !g.quad;  // k_pair_mixed_quad does it itself
     if (flags & kFlow) {
         if (g.quad)
             hipLaunchKernelGGL(k_pair_mixed_quad<true>, quad, block, 0, g.stream, g.foams,
