@@ -214,12 +214,13 @@ int time_search(Engine &e, int reps, cubble_search_times *out) {
     }
     if (!rc) rc = timed([&] { launch_search_part(g, kPartListKernel); }, kernel_ms);
     if (!rc) rc = timed([&] { launch_search_part(g, kPartReorder); }, reorder_ms);
-    // an attempt's removal launch and its share of a search phase when no foam
-    // needs them
+    // an attempt's share of the removal and search launches of a captured run
+    // when no foam needs them
     if (!rc) {
         launch_set_flags(g, 0, 0, 1);
+        const int applies = g.nb_bub <= kApplyBlocks ? 1 : kSearchEvery;
         rc = timed([&] {
-            for (int k = 0; k < kSearchEvery; ++k) launch_apply(g);
+            for (int k = 0; k < applies; ++k) launch_apply(g);
             launch_search(g);
         }, idle_ms);
         idle_ms /= kSearchEvery;

@@ -587,8 +587,8 @@ __device__ __forceinline__ void tile_masks(const Tile &t, const double o[3], con
 // instruction issue (VALU 69%, SALU 62% of the cycles).  List kernel, same
 // foams: 3D 1e6 0.49 -> 0.24 ms, 3D 1e5 (mixed, 45 bubbles a cell) 0.20 ->
 // 0.094 ms, batch of 256 foams 2.09 -> 1.23 ms, 2D 1e4 17 -> 11 us.  Its
-// bound now is latency at four waves per SIMD (a wave waits in two thirds of
-// its cycles); five, with 25 registers spilled, are 15% slower.
+// bound now is VALU issue (64% of the cycles) at four waves per SIMD, of which
+// each waits 41% of its cycles; five, with 25 registers spilled, are 15% slower.
 template <int D>
 __device__ __forceinline__ void search_span(const Foam *F, const Consts &c, const Scratch &S,
                                             const int cd[3], size_t cap, int nbr_cap, double rmax,

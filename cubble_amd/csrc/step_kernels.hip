@@ -1,19 +1,24 @@
-// step_kernels.hip -- the three kernels of one step() attempt.
+// step_kernels.hip -- the kernels of one step() attempt.
 //
-//   k_predict : AB2 predictor + block partials of S_A, S_Ar; writes the
-//               32-byte FP64 neighbour record, or in mixed precision the
-//               16-byte fixed-point one (reference preIntegrate,
+//   k_predict : (in a captured run the removal of the attempt before;) AB2
+//               predictor + block partials of S_A, S_Ar; writes the 32-byte
+//               FP64 neighbour record, or in mixed precision the 16-byte
+//               fixed-point one (reference preIntegrate,
 //               src/kernels.cu:40-170)
-//   k_pair    : pairwise Durian velocity, overlap area and gas flux, gathered
-//               per bubble over its full neighbour list; the last block
-//               reduces S_A, S_Ar, S_OA, S_OAr
+//   k_pair, k_pair_quad : pairwise Durian velocity, overlap area and gas flux,
+//               gathered per bubble over its full neighbour list, by one lane
+//               or (small launches) four; partials of S_OA, S_OAr
 //               (reference pairwiseInteraction, src/kernels.cu:172-337)
+//   k_sums    : S_A, S_Ar, S_OA, S_OAr of foams whose corrector does not form
+//               them itself
 //   k_correct : walls, liquid-mediated gas exchange, trapezoid corrector,
-//               error / expansion / radius / volume reductions, deletion
-//               marks, path; the last block runs the dt controller and, when
-//               committing, rotates the role pointers
-//               (reference postIntegrate, src/kernels.cu:339-495, :546-593,
-//                and step()/integrate(), src/simulator.cu:192-314)
+//               error / expansion / radius / volume partials, deletion marks,
+//               path (reference postIntegrate, src/kernels.cu:339-495,
+//               :546-593)
+//   k_control : one workgroup per foam: the corrector's partials, the dt
+//               controller and, when committing, the rotation of the role
+//               pointers and the plan of a removal (reference
+//               step()/integrate(), src/simulator.cu:192-314)
 //
 // The reference scatters every pair into both bubbles with FP64 atomics in
 // unspecified order.  Here each bubble gathers its own neighbours in

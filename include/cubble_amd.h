@@ -444,8 +444,9 @@ int64_t cubble_foam_footprint(const cubble_config *cfg);
 
 /* Average device time of each kernel of one attempt from the current state,
  * measured with HIP events on the handle's stream around `reps` back-to-back
- * launches of each (predictor; pair kernel; sums + corrector + controller,
- * not committing).  No counterpart in the reference (it has NVTX ranges
+ * launches of each (predictor; pair kernel, in mixed precision without the
+ * second pass that larger launches make over its FP64 pairs; corrector, not
+ * committing).  No counterpart in the reference (it has NVTX ranges
  * only, src/simulator.cu:40-363); used by the benchmark's roofline report. */
 typedef struct cubble_kernel_times {
     double predict_ms;
@@ -463,9 +464,9 @@ int cubble_batch_time_kernels(cubble_batch *b, const cubble_integrate_params *ip
  * average of `reps` back-to-back launches between one pair of HIP events:
  * a whole search of every foam; the list build alone (lists of the
  * reference's neighborSearch / sortPairs, src/kernels.cu:617-719); the list
- * kernel alone; the reorder (reorganizeByIndex, :721-770); and one attempt
- * group's removal and search kernels when no foam needs them (they return
- * at once).  No counterpart in the reference (it has NVTX ranges only). */
+ * kernel alone; the reorder (reorganizeByIndex, :721-770); and an attempt's
+ * share of the removal and search kernels when no foam needs them (they
+ * return at once).  No counterpart in the reference (it has NVTX ranges only). */
 typedef struct cubble_search_times {
     double search_ms;
     double lists_ms;
