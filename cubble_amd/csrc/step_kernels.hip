@@ -638,7 +638,10 @@ __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, c
             }
             stream_store(R.path_new + i, path + sqrt(pd));
         }
-        stream_store(field<V>(R.err) + i, (V)fmax(e, err));
+        // the largest error so far: most bubbles' stands, and a store less is
+        // 1% of the large runs (256 foams 31.54 -> 31.22 ms, 3D 1e6 20.25 -> 20.05);
+        // negated, so that a NaN is replaced as fmax does
+        if (!(e <= err)) stream_store(field<V>(R.err) + i, (V)fmax(e, err));
         a.max_err = fmax(a.max_err, e);
     }
 }
