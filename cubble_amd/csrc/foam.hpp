@@ -144,6 +144,7 @@ struct Dyn {
     // stop rules checked after every accepted step (0 = off)
     double r_stop;       // halt once the step's largest radius >= r_stop
     int32_t time_stop;   // halt once time_int + time_frac >= stop_int + stop_frac
+    int32_t marked;      // the deletion marks are the last attempt's and not yet carried out
     uint64_t stop_int;
     double stop_frac;
     // extremes and sum of the accepted steps' dt since the last window reset

@@ -48,8 +48,9 @@ void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control = tr
 // search phase clears it.  With kApply an attempt's predictor carries out the
 // removal of the attempt before, unless the foam stands still.
 void launch_apply(const Grid &g);
-// removeBubbles by itself: the plan (sorted deletion list, moves), then the
-// above.  The caller clears the flag.
+// removeBubbles by itself: the marks counted, the plan (sorted deletion list,
+// moves), then the above.  The caller sets the flag, where the marks still
+// stand (Dyn::marked), and clears it.
 void launch_remove(const Grid &g);
 
 // searchNeighbors: wrap + cell ids + counts, two-pass scan, binning,

@@ -27,6 +27,23 @@
 
 namespace cubble_amd {
 
+// The deletion marks in each block, for a removal asked for by itself: the
+// corrector's counts are of the launch shape and the count it ran with, and
+// the planner indexes with what the marks it finds give.
+__global__ __launch_bounds__(kBlock) void k_rm_count(Foam *foams, const int2 *bt) {
+    const Ctx cx = bubble_ctx(foams, bt);
+    Foam *F = cx.F;
+    if (!F->d.need_remove) return;
+    const int n = F->d.count, ipt = F->ipt;
+    int c = 0;
+    for (int k = 0; k < ipt; ++k) {
+        const int i = (cx.lb * ipt + k) * kBlock + (int)threadIdx.x;
+        c += i < n && F->s.del[i] ? 1 : 0;
+    }
+    c = block_sum_i(c);
+    if (0 == threadIdx.x) F->s.part_i[cx.lb * kPartI] = c;
+}
+
 // A removal asked for by itself (cubble_remove_bubbles); k_control plans its
 // own.
 __global__ __launch_bounds__(kBlock) void k_rm_plan(Foam *foams) {
@@ -35,12 +52,14 @@ __global__ __launch_bounds__(kBlock) void k_rm_plan(Foam *foams) {
     __shared__ DeletedBlocks s_blocks;
     if (0 == threadIdx.x) s_blocks.m = 0;
     __syncthreads();
+    int nd = 0;
     for (int b = threadIdx.x; b < F->nblk; b += kBlock) {
         const int c = F->s.part_i[b * kPartI];
         if (c > 0) s_blocks.add(b, c);
+        nd += c;
     }
-    __syncthreads();
-    plan_removal(F, s_blocks, F->d.count, F->d.n_del);
+    nd = block_sum_i(nd);  // (and every thread's blocks are in the list)
+    plan_removal(F, s_blocks, F->d.count, nd);
 }
 
 // Removals of the last attempt before a search phase, and of foams that stand
@@ -55,6 +74,7 @@ void launch_apply(const Grid &g) {
 }
 
 void launch_remove(const Grid &g) {
+    hipLaunchKernelGGL(k_rm_count, dim3(g.nb_bub), dim3(kBlock), 0, g.stream, g.foams, g.bt_bub);
     hipLaunchKernelGGL(k_rm_plan, dim3(g.nfoams), dim3(kBlock), 0, g.stream, g.foams);
     launch_apply(g);
 }

@@ -104,6 +104,7 @@ __device__ __forceinline__ void commit_removal(Foam *F, double s_v, int h, int n
     d.n_holes = h;
     d.count = nnew;
     d.removals += 1;
+    d.marked = 0;
     d.num_pairs -= pairs;
     if (d.count_stop > 0 && nnew <= d.count_stop) d.halt = 1;
 }

@@ -391,6 +391,10 @@ int cubble_search_neighbors(cubble_sim *s) {
 int cubble_remove_bubbles(cubble_sim *s) {
     if (!s) return CUBBLE_E_INVALID;
     Engine &e = s->e;
+    Foam h;
+    const int rc = e.read_header(0, h);
+    if (rc) return rc;
+    if (!h.d.marked) return CUBBLE_OK;  // carried out already, or no attempt
     const Grid g = e.grid();
     launch_set_flags(g, -1, 1, 0);
     launch_remove(g);

@@ -272,6 +272,7 @@ int set_state(Engine &e, int k, const cubble_state_view *v, const cubble_scalars
     for (int q = 0; q < 3; ++q) d.cell_dim[q] = sc->cell_dim[q];
     d.need_search = 0;
     d.need_remove = 0;
+    if (n != f.d.count) d.marked = 0;  // marks of other bubbles
     d.halt = 0;
     d.overflow = 0;
     d.step_limit = 0;

@@ -669,6 +669,7 @@ __device__ __forceinline__ bool control(Foam *F, const Dyn &was, const Roles &R,
     d.max_r = a.max_r;
     d.max_exp = a.max_exp;
     d.n_del = a.n_del;
+    d.marked = 1;
     d.attempts = was.attempts + 1;
     d.dt = ndt;
     d.accepted = too_large ? 0 : 1;

@@ -229,7 +229,9 @@ int cubble_run_steps(cubble_sim *sim, const cubble_integrate_params *ip, int64_t
 int cubble_search_neighbors(cubble_sim *sim);
 
 /* removeBubbles() (src/simulator.cu:180-190) using the deletion marks of the
- * last attempt. */
+ * last attempt.  Nothing happens when there are none to use: no attempt yet,
+ * its removal carried out already (by integrate, run_steps or a call before
+ * this one), or a state of another count set since. */
 int cubble_remove_bubbles(cubble_sim *sim);
 
 /* ---- observables, stop rules and the print window ------------------------ */
