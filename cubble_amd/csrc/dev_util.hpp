@@ -158,6 +158,13 @@ __device__ __forceinline__ float wave_sum_f(float v) {
     return wave_all(v, [](float a, float b) { return a + b; });
 }
 
+// Memory written by the wave's lanes before it is read by them after it.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 constexpr int kWaves = kBlock / 64;
 
 __device__ __forceinline__ double block_sum(double v) {

@@ -44,7 +44,7 @@ __device__ __forceinline__ void move_state(const Foam *F, int i, int src, double
 // Bubble i's list from src's, by one wave: deleted neighbours dropped, moved
 // ones mapped to their new slots, ascending.  Up to 64 entries one lane each
 // (their marks and new slots are then one load each, and an entry's place is
-// the number of smaller ones); longer lists entry by entry.
+// the number of smaller ones); longer lists 64 entries at a time.
 __device__ __forceinline__ void filter_list(const Scratch &S, size_t cap, int nnew, int i,
                                             int src) {
     const int lane = (int)(threadIdx.x & 63);
@@ -65,29 +65,59 @@ __device__ __forceinline__ void filter_list(const Scratch &S, size_t cap, int nn
         if (0 == lane) S.nn[i] = __popcll(kept);
         return;
     }
-    if (lane) return;
-    // writes stay at positions <= the entries consumed, so this also runs in
-    // place (src == i)
-    int out = 0, last = -1;  // largest entry written so far
-    for (int q = 0; q < m; ++q) {
-        const int j = S.nbr[(size_t)q * cap + src];
-        if (S.del[j]) continue;
-        const int jj = j >= nnew ? S.moved_to[j - nnew] : j;
-        int pos = out;
-        if (jj < last) {  // a moved bubble's new index: insertion keeps the order
-            while (pos > 0) {
-                const int prev = S.nbr[(size_t)(pos - 1) * cap + i];
-                if (prev <= jj) break;
-                S.nbr[(size_t)pos * cap + i] = prev;
-                --pos;
-            }
-        } else {
-            last = jj;
+    // Entries below the new count keep their order; writes stay at positions <=
+    // those read, so this also runs in place (src == i).
+    constexpr int kNone = 0x7fffffff;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    auto at = [&](int q, int of) -> int & { return S.nbr[(size_t)q * cap + of]; };
+    int out = 0, first = m;  // the moved ones, with the largest indices, come last
+    for (int q = 0; q < m; q += 64) {
+        const int j = q + lane < m ? at(q + lane, src) : kNone;
+        const bool keep = j < nnew && !S.del[j];
+        const unsigned long long kept = __builtin_amdgcn_ballot_w64(keep);
+        if (keep) at(out + __popcll(kept & below), i) = j;
+        out += __popcll(kept);
+        const unsigned long long low = __builtin_amdgcn_ballot_w64(j < nnew);
+        if (~low) {
+            first = q + __popcll(low);
+            break;
         }
-        S.nbr[(size_t)pos * cap + i] = jj;
-        ++out;
     }
-    S.nn[i] = out;
+    // 64 moved ones merged into the list at a time, from its back: an entry goes
+    // up by as many as are smaller than it
+    for (int q = first; q < m; q += 64) {
+        const int j = q + lane < m ? at(q + lane, src) : -1;
+        const bool keep = j >= 0 && !S.del[j];
+        const int e = keep ? S.moved_to[j - nnew] : kNone;
+        const unsigned long long kept = __builtin_amdgcn_ballot_w64(keep);
+        if (!kept) continue;
+        int pos = 0;  // of e: the smaller moved ones and list entries
+        for (unsigned long long t = kept; t; t &= t - 1ull)
+            pos += __builtin_amdgcn_readlane(e, __builtin_ctzll(t)) < e ? 1 : 0;
+        for (int top = out; top > 0; top -= 64) {
+            const int k = top - 64 + lane;
+            wave_sync();  // entries that other lanes wrote
+            const int v = k >= 0 ? at(k, i) : kNone;
+            int up = 0;
+            for (unsigned long long t = kept; t; t &= t - 1ull) {
+                const int l = __builtin_ctzll(t), n = __builtin_amdgcn_readlane(e, l);
+                const int smaller = __popcll(__builtin_amdgcn_ballot_w64(v < n));
+                up += k >= 0 && n < v ? 1 : 0;
+                if (lane == l) pos += smaller;
+            }
+            wave_sync();
+            if (up > 0) at(k + up, i) = v;
+            // the rest is smaller than all of them once its last one is
+            if (0 == __builtin_amdgcn_readlane(up, max(64 - top, 0))) {
+                pos += max(top - 64, 0);
+                break;
+            }
+        }
+        wave_sync();
+        if (keep) at(pos, i) = e;
+        out += __popcll(kept);
+    }
+    if (0 == lane) S.nn[i] = out;
 }
 
 // Bubble i's own list of at most 16 entries, filtered by 16 lanes (g: which of
@@ -149,7 +179,16 @@ __device__ __forceinline__ void apply_removal(const Foam *F, int lb) {
         for (int e = kWaves - 1 - wave; e < holes; e += kWaves) {
             const int b = uniform_i(s_list[kBlock - 1 - e]);
             int src = b;  // the k-th entry of the deletion list is the k-th hole
-            for (int k0 = 0; k0 < h; k0 += 64) {
+            int k0 = 0;
+            for (int len = h; len > 256;) {  // (ascending: 64 steps at once)
+                const int step = (len + 63) >> 6;
+                const int at = k0 + lane * step;
+                const bool reached = lane * step < len && S.del_list[at] <= b;
+                const int c = __popcll(__builtin_amdgcn_ballot_w64(reached)) - 1;
+                len = min(step, len - c * step);
+                k0 += c * step;
+            }
+            for (; k0 < h; k0 += 64) {
                 const bool in = k0 + lane < h;
                 const int d = in ? S.del_list[k0 + lane] : -1;
                 const int s = in ? S.plan_src[k0 + lane] : -1;

@@ -62,12 +62,6 @@ struct Piece {
     int n_code;  // n | code << 8
 };
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // A wave-uniform value of vector arithmetic, into scalar registers.
 __device__ __forceinline__ double uniform_d(double v) { return readlane_d(v, 0); }
 __device__ __forceinline__ float uniform_f(float v) {
