@@ -465,7 +465,7 @@ Grid Engine::grid() const {
     g.nb_scell = nb_scell_;
     g.nfoams = (int)foams.size();
     g.stream = stream;
-    g.walls = g.big = false;
+    g.walls = g.big = g.plans = false;
     g.search_threads = 64;
     g.quad = true;
     bool all3 = true;
@@ -474,6 +474,7 @@ Grid Engine::grid() const {
         all3 = all3 && 3 == r.h.c.dim;
         g.quad = g.quad && 1 == r.h.ipt;
         g.big = g.big || r.h.nblk > (one ? kFuseBlocks : kFuseBatch);
+        g.plans = g.plans || r.h.nblk > kControlPlans;
         g.search_threads =
             std::max(g.search_threads, std::min(kBlock, (r.h.stile + 63) / 64 * 64));
     }
@@ -499,6 +500,7 @@ void Engine::enqueue_groups(uint32_t flags, int groups) {
     for (int k = 1; k <= groups; ++k) {
         enqueue_attempt(in_predict ? flags | kApply : flags);
         const bool phase = 0 == k % kSearchEvery || groups == k;
+        if (phase && g.plans) launch_plan(g);
         if (phase || !in_predict) launch_apply(g);
         if (phase) launch_search(g);
     }
@@ -509,7 +511,7 @@ int Engine::capture(uint32_t flags, int groups) {
     // (walls or not, a sums launch or not)
     const Grid g = grid();
     if (graph_ && graph_flags_ == flags && graph_groups_ == groups && graph_walls_ == g.walls &&
-        graph_big_ == g.big && graph_quad_ == g.quad && graph_threads_ == g.search_threads)
+        graph_big_ == g.big && graph_plans_ == g.plans && graph_quad_ == g.quad && graph_threads_ == g.search_threads)
         return CUBBLE_OK;
     if (graph_) {
         (void)hipGraphExecDestroy(graph_);
@@ -529,6 +531,7 @@ int Engine::capture(uint32_t flags, int groups) {
     graph_groups_ = groups;
     graph_walls_ = g.walls;
     graph_big_ = g.big;
+    graph_plans_ = g.plans;
     graph_quad_ = g.quad;
     graph_threads_ = g.search_threads;
     return CUBBLE_OK;
@@ -742,13 +745,19 @@ int Engine::integrate(uint32_t flags, std::vector<Dyn> &d) {
     if (rc) return rc;
     for (int tries = 0; tries < 100000; ++tries) {
         enqueue_attempt(flags, pinned_);
-        launch_apply(grid());
         if ((rc = read_mirror(d))) return rc;
-        // the search's launches only when some foam needs them
-        bool search = false;
-        for (const Dyn &x : d) search = search || x.need_search;
-        if (search) {
-            launch_search(grid());
+        // the launches of removals and of the search only when some foam needs
+        // them
+        bool plan = false, apply = false, search = false;
+        for (const Dyn &x : d) {
+            plan = plan || kMarked == x.need_remove;
+            apply = apply || x.need_remove;
+            search = search || x.need_search;
+        }
+        if (plan) launch_plan(grid());
+        if (apply) launch_apply(grid());
+        if (search) launch_search(grid());
+        if (apply || search) {
             E_TRY(hipGetLastError());
             if ((rc = read_dyn_all(d))) return rc;
         }

@@ -200,7 +200,7 @@ class Engine {
     hipGraphExec_t graph_ = nullptr;
     uint32_t graph_flags_ = 0;
     int graph_groups_ = 0;
-    bool graph_walls_ = false, graph_big_ = false, graph_quad_ = false;
+    bool graph_walls_ = false, graph_big_ = false, graph_quad_ = false, graph_plans_ = false;
     int graph_threads_ = 0;
     mutable bool clean_ = false;  // no foam is halted or has a step limit
     bool opened_ = false;  // counted among the users of the pinned blocks

@@ -32,6 +32,10 @@ constexpr int kFuseBlocks = 640, kFuseBatch = 128;
 // four: 3D mixed 6e4 6.2 / 5.8 ms, 1e5 7.45 / 7.1, 1.3e5 7.5 / 7.7; 2D mixed 6e4
 // 5.9 / 5.1, 2e5 9.0 / 8.6; 128 foams of 2e3 24.4 / 23.1).
 constexpr int kQuadBlocks = 1024, kQuadMixed3 = 400;
+// Foams of more than this many blocks have a removal of more than kBlock bubbles
+// planned by launches before the search phase instead of by k_control (see
+// remove_plan.hpp).
+constexpr int kControlPlans = 256;
 constexpr int kSearchParts = 64;    // records the search workgroups add their totals to
 constexpr int kPartD = 8;           // doubles per block partial record
 constexpr int kPartI = 4;           // ints per block partial record
@@ -120,7 +124,7 @@ struct Dyn {
     int32_t num_cells;
     int32_t accepted;
     int32_t need_search;
-    int32_t need_remove;
+    int32_t need_remove; // 0, or one of the values below
     int32_t halt;        // device loop stop (limit reached or capacity error)
     int32_t overflow;    // neighbour list capacity exceeded
     int32_t n_del;
@@ -151,6 +155,10 @@ struct Dyn {
     double ts_min, ts_max, ts_sum;
 };
 
+// need_remove: the removal is planned, and apply_removal carries it out; or the
+// bubbles are marked only, and the foam stands still until launch_plan.
+constexpr int kPlanned = 1, kMarked = 2;
+
 // Empty time-step window (reference src/simulator.cu:980-982).
 constexpr double kTsMinEmpty = 9999999.9;
 constexpr double kTsMaxEmpty = -1.0;
@@ -164,9 +172,11 @@ __host__ __device__ inline bool stop_reached(const Dyn &d) {
            (d.time_int > d.stop_int || (d.time_int == d.stop_int && d.time_frac >= d.stop_frac));
 }
 
-// A foam that stands still in an attempt: halted, or waiting for its search
-// (a graph holds one search for several attempts).
-__host__ __device__ inline bool standing(const Dyn &d) { return (d.halt | d.need_search) != 0; }
+// A foam that stands still in an attempt: halted, or waiting for its search or
+// the plan of a large removal (a graph holds one of each for several attempts).
+__host__ __device__ inline bool standing(const Dyn &d) {
+    return (d.halt | d.need_search | (d.need_remove & kMarked)) != 0;
+}
 
 struct Foam {
     Consts c;

@@ -24,6 +24,7 @@ struct Grid {
     bool walls;  // some foam of the launch has a wall
     bool quad;   // the FP64 pair kernel is k_pair_quad: one bubble a thread, few blocks
     bool big;    // some foam of the launch has more blocks than k_correct sums itself
+    bool plans;  // some foam of the launch leaves large removals to launch_plan
 };
 
 void launch_predict(const Grid &g, uint32_t flags);
@@ -42,15 +43,17 @@ void launch_sums(const Grid &g);
 void launch_correct(const Grid &g, uint32_t flags, bool mixed, bool control = true,
                     Dyn *mirror = nullptr);
 
-// The planned removals: move the tail survivors into the holes, filter /
-// remap the neighbour lists and apply the volume fix.  Runs only for foams
-// whose need_remove flag is set; the next controller or the end of the next
-// search phase clears it.  With kApply an attempt's predictor carries out the
-// removal of the attempt before, unless the foam stands still.
+// The planned removals (need_remove kPlanned): move the tail survivors into the
+// holes, filter / remap the neighbour lists and apply the volume fix.  The next
+// controller or the end of the next search phase clears the flag.  With kApply
+// an attempt's predictor carries out the removal of the attempt before, unless
+// the foam stands still.
 void launch_apply(const Grid &g);
-// removeBubbles by itself: the marks counted, the plan (sorted deletion list,
-// moves), then the above.  The caller sets the flag, where the marks still
-// stand (Dyn::marked), and clears it.
+// Plans the removals that are only marked (kMarked), for launch_apply.
+void launch_plan(const Grid &g);
+// removeBubbles by itself: the marks counted, planned and carried out.  The
+// caller sets the flag (kMarked), where the marks still stand (Dyn::marked),
+// and clears it.
 void launch_remove(const Grid &g);
 
 // searchNeighbors: wrap + cell ids + counts, two-pass scan, binning,

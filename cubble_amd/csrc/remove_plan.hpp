@@ -1,7 +1,7 @@
 // remove_plan.hpp -- planning a removal, by one workgroup of the foam: the
 // sorted deletion list, the moves of the tail survivors into the holes, the
 // marks on the neighbour lists that change, the new count and pair count, and
-// the volume-fix multiplier (reference src/kernels.cu:775-867).  k_rm_apply
+// the volume-fix multiplier (reference src/kernels.cu:775-867).  apply_removal
 // then does the work on every slot.
 //
 // A removal touches few bubbles (one to a few dozen of 1e5 .. 1e7), so its
@@ -10,16 +10,21 @@
 // whether or not a foam had a removal (1e5 foam, mixed: 15 us per attempt group
 // with one).  Up to kBlock deletions, plan_few keeps the lists in LDS and loads
 // ahead what does not depend on them; more take plan_many.
+//
+// Thousands of deletions in one step (bubbles set below the smallest radius,
+// coarsening of a large foam at a large time step) are work, which one
+// workgroup takes too long for; foams of more than kControlPlans blocks leave
+// them to the launches of remove_kernels.hip.
 #pragma once
 
 #include "dev_util.hpp"
 
 namespace cubble_amd {
 
-// Blocks holding deletions that the planner sorts in LDS; a removal spread
-// over more blocks (thousands of bubbles in one step) takes the block by block
-// walk.
-constexpr int kPlanBlocks = 1024;
+// Most blocks with deletions in a removal planned here: foams of that many
+// blocks, or removals of at most kBlock bubbles.
+constexpr int kPlanBlocks = kControlPlans;
+static_assert(kPlanBlocks >= kBlock, "a deletion per block");
 
 // The blocks with deletions, as k_control comes to their counts.
 struct DeletedBlocks {
@@ -79,22 +84,6 @@ __device__ __forceinline__ void emit_blocks(const Scratch &S, const DeletedBlock
     }
 }
 
-// The same for deletions in more blocks than kPlanBlocks, block by block.
-__device__ __forceinline__ void emit_deleted(const Scratch &S, int n, int ipt, int nblk) {
-    int off = 0;
-    for (int b = 0; b < nblk; ++b) {
-        if (0 == S.part_i[b * kPartI + 0]) continue;  // uniform
-        for (int k = 0; k < ipt; ++k) {
-            const int i = (b * ipt + k) * kBlock + (int)threadIdx.x;
-            const int f = i < n && S.del[i] ? 1 : 0;
-            int tot = 0;
-            const int pre = block_excl_scan(f, tot);
-            if (f) S.del_list[off + pre] = i;
-            off += tot;
-        }
-    }
-}
-
 // What a planned removal changes in the foam's header; one thread.
 __device__ __forceinline__ void commit_removal(Foam *F, double s_v, int h, int nnew, int pairs) {
     Dyn &d = F->d;
@@ -109,18 +98,11 @@ __device__ __forceinline__ void commit_removal(Foam *F, double s_v, int h, int n
     if (d.count_stop > 0 && nnew <= d.count_stop) d.halt = 1;
 }
 
-// Plans the removal of the `nd` marked bubbles of the foam's n, which are in
-// the blocks B, and commits the counters.  The whole workgroup (kBlock threads)
-// calls it.
-__device__ __forceinline__ void plan_many(Foam *F, const DeletedBlocks &B, int n, int nd) {
-    const Scratch S = F->s;
+// The moves, from the deletion list of `nd` bubbles of n: the k-th hole below
+// the new count receives the k-th surviving bubble counted from the back.
+// Returns the number of holes.  By the whole workgroup; ends without a barrier.
+__device__ __forceinline__ int plan_moves(const Scratch &S, int n, int nd) {
     const int nnew = n - nd;
-    const size_t cap = (size_t)F->cap;
-    if (B.m <= kPlanBlocks) emit_blocks(S, B, n, F->ipt, nullptr);
-    else emit_deleted(S, n, F->ipt, F->nblk);
-    __syncthreads();
-    // the k-th hole below the new count receives the k-th surviving bubble
-    // counted from the back
     int below = 0;
     for (int k = threadIdx.x; k < nd; k += kBlock) below += S.del_list[k] < nnew ? 1 : 0;
     const int h = block_sum_i(below);
@@ -136,6 +118,19 @@ __device__ __forceinline__ void plan_many(Foam *F, const DeletedBlocks &B, int n
         }
         got += tot;
     }
+    return h;
+}
+
+// Plans the removal of the `nd` marked bubbles of the foam's n, which are in
+// the blocks B, and commits the counters.  The whole workgroup (kBlock threads)
+// calls it.
+__device__ __forceinline__ void plan_many(Foam *F, const DeletedBlocks &B, int n, int nd) {
+    const Scratch S = F->s;
+    const int nnew = n - nd;
+    const size_t cap = (size_t)F->cap;
+    emit_blocks(S, B, n, F->ipt, nullptr);
+    __syncthreads();
+    const int h = plan_moves(S, n, nd);
     __syncthreads();
     // mark the lists that change, those of the neighbours of the deleted
     // bubbles and of the moving survivors: 16 lanes per bubble.  The pairs

@@ -220,6 +220,7 @@ int time_search(Engine &e, int reps, cubble_search_times *out) {
         launch_set_flags(g, 0, 0, 1);
         const int applies = g.nb_bub <= kApplyBlocks ? 1 : kSearchEvery;
         rc = timed([&] {
+            if (g.plans) launch_plan(g);
             for (int k = 0; k < applies; ++k) launch_apply(g);
             launch_search(g);
         }, idle_ms);
@@ -396,7 +397,7 @@ int cubble_remove_bubbles(cubble_sim *s) {
     if (rc) return rc;
     if (!h.d.marked) return CUBBLE_OK;  // carried out already, or no attempt
     const Grid g = e.grid();
-    launch_set_flags(g, -1, 1, 0);
+    launch_set_flags(g, -1, kMarked, 0);
     launch_remove(g);
     launch_set_flags(g, -1, 0, 0);
     R_TRY(e, hipGetLastError());

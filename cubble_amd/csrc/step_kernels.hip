@@ -649,7 +649,8 @@ __device__ __forceinline__ void correct_range(const Consts &c, const Roles &R, c
 // dt controller and commit: reference src/simulator.cu:239-246, :258-321, by
 // one thread, from copies of the header's parts that were read before (the
 // pointers' rotation in place took a load's time for each buffer: a load does
-// not pass the stores before it).  Returns whether the step removes bubbles.
+// not pass the stores before it).  Returns whether the step removes bubbles that
+// the calling workgroup plans.
 __device__ __forceinline__ bool control(Foam *F, const Dyn &was, const Roles &R, uint32_t flags,
                                         const CorrAcc &a) {
     Dyn &d = F->d;
@@ -706,13 +707,14 @@ __device__ __forceinline__ bool control(Foam *F, const Dyn &was, const Roles &R,
     d.time_frac = now.time_frac;
     const bool removes = gas && a.n_del > 0;
     if (gas) d.max_r_cell = a.max_r;
-    d.need_remove = removes ? 1 : 0;
+    const bool launched = removes && a.n_del > kBlock && F->nblk > kControlPlans;
+    d.need_remove = !removes ? 0 : launched ? kMarked : kPlanned;
     d.need_search = a.max_exp >= 0.5 * skin ? 1 : 0;
     d.ts_min = fmin(was.ts_min, ndt);
     d.ts_max = fmax(was.ts_max, ndt);
     d.ts_sum = was.ts_sum + ndt;
     if (stop_reached(now)) d.halt = 1;
-    return removes;
+    return removes && !launched;
 }
 
 template <int D, bool M, bool W, bool OWN, typename Sums>
@@ -781,9 +783,10 @@ __global__ __launch_bounds__(kBlock) void k_correct(Foam *foams, const int2 *bt,
 // the next launch applies.
 __device__ __forceinline__ void control_block(Foam *F, uint32_t flags) {
     if (standing(F->d)) {
-        // the removal of its last step is done, or (kApply) waits for the
-        // search phase
-        if (0 == threadIdx.x && !(flags & kApply)) F->d.need_remove = 0;
+        // the removal of its last step is done, or waits for the search phase
+        // (kApply, or for its plan)
+        if (0 == threadIdx.x && !(flags & kApply) && kPlanned == F->d.need_remove)
+            F->d.need_remove = 0;
         return;
     }
     __shared__ int s_del;
