@@ -561,7 +561,23 @@ __device__ __forceinline__ void cell_dims(const Consts &c, double max_r, int cap
         cd[k] = (int)q;
     }
     if (2 == c.dim) cd[2] = 1;
-    while ((long long)cd[0] * cd[1] * cd[2] > (long long)cap) {
+    // Too many cells: the axis with the most loses one, the first of equals, until
+    // they fit.  That lowers the largest axes to a common level, and that level
+    // step by step, so the levels that are all too many are skipped by
+    // bisection (a sparse box has up to millions of steps).
+    auto cells = [&](int level) {
+        return (long long)min(cd[0], level) * min(cd[1], level) * min(cd[2], level);
+    };
+    int fits = 1, over = max(cd[0], max(cd[1], cd[2]));
+    if (cells(over) > (long long)cap) {
+        while (over - fits > 1) {
+            const int level = (fits + over) >> 1;
+            if (cells(level) > (long long)cap) over = level;
+            else fits = level;
+        }
+        for (int k = 0; k < 3; ++k) cd[k] = min(cd[k], over);
+    }
+    while ((long long)cd[0] * cd[1] * cd[2] > (long long)cap) {  // at most three
         int big = 0;
         for (int k = 1; k < 3; ++k)
             if (cd[k] > cd[big]) big = k;
