@@ -565,18 +565,16 @@ __device__ __forceinline__ void cell_dims(const Consts &c, double max_r, int cap
     // they fit.  That lowers the largest axes to a common level, and that level
     // step by step, so the levels that are all too many are skipped by
     // bisection (a sparse box has up to millions of steps).
-    auto cells = [&](int level) {
-        return (long long)min(cd[0], level) * min(cd[1], level) * min(cd[2], level);
-    };
+    if ((long long)cd[0] * cd[1] * cd[2] <= (long long)cap) return;
     int fits = 1, over = max(cd[0], max(cd[1], cd[2]));
-    if (cells(over) > (long long)cap) {
-        while (over - fits > 1) {
-            const int level = (fits + over) >> 1;
-            if (cells(level) > (long long)cap) over = level;
-            else fits = level;
-        }
-        for (int k = 0; k < 3; ++k) cd[k] = min(cd[k], over);
+    while (over - fits > 1) {
+        const int level = (fits + over) >> 1;
+        const long long cells =
+            (long long)min(cd[0], level) * min(cd[1], level) * min(cd[2], level);
+        if (cells > (long long)cap) over = level;
+        else fits = level;
     }
+    for (int k = 0; k < 3; ++k) cd[k] = min(cd[k], over);
     while ((long long)cd[0] * cd[1] * cd[2] > (long long)cap) {  // at most three
         int big = 0;
         for (int k = 1; k < 3; ++k)
