@@ -259,15 +259,20 @@ struct PairInput {
     const double *x, *y, *z, *r;
 };
 
-// Pair (i, j) of the caller's bubbles within r_i + r_j + skin (comparePair).
+// Bubble i's wrapped position and radius.
 template <int D>
-__device__ __forceinline__ bool within(const Consts &c, const PairInput &in, int i, int j) {
+__device__ __forceinline__ D4 wrapped(const Consts &c, const PairInput &in, int i) {
+    return D4{wrap_in(c, 0, in.x[i]), wrap_in(c, 1, in.y[i]),
+              3 == D ? wrap_in(c, 2, in.z[i]) : 0.0, in.r[i]};
+}
+
+// Two bubbles within r_i + r_j + skin (comparePair).
+template <int D>
+__device__ __forceinline__ bool within(const Consts &c, const D4 &a, const D4 &b) {
 #pragma clang fp contract(off)
     double d[3];
-    wrapped_diff<D>(c, wrap_in(c, 0, in.x[i]), wrap_in(c, 1, in.y[i]),
-                    3 == D ? wrap_in(c, 2, in.z[i]) : 0.0, wrap_in(c, 0, in.x[j]),
-                    wrap_in(c, 1, in.y[j]), 3 == D ? wrap_in(c, 2, in.z[j]) : 0.0, d);
-    const double maxd = in.r[i] + in.r[j] + c.skin;
+    wrapped_diff<D>(c, a.x, a.y, a.z, b.x, b.y, b.z, d);
+    const double maxd = a.r + b.r + c.skin;
     return sq_len(d) < maxd * maxd;
 }
 
@@ -286,12 +291,17 @@ __device__ __forceinline__ void sort_group(int32_t *pair_j, long long o0, long l
     }
 }
 
-// Any grid: a thread per slot walks the stencil of its cell.
+// Any grid: a thread per slot walks the stencil of its cell, four candidates at
+// a time (independent loads).  Lanes of one cell read the same candidates, so
+// their loads are one line each.  In the bubbles' order, which lets a wave skip
+// candidates before all of its bubbles, 64 scattered lanes a load cost more:
+// 2e5 bubbles in 27 cells 760 ms a call.
 template <int D, bool FILL>
 __device__ __forceinline__ void walk_slot(const Consts &c, const PairInput &in,
                                           const PairScratch &P, const PairGrid &g, int slot,
                                           int32_t *pair_i, int32_t *pair_j, long long pair_cap) {
     const int i = P.members[slot], cid = P.cell_s[slot];
+    const D4 own = wrapped<D>(c, in, i);
     const int cc[3] = {cid % g.cd[0], (cid / g.cd[0]) % g.cd[1], cid / (g.cd[0] * g.cd[1])};
     int ax[3][3], na[3] = {1, 1, 1};
     ax[2][0] = 0;
@@ -302,15 +312,28 @@ __device__ __forceinline__ void walk_slot(const Consts &c, const PairInput &in,
         for (int b = 0; b < na[1]; ++b)
             for (int e = 0; e < na[0]; ++e) {
                 const int cell = (ax[2][a] * g.cd[1] + ax[1][b]) * g.cd[0] + ax[0][e];
-                for (int s = P.cell_start[cell]; s < P.cell_start[cell + 1]; ++s) {
-                    const int j = P.members[s];
-                    if (j <= i) continue;
-                    if (!within<D>(c, in, i, j)) continue;
-                    if (FILL && o0 + k < pair_cap) {
-                        pair_i[o0 + k] = i;
-                        pair_j[o0 + k] = j;
+                const int s1 = P.cell_start[cell + 1];
+                for (int s = P.cell_start[cell]; s < s1; s += 4) {
+                    int js[4];
+                    bool later = false;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        js[u] = s + u < s1 ? P.members[s + u] : i;
+                        later = later || js[u] > i;
                     }
-                    ++k;
+                    if (!later) continue;
+                    D4 other[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) other[u] = wrapped<D>(c, in, js[u]);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        if (js[u] <= i || !within<D>(c, own, other[u])) continue;
+                        if (FILL && o0 + k < pair_cap) {
+                            pair_i[o0 + k] = i;
+                            pair_j[o0 + k] = js[u];
+                        }
+                        ++k;
+                    }
                 }
             }
     if (FILL) sort_group(pair_j, o0, min(o0 + k, pair_cap));
@@ -440,7 +463,8 @@ __device__ __forceinline__ void walk_tiles(const Consts &c, const PairInput &in,
                     const int dx = cx - P.cell_s[pc.j0 + r] % g.cd[0];
                     const bool near = (dx >= -1 && dx <= 1) ||
                                       (!wall[0] && (dx == g.cd[0] - 1 || dx == 1 - g.cd[0]));
-                    const bool hit = near && within<D>(c, in, b, mem[pc.j0 + r]);
+                    const bool hit = near && within<D>(c, wrapped<D>(c, in, b),
+                                                     wrapped<D>(c, in, mem[pc.j0 + r]));
                     w = hit ? w | 1u << r : w & ~(1u << r);
                 }
                 half[2 * kSub * tile] = (uint16_t)w;
@@ -495,8 +519,8 @@ __device__ __forceinline__ void walk_tiles(const Consts &c, const PairInput &in,
     }
 }
 
-// Pairs j > i of 64 slots per workgroup, a wave per 32 (matrix tiles) or a
-// thread per slot (small and odd grids).  What bounds it is latency, as the
+// Pairs j > i of 64 slots per workgroup, a wave per 32 (matrix tiles), or of 128
+// slots, one a thread (small and odd grids).  What bounds it is latency, as the
 // list kernel of the simulation; two passes, because the pairs' places are
 // known only after all are counted and the scratch holds no pairs.
 template <int D, bool FILL>
@@ -505,15 +529,14 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     int32_t *pair_j, long long pair_cap) {
     __shared__ PairLds lds[2];
     const PairGrid g = grid_of(c, P, nmax, cells_cap);
-    const int span0 = blockIdx.x * 64 + (int)(threadIdx.x >> 6) * kSub;
-    if (span0 >= n) return;
     if (g.fast) {
-        walk_tiles<D, FILL>(c, in, P, g, span0, n, pair_i, pair_j, pair_cap,
-                            lds[threadIdx.x >> 6]);
-    } else {
-        const int lane = (int)(threadIdx.x & 63);
-        if (lane < kSub && span0 + lane < n)
-            walk_slot<D, FILL>(c, in, P, g, span0 + lane, pair_i, pair_j, pair_cap);
+        const int span0 = blockIdx.x * 64 + (int)(threadIdx.x >> 6) * kSub;
+        if (span0 < n)
+            walk_tiles<D, FILL>(c, in, P, g, span0, n, pair_i, pair_j, pair_cap,
+                                lds[threadIdx.x >> 6]);
+    } else {  // (128 slots a workgroup: half of them suffice)
+        const int slot = blockIdx.x * 128 + (int)threadIdx.x;
+        if (slot < n) walk_slot<D, FILL>(c, in, P, g, slot, pair_i, pair_j, pair_cap);
     }
 }
 
