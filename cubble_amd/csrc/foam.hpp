@@ -143,7 +143,8 @@ struct Dyn {
     double bubble_steps;
     double s_a, s_ar, s_oa, s_oar, s_v, max_err, max_r, max_exp;
     double vol_fix;      // multiplier of the pending volume fix
-    double search_max_r; // largest radius at the running search (k_s_cells), 0 otherwise
+    double search_max_r; // largest radius at the running search (k_s_cells), 0 otherwise;
+                         // infinite when a bubble lies more than a period outside
     double list_max_r;   // largest radius at the last search
     // stop rules checked after every accepted step (0 = off)
     double r_stop;       // halt once the step's largest radius >= r_stop

@@ -55,6 +55,9 @@ __device__ __forceinline__ double cells_range(const Consts &c, const Roles &R, c
                     p[q] = xv + (c.tfr[q] - c.lbb[q]) * (double)mult;
                     R.x[q][i] = p[q];
                     R.wc[q][i] -= mult;
+                    // more than a period outside: it stays in an edge cell, far
+                    // from where the matrix tiles take its pairs to be
+                    if (!(p[q] >= c.lbb[q] && p[q] <= c.tfr[q])) rmax = __builtin_inf();
                 }
             }
             int id[3] = {0, 0, 0};
@@ -693,7 +696,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
     const int nbr_cap = F->nbr_cap;
     int sum_nn = 0, max_nn = 0, ovf = 0;
     // the fast path needs 5 or more cells along every periodic axis, and
-    // cells no pair within reach can skip
+    // cells no pair within reach can skip (rmax: none is known to be such when
+    // a bubble lies more than a period outside)
     bool fast = rmax > 0.0;
 #pragma unroll
     for (int k = 0; k < 3; ++k)

@@ -100,3 +100,33 @@ def test_bubbles_outside_a_walled_box(ora, dim, wall, reach):
     st["x"][0][out[30:]] = sc["tfr"][0] + rng.uniform(0.0, reach, 30)
     _search_equals_oracle(ora, sim, st, sc)
     sim.close()
+
+
+@pytest.mark.parametrize("dim,wall", [(2, (0, 0, 0)), (2, (0, 1, 0)), (3, (0, 0, 0)),
+                                      (3, (0, 0, 1))])
+@pytest.mark.parametrize("n", [1500, 6000])
+def test_bubbles_more_than_a_period_outside(ora, dim, wall, n):
+    """One wrap leaves them outside, in an edge cell, so that under the minimum
+    image they touch bubbles of cells that are not that one's neighbours: the
+    cells decide which pairs may meet."""
+    print(f"search off the period dim={dim} wall={wall} n={n}", flush=True)
+    sim = ca.Simulator(config(dim, n, seed=41 + dim, wall=wall))
+    st, sc = sim.get_state()
+    rng = np.random.default_rng(n)
+    far = rng.permutation(n)[:150].reshape(3, 50)
+    L = [sc["interval"][k] for k in range(3)]
+    for k in range(dim):
+        if wall[k]:
+            continue
+        st["x"][k][far[0]] = -rng.uniform(1.0, 1.9, 50) * L[k]
+        st["x"][k][far[1]] = rng.uniform(2.0, 2.9, 50) * L[k]
+    st["x"][0][far[2]] = rng.uniform(2.0, 2.9, 50) * L[0]
+    for _ in range(2):  # the second search finds most of them a period nearer
+        gst, gsc = _search_equals_oracle(ora, sim, st, sc, brute=False)
+        assert min(gsc["cell_dim"][k] for k in range(dim)) >= 5
+        pairs = set(map(tuple, np.stack([np.repeat(np.arange(n), np.diff(gst["nbr_off"])),
+                                         gst["nbr"]], 1).tolist()))
+        assert all((j, i) in pairs for i, j in pairs)
+        st, sc = gst, gsc
+    sim.run_steps(5, ca.IntegrationParams(True, False, True))
+    sim.close()
