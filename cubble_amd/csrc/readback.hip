@@ -49,9 +49,13 @@ struct PackArgs {
     PackSeg seg[kPackSegs];
     int32_t nseg;
     int32_t bubbles;
-    const int32_t *ends, *nbr;
+    const uint32_t *ends;
+    const int64_t *base;
+    const int32_t *nbr;
     uint64_t cap;
 };
+
+constexpr int kEndsTile = 4 * kBlock;  // bubbles per workgroup of k_ends
 
 __global__ __launch_bounds__(kBlock) void k_pack(PackArgs a, char *out) {
     int s = 0;
@@ -67,14 +71,23 @@ __global__ __launch_bounds__(kBlock) void k_pack(PackArgs a, char *out) {
             reinterpret_cast<uint64_t *>(out + g.dst)[e] =
                 static_cast<const uint64_t *>(g.src)[k];
         } else if (Readback::kLists == g.kind) {
-            // the bubble whose list holds entry k: the first that ends past it
-            int lo = 0, hi = a.bubbles - 1;
+            // the tile, and in it the bubble, whose lists hold entry k: the first
+            // that ends past it
+            int t = 0, hi = (a.bubbles - 1) / kEndsTile;
+            while (t < hi) {
+                const int mid = (t + hi) >> 1;
+                if ((uint64_t)a.base[mid + 1] > k) hi = mid;
+                else t = mid + 1;
+            }
+            const uint32_t first = (uint32_t)a.base[t], rel = (uint32_t)k - first;
+            int lo = t * kEndsTile;
+            hi = min(a.bubbles, lo + kEndsTile) - 1;
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
-                if ((uint64_t)a.ends[mid] > k) hi = mid;
+                if (a.ends[mid] - first > rel) hi = mid;
                 else lo = mid + 1;
             }
-            const uint64_t q = k - (lo > 0 ? (uint64_t)a.ends[lo - 1] : 0);
+            const uint32_t q = rel - (lo > t * kEndsTile ? a.ends[lo - 1] - first : 0u);
             reinterpret_cast<int32_t *>(out + g.dst)[e] = a.nbr[q * a.cap + lo];
         } else {  // FP32 as it is; bytes in words of four
             reinterpret_cast<uint32_t *>(out + g.dst)[e] =
@@ -82,8 +95,6 @@ __global__ __launch_bounds__(kBlock) void k_pack(PackArgs a, char *out) {
         }
     }
 }
-
-constexpr int kEndsTile = 4 * kBlock;  // bubbles per workgroup
 
 __global__ __launch_bounds__(kBlock) void k_ends_part(const int32_t *nn, int n, int32_t *part) {
     int s = 0;
@@ -96,19 +107,22 @@ __global__ __launch_bounds__(kBlock) void k_ends_part(const int32_t *nn, int n, 
     if (0 == threadIdx.x) part[blockIdx.x] = s;
 }
 
+// (A foam's lists may hold more than 2^31 entries, those of 1024 bubbles not.)
 __global__ __launch_bounds__(kBlock) void k_ends(const int32_t *nn, int n, const int32_t *part,
-                                                 int32_t *ends) {
-    int acc = 0;
-    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kBlock) acc += part[b];
-    int off = block_sum_i(acc);
+                                                 uint32_t *ends, int64_t *base) {
+    double acc = 0.0;  // whole numbers: exact
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kBlock) acc += (double)part[b];
+    int64_t off = (int64_t)block_sum(acc);
+    if (0 == threadIdx.x) base[blockIdx.x] = off;
     for (int u = 0; u < 4; ++u) {
         const int i = blockIdx.x * kEndsTile + u * kBlock + (int)threadIdx.x;
         const int v = i < n ? nn[i] : 0;
         int tot = 0;
         const int pre = block_excl_scan(v, tot);
-        if (i < n) ends[i] = off + pre + v;
+        if (i < n) ends[i] = (uint32_t)(off + pre + v);
         off += tot;
     }
+    if (0 == threadIdx.x && blockIdx.x + 1 == gridDim.x) base[gridDim.x] = off;
 }
 
 // Pinned memory in slots and the events of the kernels that fill them.
@@ -246,7 +260,7 @@ void bounce_engine_closed() {
     g_idle.clear();
 }
 
-void Readback::lists(int32_t *dst, const int32_t *ends, const int32_t *nbr, size_t cap, int n,
+void Readback::lists(int32_t *dst, const ListEnds &ends, const int32_t *nbr, size_t cap, int n,
                      size_t total) {
     ends_ = ends;
     nbr_ = nbr;
@@ -275,7 +289,8 @@ int Readback::run(Engine &e) {
     // the next chunk's kernel, into slot h; false: nothing is left
     auto launch = [&](int h) {
         PackArgs a{};
-        a.ends = ends_;
+        a.ends = ends_.ends;
+        a.base = ends_.base;
         a.nbr = nbr_;
         a.cap = cap_;
         a.bubbles = bubbles_;
@@ -337,11 +352,17 @@ int Readback::run(Engine &e) {
     return CUBBLE_OK;
 }
 
-void launch_list_ends(const int32_t *nn, int n, int32_t *ends, int32_t *part,
-                      hipStream_t stream) {
+ListEnds launch_list_ends(const int32_t *nn, int n, int32_t *ends, int32_t *scratch,
+                          hipStream_t stream) {
     const int nb = (n + kEndsTile - 1) / kEndsTile;
+    ListEnds e;
+    e.ends = reinterpret_cast<uint32_t *>(ends);
+    e.base = reinterpret_cast<int64_t *>(scratch);
+    e.total = e.base + nb;
+    int32_t *const part = scratch + 2 * (nb + 1);
     hipLaunchKernelGGL(k_ends_part, dim3(nb), dim3(kBlock), 0, stream, nn, n, part);
-    hipLaunchKernelGGL(k_ends, dim3(nb), dim3(kBlock), 0, stream, nn, n, part, ends);
+    hipLaunchKernelGGL(k_ends, dim3(nb), dim3(kBlock), 0, stream, nn, n, part, e.ends, e.base);
+    return e;
 }
 
 }  // namespace cubble_amd

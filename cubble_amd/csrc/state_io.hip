@@ -132,13 +132,14 @@ int get_state(Engine &e, int k, cubble_state_view *v) {
     }
     rb.i32(v->index, f.r.idx, n);
     rb.i32(v->degree, f.s.deg, n);
-    int32_t total = 0;
+    int64_t total = 0;
+    ListEnds ends;
     if ((v->nbr_off || v->nbr) && n > 0) {
         // (scratch of a removal, which runs as a whole within a step)
-        launch_list_ends(f.s.nn, (int)n, f.s.plan_src, f.s.moved_to, e.stream);
+        ends = launch_list_ends(f.s.nn, (int)n, f.s.plan_src, f.s.moved_to, e.stream);
         R_TRY(e, hipGetLastError());
-        rb.i32(&total, f.s.plan_src + (n - 1), 1);
-        if (v->nbr_off) rb.i32(v->nbr_off + 1, f.s.plan_src, n);
+        rb.i64(&total, ends.total, 1);
+        if (v->nbr_off) rb.i32(v->nbr_off + 1, ends.ends, n);
     }
     if (v->nbr_off) v->nbr_off[0] = 0;
     if ((rc = rb.run(e))) return rc;
@@ -146,7 +147,7 @@ int get_state(Engine &e, int k, cubble_state_view *v) {
         if (total > v->nbr_cap)
             return e.fail(CUBBLE_E_CAPACITY, "get_state: nbr buffer too small");
         Readback lists;
-        lists.lists(v->nbr, f.s.plan_src, f.s.nbr, (size_t)f.cap, (int)n, (size_t)total);
+        lists.lists(v->nbr, ends, f.s.nbr, (size_t)f.cap, (int)n, (size_t)total);
         return lists.run(e);
     }
     return CUBBLE_OK;
