@@ -36,11 +36,13 @@ struct PackSeg {
 
 constexpr int kPackSegs = 32;
 constexpr unsigned kPackTile = 4 * kBlock;  // elements per workgroup
-// The pinned block's bytes and the kernels in flight on it: eight of up to
-// 512 kB each, so that the copies of a small read start early, or four of 1 MB.
-constexpr size_t kBlockBytes = (size_t)4 << 20;
-constexpr int kSlots = 8;
-// Reads above it copy with three threads more (starting them takes 30 us).
+// The pinned block: room for the chunk that the host copies and the two whose
+// kernels are in flight meanwhile, the one behind it and the one after.
+constexpr int kSlots = 3;
+constexpr size_t kRoom = (size_t)1 << 20;
+// Reads above it go in chunks of kRoom and copy with three threads more
+// (starting them takes 30 us); smaller ones in half of it at most, so that their
+// copies start early.
 constexpr size_t kHelpFrom = (size_t)4 << 20;
 constexpr int kHelpers = 3;
 constexpr size_t kPiece = (size_t)64 << 10;  // bytes a thread copies at a time
@@ -133,9 +135,10 @@ struct Bounce {
 };
 
 std::mutex g_lock;
-std::vector<Bounce> g_idle;  // at most kIdle; emptied with the last engine
+constexpr int kIdle = 2;
+Bounce g_idle[kIdle];  // emptied with the last engine
+int g_num_idle = 0;
 int g_engines = 0;
-constexpr size_t kIdle = 2;
 
 void destroy(Bounce &b) {
     for (hipEvent_t &d : b.done)
@@ -151,15 +154,15 @@ class Lease {
     hipError_t take(int device) {
         {
             std::lock_guard<std::mutex> l(g_lock);
-            for (size_t k = 0; k < g_idle.size(); ++k)
+            for (int k = 0; k < g_num_idle; ++k)
                 if (g_idle[k].device == device) {
                     b = g_idle[k];
-                    g_idle.erase(g_idle.begin() + (long)k);
+                    g_idle[k] = g_idle[--g_num_idle];
                     return hipSuccess;
                 }
         }
         b.device = device;
-        hipError_t e = hipHostMalloc((void **)&b.mem, kBlockBytes, hipHostMallocDefault);
+        hipError_t e = hipHostMalloc((void **)&b.mem, kSlots * kRoom, hipHostMallocDefault);
         for (hipEvent_t &d : b.done)
             if (hipSuccess == e) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
         return e;
@@ -169,8 +172,8 @@ class Lease {
     ~Lease() {
         if (complete && b.done[kSlots - 1]) {
             std::lock_guard<std::mutex> l(g_lock);
-            if (g_engines > 0 && g_idle.size() < kIdle) {
-                g_idle.push_back(b);
+            if (g_engines > 0 && g_num_idle < kIdle) {
+                g_idle[g_num_idle++] = b;
                 return;
             }
         }
@@ -256,8 +259,7 @@ void bounce_engine_opened() {
 void bounce_engine_closed() {
     std::lock_guard<std::mutex> l(g_lock);
     if (--g_engines > 0) return;
-    for (Bounce &b : g_idle) destroy(b);
-    g_idle.clear();
+    while (g_num_idle > 0) destroy(g_idle[--g_num_idle]);
 }
 
 void Readback::lists(int32_t *dst, const ListEnds &ends, const int32_t *nbr, size_t cap, int n,
@@ -280,10 +282,9 @@ int Readback::run(Engine &e) {
     if (err != hipSuccess) return bad(err, "readback: pinned memory");
     size_t all = 0;
     for (const Item &it : items_) all += it.n * it.size;
-    const int slots = all <= kBlockBytes ? kSlots : kSlots / 2;
-    const size_t room = kBlockBytes / slots;
     // (a small read in equal parts, so that the copies overlap the kernels)
-    const size_t chunk = std::min(room, std::max((all / 4 + 255) & ~(size_t)255, (size_t)128 << 10));
+    const size_t chunk = std::min(all > kHelpFrom ? kRoom : kRoom / 2,
+                                  std::max((all / 4 + 255) & ~(size_t)255, (size_t)128 << 10));
     std::vector<Copy> copies[kSlots];
     size_t item = 0, at = 0;  // the next element to fetch
     // the next chunk's kernel, into slot h; false: nothing is left
@@ -295,7 +296,7 @@ int Readback::run(Engine &e) {
         a.cap = cap_;
         a.bubbles = bubbles_;
         copies[h].clear();
-        char *const out = lease.b.mem + (size_t)h * room;
+        char *const out = lease.b.mem + (size_t)h * kRoom;
         size_t off = 0;
         unsigned tiles = 0;
         while (item < items_.size() && a.nseg < kPackSegs) {
@@ -338,10 +339,9 @@ int Readback::run(Engine &e) {
     // (two to begin with: the first copy waits for their launches)
     for (; ahead < 2 && hipSuccess == err && (busy[ahead] = launch(ahead)); ++ahead) {}
     Copier copier(all > kHelpFrom ? kHelpers : 0);
-    for (int h = 0; hipSuccess == err && busy[h]; h = (h + 1) % slots) {
-        // as many kernels in flight as there are slots free
-        if (!busy[ahead] && hipSuccess == err && (busy[ahead] = launch(ahead)))
-            ahead = (ahead + 1) % slots;
+    for (int h = 0; hipSuccess == err && busy[h]; h = (h + 1) % kSlots) {
+        // the slot copied last takes the chunk after the one in flight
+        if (!busy[ahead] && (busy[ahead] = launch(ahead))) ahead = (ahead + 1) % kSlots;
         if (hipSuccess == err) err = hipEventSynchronize(lease.b.done[h]);
         if (err != hipSuccess) break;
         copier.run(copies[h]);
