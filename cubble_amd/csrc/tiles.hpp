@@ -28,10 +28,22 @@ constexpr int kSegment = 512;   // candidate places per pass of a tile
 // Error bound of the matrix product's |d|^2 - (r_i + r_j + skin)^2 for a pair
 // within reach, or nearly so, relative to Q, which bounds |u|^2 + r^2 of own
 // bubbles and candidates (u relative to the window's centre).  In units of
-// 2^-22 Q: rounding the coordinates and radii to FP32 1, their split into two
-// FP16 values (2^-22 each, both sides) 4, the products of the two low parts
-// left out 2, the FP32 norms and their split 4, sixteen products added with
-// partial sums of at most 2 Q 8.  Pairs farther apart have a larger value by
+// 2^-22 Q:
+//   1    coordinates and radii rounded to FP32 (0.6 near the cutoff, where |d|
+//        is at most a cell and Q at least 4.5 cells squared)
+//   4    their split into two FP16 values, 2^-22 each, both sides
+//   1.5  low parts below FP16's normal range, which the instruction keeps: steps
+//        of 2^-24 where the largest cell edge is 0.5 to 1
+//   2    the products of the two low parts, left out
+//   4    the FP32 norms and their split
+//   8    the instruction.  It adds the eight products of a half of K at a time,
+//        aligned to the largest, and drops what lies below 2^-24 of that (its
+//        results for 1 +- 15 x 2^-24, x = 1/8 .. 3/2, with the 1 in any place):
+//        7 2^-24 2 Q and, with the norms, 7 2^-24 Q, then the halves' sum
+//        rounded, 6 in all; one after the other with partial sums of at most
+//        2 Q, 8
+// Pairs at the cutoff in windows of 1 to 10 cells measured 0.4 to 2.7 in all, 0.3
+// to 1.9 of it from the instruction.  Pairs farther apart have a larger value by
 // more than their error grows.
 constexpr float kBand = 0x1.6p-18f;  // 22 2^-22
 constexpr float kFar = 3e4f;         // norm of an empty place: never a hit
