@@ -347,10 +347,11 @@ int Engine::commit_layout() {
     std::vector<int2> bb, bc, bs;
     for (int f = 0; f < nf; ++f) {
         hs[f] = foams[f].h;
+        dev_index_[f] = f;
+        if (1 == nf) continue;  // its blocks are the launch's: no tables
         for (int l = 0; l < hs[f].nblk; ++l) bb.push_back(make_int2(f, l));
         for (int l = 0; l < hs[f].cblk; ++l) bc.push_back(make_int2(f, l));
         for (int l = 0; l < hs[f].sblk; ++l) bs.push_back(make_int2(f, l));
-        dev_index_[f] = f;
     }
     if (nf > 0) E_TRY(hipMemcpy(dfoams_, hs.data(), sizeof(Foam) * nf, hipMemcpyHostToDevice));
     auto upload = [&](int2 *&buf, size_t &cap, const std::vector<int2> &v) -> int {
@@ -366,9 +367,9 @@ int Engine::commit_layout() {
     if ((rc = upload(bt_bub_, bt_bub_cap_, bb)) || (rc = upload(bt_cell_, bt_cell_cap_, bc)) ||
         (rc = upload(bt_scell_, bt_scell_cap_, bs)))
         return rc;
-    nb_bub_ = (int)bb.size();
-    nb_cell_ = (int)bc.size();
-    nb_scell_ = (int)bs.size();
+    nb_bub_ = 1 == nf ? hs[0].nblk : (int)bb.size();
+    nb_cell_ = 1 == nf ? hs[0].cblk : (int)bc.size();
+    nb_scell_ = 1 == nf ? hs[0].sblk : (int)bs.size();
     // the captured graph holds the header array, the block tables and the
     // grid sizes; it stays valid while none of them moved or changed size
     const bool same = old_foams == dfoams_ && old_bt[0] == bt_bub_ && old_bt[1] == bt_cell_ &&
