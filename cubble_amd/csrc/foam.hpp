@@ -29,9 +29,10 @@ constexpr int kFuseBlocks = 640, kFuseBatch = 128;
 // Launches of at most this many blocks, one bubble a thread, take four lanes a
 // bubble in the pair kernel; mixed ones of 3D foams only up to the second, where
 // the longer lists give the wider kernel less to gain (200 steps, one lane /
-// four: 3D mixed 6e4 6.2 / 5.8 ms, 1e5 7.45 / 7.1, 1.3e5 7.5 / 7.7; 2D mixed 6e4
-// 5.9 / 5.1, 2e5 9.0 / 8.6; 128 foams of 2e3 24.4 / 23.1).
-constexpr int kQuadBlocks = 1024, kQuadMixed3 = 400;
+// four: 3D mixed 5e4 6.58 / 5.82 ms, 8e4 7.20 / 6.52, 1e5 7.49 / 7.15, 1.1e5 7.38
+// / 7.18, 1.2e5 (469 blocks) 7.47 / 7.39, 1.3e5 (508) 7.62 / 7.76, 1.4e5 8.54 /
+// 8.76; 2D mixed 6e4 5.9 / 5.1, 2e5 9.0 / 8.6; 128 foams of 2e3 24.4 / 23.1).
+constexpr int kQuadBlocks = 1024, kQuadMixed3 = 480;
 // Foams of more than this many blocks have a removal of more than kBlock bubbles
 // planned by launches before the search phase instead of by k_control (see
 // remove_plan.hpp).
