@@ -535,8 +535,9 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
             walk_tiles<D, FILL>(c, in, P, g, span0, n, pair_i, pair_j, pair_cap,
                                 lds[threadIdx.x >> 6]);
     } else {  // (128 slots a workgroup: half of them suffice)
-        const int slot = blockIdx.x * 128 + (int)threadIdx.x;
-        if (slot < n) walk_slot<D, FILL>(c, in, P, g, slot, pair_i, pair_j, pair_cap);
+        const unsigned slot = blockIdx.x * 128u + threadIdx.x;  // (up to 2^32)
+        if (slot < (unsigned)n)
+            walk_slot<D, FILL>(c, in, P, g, (int)slot, pair_i, pair_j, pair_cap);
     }
 }
 
