@@ -162,9 +162,15 @@ class Lease {
                 }
         }
         b.device = device;
-        hipError_t e = hipHostMalloc((void **)&b.mem, kSlots * kRoom, hipHostMallocDefault);
+        // an event belongs to the device that is current, which need not be the
+        // engine's in the calling thread
+        int was = device;
+        hipError_t e = hipGetDevice(&was);
+        if (hipSuccess == e && was != device) e = hipSetDevice(device);
+        if (hipSuccess == e) e = hipHostMalloc((void **)&b.mem, kSlots * kRoom, hipHostMallocDefault);
         for (hipEvent_t &d : b.done)
             if (hipSuccess == e) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
+        if (was != device) (void)hipSetDevice(was);
         return e;
     }
     // complete: nothing on the device uses the block any more
