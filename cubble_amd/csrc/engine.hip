@@ -758,10 +758,10 @@ int Engine::integrate(uint32_t flags, std::vector<Dyn> &d) {
         if (plan) launch_plan(grid());
         if (apply) launch_apply(grid());
         if (search) launch_search(grid());
-        if (apply || search) {
-            E_TRY(hipGetLastError());
-            if ((rc = read_dyn_all(d))) return rc;
-        }
+        E_TRY(hipGetLastError());
+        // (a planned removal changes no scalar, and whatever comes next waits for
+        // the stream or goes behind it there)
+        if ((plan || search) && (rc = read_dyn_all(d))) return rc;
         if ((rc = settle_read(d))) return rc;
         if (one && d[0].accepted && !d[0].halt && !d[0].overflow) {
             clean_ = true;
