@@ -5,8 +5,8 @@
 // partials to reduce), bubbles per neighbour-search workgroup (the search
 // tile: small tiles give the few searching foams of a batch enough
 // workgroups, large ones cheapen the idle launch over every foam's tiles),
-// and attempt groups per captured graph replay (host synchronisations against the groups a replay
-// wastes after every foam reached its step limit).
+// and attempt groups per captured graph replay (host synchronisations against
+// the groups a replay wastes after every foam reached its step limit).
 //
 // The tuner copies the whole device state aside, then for each candidate
 // restores it, applies the shapes, primes the captured graph, restores again

@@ -271,10 +271,11 @@ __device__ __forceinline__ void reduce_parts4(Read &&read, const int32_t *part_i
 // The body has no branch per neighbour: the four chains of a chunk overlap,
 // where one after another each waited for its own square root and
 // reciprocals (2D 1e4: 9.0 -> 7.5 us a launch), and terms that do not count
-// are selected away (adding 0).  At 1e6 bubbles it is bound by the gathers'
-// cache accesses, 64 lines a load: 78 us either way, and neither six waves
-// (114 us, spilled) nor halves of records gathered by neighbouring lanes (110
-// us) help.
+// are selected away (adding 0).  At 1e6 bubbles (65 to 78 us) it is bound by
+// instruction issue: VALU work in 61% of the cycles, and waves wait to issue for
+// 46% of theirs, on memory for 30%, with the address units busy for 37%.  Neither
+// six waves (114 us, spilled) nor halves of records gathered by neighbouring
+// lanes (110 us) help.
 template <bool FLOW>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FLOW ? 4 : 5, 8))) void
 k_pair(Foam *foams, const int2 *bt, uint32_t flags) {
